@@ -149,6 +149,11 @@ namespace {
 
 int build_fac32(ptq2_ctx *c) { return ptq2_internal_build_fac32(c); }
 
+// how the FP64 A11 pass leaves y (it writes the Dirichlet rows of a MatMult itself)
+ptq2::OutMode out_mode(const ptq2_ctx *c, bool mm, bool add) {
+  return mm && c->mask ? ptq2::OUT_BC : (add ? ptq2::OUT_ADD : ptq2::OUT_SET);
+}
+
 // resident FP64 geometry of the stored-geometry A11 kernel (depends on the mesh only)
 int build_geo64(ptq2_ctx *c) {
   if (c->geo64_valid) return PTQ2_OK;
@@ -276,6 +281,27 @@ int ptq2_sizes(const ptq2_ctx *c, int64_t *nv, int64_t *np, int64_t *ne) {
   return PTQ2_OK;
 }
 
+}  // extern "C"
+
+namespace {
+// sets the flag of every brick whose tile holds box node n
+void mark_bricks(const Box &b, int64_t n, uint8_t *flag) {
+  const int e[3] = {(int)(n % b.NX) - b.i0, (int)(n / b.NX % b.NY) - b.j0, (int)(n / ((int64_t)b.NX * b.NY)) - b.k0};
+  const int m[3] = {b.mx, b.my, b.mz}, nb[3] = {b.nbx, b.nby, b.nbz};
+  int lo[3], hi[3];
+  for (int d = 0; d < 3; d++) {
+    if (e[d] < 0 || e[d] > 2 * m[d]) return;  // a ghost node of no owned element
+    hi[d] = std::min(e[d] / (2 * ptq2::BE), nb[d] - 1);
+    lo[d] = e[d] % (2 * ptq2::BE) == 0 && e[d] > 0 ? e[d] / (2 * ptq2::BE) - 1 : hi[d];
+  }
+  for (int z = lo[2]; z <= hi[2]; z++)
+    for (int y = lo[1]; y <= hi[1]; y++)
+      for (int x = lo[0]; x <= hi[0]; x++) flag[x + (int64_t)b.nbx * (y + (int64_t)b.nby * z)] = 1;
+}
+}  // namespace
+
+extern "C" {
+
 int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int NZ, int i0, int j0, int k0,
                         const double *coords, const uint8_t *mask) {
   if (!c || !coords) return fail(c, PTQ2_ERR_INVALID_ARG, "null context or coordinates");
@@ -300,11 +326,12 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   dev_free(c->coords); dev_free(c->mask); dev_free(c->dir_idx); dev_free(c->eta_bm);
   dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf);
   c->coords = nullptr; c->mask = nullptr; c->dir_idx = nullptr; c->eta_bm = nullptr;
+  c->xtile = nullptr; c->bdir = nullptr;
   c->fac32 = nullptr; c->facb32 = nullptr; c->geo64 = nullptr; c->facebuf = nullptr;
   c->mesh_ready = c->eta_ready = c->fac32_valid = c->facb32_valid = c->geo64_valid = c->has_state = false;
   c->ndir = 0;
 
-  Box b;
+  Box b{};
   b.mx = mx; b.my = my; b.mz = mz; b.NX = NX; b.NY = NY; b.NZ = NZ; b.i0 = i0; b.j0 = j0; b.k0 = k0;
   b.nbx = (mx + ptq2::BE - 1) / ptq2::BE; b.nby = (my + ptq2::BE - 1) / ptq2::BE; b.nbz = (mz + ptq2::BE - 1) / ptq2::BE;
   {
@@ -319,22 +346,38 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   HIPCHK(c, hipMemcpy(c->coords, coords, sizeof(double) * 3 * (size_t)nn, hipMemcpyHostToDevice));
   if (mask) {
     std::vector<int64_t> idx;
+    std::vector<uint8_t> bdir((size_t)nb, 0);
     for (int64_t i = 0; i < 3 * nn; i++)
-      if (mask[i]) idx.push_back(i);
-    if ((rc = dev_alloc(c, (void **)&c->mask, 3 * (size_t)nn))) return rc;
+      if (mask[i]) {
+        idx.push_back(i);
+        mark_bricks(b, i / 3, bdir.data());
+      }
+    if ((rc = dev_alloc(c, (void **)&c->mask, 3 * (size_t)nn + (size_t)nb))) return rc;
     HIPCHK(c, hipMemcpy(c->mask, mask, 3 * (size_t)nn, hipMemcpyHostToDevice));
+    c->bdir = c->mask + 3 * (size_t)nn;
+    HIPCHK(c, hipMemcpy(c->bdir, bdir.data(), (size_t)nb, hipMemcpyHostToDevice));
+    b.bdir = c->bdir;
     c->ndir = (int64_t)idx.size();
     if (c->ndir) {
       if ((rc = dev_alloc(c, (void **)&c->dir_idx, sizeof(int64_t) * idx.size()))) return rc;
       HIPCHK(c, hipMemcpy(c->dir_idx, idx.data(), sizeof(int64_t) * idx.size(), hipMemcpyHostToDevice));
     }
   }
+  // Viscosity and the resident coordinate tiles share an allocation.  The tiles pay where the vectors
+  // come from HBM, not from the 256 MB cache before it: FP64 apply 1113 us with, 1163 us without at
+  // 128^3 elements (32768 bricks), 145 us with and without at 64^3 (4096 bricks), where they would only
+  // make the set-up longer (by a tenth at 33^3).  A mesh that fits the device only without them runs
+  // its FP64 passes from the coordinates too.
+  const size_t neta = (size_t)nb * 27 * ptq2::BEL, nxt = nb >= 8192 ? (size_t)nb * 3 * ptq2::TCS : 0;
+  if (nxt && dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * (neta + nxt)) == PTQ2_OK)
+    c->xtile = c->eta_bm + neta;
+  else if ((rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * neta)))
+    return rc;
+  b.xtile = c->xtile;
   c->box = b;
   c->nnodes = nn; c->nvel = 3 * nn; c->nel = ne; c->npres = 4 * ne; c->nbricks = nb;
-  if ((rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * (size_t)nb * 27 * ptq2::BEL))) return rc;
-
   if ((rc = clear_err(c))) return rc;
-  HIPCHK(c, ptq2::launch_check_mesh(b, c->coords, c->err, c->stream));
+  HIPCHK(c, ptq2::launch_check_mesh(b, c->coords, c->xtile, c->err, c->stream));
   int bits = 0;
   if ((rc = read_err(c, &bits))) return rc;
   if (bits & ptq2::ERRBIT_MESH) return fail(c, PTQ2_ERR_MESH, "non-positive Jacobian determinant in the mesh");
@@ -446,12 +489,12 @@ int ptq2_a11_apply(ptq2_ctx *c, const void *u, void *y, unsigned flags) {
     if (mm) HIPCHK(c, ptq2::launch_bc_rows<float>(c->ndir, c->dir_idx, (const float *)du, (float *)dy, 0, c->stream));
   } else {
     if (otf)
-      HIPCHK(c, ptq2::launch_a11_fp64(c->box, c->coords, (const double *)du, mask, c->eta_bm, (double *)dy, add,
-                                      c->stream, (double *)tb));
+      HIPCHK(c, ptq2::launch_a11_fp64(c->box, c->coords, (const double *)du, mask, c->eta_bm, (double *)dy,
+                                      out_mode(c, mm, add), c->stream, (double *)tb));
     else
       HIPCHK(c, ptq2::launch_a11_fp64g(c->box, (const double *)du, mask, c->geo64, c->eta_bm, (double *)dy, add,
                                        c->stream, (double *)tb));
-    if (mm) HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, (const double *)du, (double *)dy, 0, c->stream));
+    if (mm && !otf) HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, (const double *)du, (double *)dy, 0, c->stream));
   }
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(y, c->sy, es * (size_t)n, hipMemcpyDeviceToHost, c->stream));
@@ -480,8 +523,8 @@ int ptq2_a11_apply_noalloc(ptq2_ctx *c, const double *u, double *y, unsigned fla
   const bool mm = flags & PTQ2_MATMULT, add = flags & PTQ2_ADD;
   // every face slot the gather pass reads is written by the apply launch before it in stream
   // order, so the array needs no clearing between calls
-  HIPCHK(c, ptq2::launch_a11_fp64(c->box, c->coords, u, mm ? c->mask : nullptr, c->eta_bm, y, add, c->stream, scr));
-  if (mm) HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, u, y, 0, c->stream));
+  HIPCHK(c, ptq2::launch_a11_fp64(c->box, c->coords, u, mm ? c->mask : nullptr, c->eta_bm, y, out_mode(c, mm, add),
+                                  c->stream, scr));
   return PTQ2_OK;
 }
 
@@ -501,7 +544,7 @@ int a11_batch(ptq2_ctx *const *cs, int n, const void *const *u, void *const *y, 
   if (rc) return rc;
   ptq2::BatchArgs<T> a{};
   a.n = n;
-  a.add = add ? 1 : 0;
+  a.mode = f32 ? (add ? ptq2::OUT_ADD : ptq2::OUT_SET) : (mm ? ptq2::OUT_BC : (add ? ptq2::OUT_ADD : ptq2::OUT_SET));
   int64_t blocks = 0;
   for (int i = 0; i < n; i++) {
     ptq2_ctx *c = cs[i];
@@ -540,7 +583,7 @@ int a11_batch(ptq2_ctx *const *cs, int n, const void *const *u, void *const *y, 
     HIPCHK(c0, hipStreamWaitEvent(c0->stream, c->ev, 0));
   }
   HIPCHK(c0, ptq2::launch_a11_batch<T>(a, c0->stream));
-  if (mm)
+  if (mm && f32)  // the FP64 pass writes the Dirichlet rows itself
     for (int i = 0; i < n; i++)
       HIPCHK(c0, ptq2::launch_bc_rows<T>(cs[i]->ndir, cs[i]->dir_idx, (const T *)u[i], (T *)y[i], 0, c0->stream));
   bool others = false;

@@ -15,7 +15,9 @@ struct ptq2_ctx {
   ptq2::Box box{};
   int64_t nnodes = 0, nvel = 0, nel = 0, npres = 0, nbricks = 0;
   double *coords = nullptr;
+  double *xtile = nullptr;  // box.xtile: the bricks' coordinate tiles
   uint8_t *mask = nullptr;
+  uint8_t *bdir = nullptr;  // box.bdir: bricks that hold a Dirichlet dof
   int64_t *dir_idx = nullptr;
   int64_t ndir = 0;
   double *eta_bm = nullptr;

@@ -47,6 +47,9 @@ struct Box {
   int i0, j0, k0;
   int nbx, nby, nbz;
   int fast32;  // element offsets inside a 9^3-node tile fit 32 bits (the fast tile paths)
+  // Resident per-brick data of the FP64 operators (either may be null):
+  const double *xtile;   // every brick's coordinate tile in its LDS layout, 3*TCS doubles per brick
+  const uint8_t *bdir;   // nonzero where the brick's tile holds a Dirichlet dof
 };
 
 // 1D Q2 Lagrange basis on nodes {-1,0,1} at the Gauss points {-sqrt(3/5),0,sqrt(3/5)}:
@@ -124,6 +127,9 @@ __device__ __forceinline__ Tile tile_of(const Box &b, const BrickId &br) {
 // loads of a pass are issued before the first LDS store (one exposed memory latency
 // per tile instead of one per value).
 constexpr int TPAIRS = (TROWS + 1) / 2;
+// Three waves share a tile's traffic by planes: wave w takes z = 3 w .. 3 w + 2, 27 rows.
+constexpr int WPLANES = TN / 3;
+constexpr int WSTEPS = (WPLANES * TN + 1) / 2;
 struct TileLane {
   int p;           // row parity of this lane (0/1), 2 = idle lane
   int lds_col;     // LDS offset of the column: c*TCS + tx(ii)
@@ -204,9 +210,11 @@ __host__ __device__ __forceinline__ uint32_t fast_step(const Box &b, int it) {
 }
 __host__ __device__ __forceinline__ constexpr int fast_lds_step(int it) { return 20 * it + 2 * ((2 * it) / 9); }
 __host__ __device__ __forceinline__ constexpr bool fast_wrap(int it) { return (2 * it) % 9 == 8; }
-// this lane's element offset at step it (row 0 for the lanes that store nothing at that step)
+// this lane's element offset at step it (row 0 for the lanes that store nothing at that step);
+// STEPS row pairs: the whole tile, or one third of it (WSTEPS, from the third's first plane)
+template <int STEPS = TPAIRS>
 __host__ __device__ __forceinline__ uint32_t fast_eoff(const Box &b, const FastLane &L, int it) {
-  if (it == TPAIRS - 1 && L.p == 1) return (uint32_t)L.col;
+  if (it == STEPS - 1 && L.p == 1) return (uint32_t)L.col;
   return (fast_wrap(it) ? L.ew : L.e0) + fast_step(b, it);
 }
 // (y, z) of this lane's row at step it
@@ -215,8 +223,9 @@ __host__ __device__ __forceinline__ void fast_row(const FastLane &L, int it, int
   y = fast_wrap(it) ? (odd ? 0 : y0) : y0 + odd;
   z = fast_wrap(it) ? z0 + odd : z0;
 }
+template <int STEPS = TPAIRS>
 __host__ __device__ __forceinline__ bool fast_stores(const FastLane &L, int it) {
-  return L.p == 0 || (L.p == 1 && it < TPAIRS - 1);
+  return L.p == 0 || (L.p == 1 && it < STEPS - 1);
 }
 // element e of a field from a wave-uniform base: the byte offset is formed in 32 bits, so the
 // access is one global instruction with a scalar base and a 32-bit vector offset
@@ -229,6 +238,10 @@ template <typename S>
 __device__ __forceinline__ const S &fast_at(const S *base, uint32_t e) {
   const uint32_t bo = e * (uint32_t)sizeof(S);
   return *reinterpret_cast<const S *>(reinterpret_cast<const char *>(base) + bo);
+}
+template <typename S>
+__device__ __forceinline__ S &fast_at(S *base, int64_t e) {
+  return base[e];
 }
 
 // two fields, the second masked (Dirichlet dofs read as zero) if HM
@@ -445,34 +458,36 @@ __host__ __device__ __forceinline__ T cheb_update(const ChebOut<T> &co, int64_t 
   return cheb_value(co, co.dinv[i], co.b[i], y, co.x[i], co.pkm1 ? co.pkm1[i] : T(0), co.pkm1 != nullptr);
 }
 
-// the full-tile case with the addressing of load_tile2_fast
-template <bool CH, typename S, typename T>
+// the full-tile case with the addressing of load_tile2_fast; STEPS row pairs from plane z0
+template <bool CH, int STEPS, typename S, typename T>
 __device__ __forceinline__ void store_tile_own_fast(const Box &b, const BrickId &br, const Tile &t,
                                                     const S *__restrict__ s, T *__restrict__ g,
                                                     T *__restrict__ face, bool add_mode, int lane,
-                                                    const ChebOut<T> *co) {
+                                                    const ChebOut<T> *co, int z0) {
   const FastLane L = fast_lane(b, lane);
   const bool ownx = L.ii < 2 * BE || br.bx == b.nbx - 1;
   const bool lasty = br.by == b.nby - 1, lastz = br.bz == b.nbz - 1;
-  T *gb = g + 3 * t.node0;
+  const int64_t node0 = t.node0 + (int64_t)b.NX * b.NY * z0;
+  s += TPS * z0;
+  T *gb = g + 3 * node0;
   T *fo = face + (int64_t)br.lin * FACEVALS + L.c;
   if constexpr (CH) {
     // the update's operands of a chunk of steps are all loaded before the first is used (one
     // exposed memory latency per chunk, not per step); every tile address is inside the box
-    constexpr int CHUNK = sizeof(T) == 4 ? TPAIRS : 14;
-    const T *bb = co->b + 3 * t.node0, *bd = co->dinv + 3 * t.node0, *bx = co->x + 3 * t.node0;
-    const T *bp = co->pkm1 ? co->pkm1 + 3 * t.node0 : nullptr;
-    const uint8_t *bm = co->mask ? co->mask + 3 * t.node0 : nullptr;
-    T *bo = co->out + 3 * t.node0;
+    constexpr int CHUNK = sizeof(T) == 4 ? STEPS : 14;
+    const T *bb = co->b + 3 * node0, *bd = co->dinv + 3 * node0, *bx = co->x + 3 * node0;
+    const T *bp = co->pkm1 ? co->pkm1 + 3 * node0 : nullptr;
+    const uint8_t *bm = co->mask ? co->mask + 3 * node0 : nullptr;
+    T *bo = co->out + 3 * node0;
 #pragma unroll
-    for (int c0 = 0; c0 < TPAIRS; c0 += CHUNK) {
+    for (int c0 = 0; c0 < STEPS; c0 += CHUNK) {
       T vb[CHUNK], vd[CHUNK], vx[CHUNK], vp[CHUNK];
       int vm[CHUNK];
 #pragma unroll
       for (int k = 0; k < CHUNK; k++) {
         const int it = c0 + k;
-        if (it >= TPAIRS) break;
-        const uint32_t e = fast_eoff(b, L, it);
+        if (it >= STEPS) break;
+        const uint32_t e = fast_eoff<STEPS>(b, L, it);
         vb[k] = fast_at(bb, e);
         vd[k] = fast_at(bd, e);
         vx[k] = fast_at(bx, e);
@@ -483,13 +498,14 @@ __device__ __forceinline__ void store_tile_own_fast(const Box &b, const BrickId 
 #pragma unroll
       for (int k = 0; k < CHUNK; k++) {
         const int it = c0 + k;
-        if (it >= TPAIRS) break;
-        if (!fast_stores(L, it)) continue;
+        if (it >= STEPS) break;
+        if (!fast_stores<STEPS>(L, it)) continue;
         int y, z;
         fast_row(L, it, y, z);
+    z += z0;
         const bool owny = y < 2 * BE || lasty, ownz = z < 2 * BE || lastz;
         const S val = s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)];
-        const uint32_t e = fast_eoff(b, L, it);
+        const uint32_t e = fast_eoff<STEPS>(b, L, it);
         if (ownx && owny && ownz) {
           const bool lower = (L.ii == 0 && br.bx > 0) || (y == 0 && br.by > 0) || (z == 0 && br.bz > 0);
           if (vm[k] || !lower) {
@@ -505,21 +521,22 @@ __device__ __forceinline__ void store_tile_own_fast(const Box &b, const BrickId 
     }
     return;
   }
-  T v[TPAIRS];
+  T v[STEPS];
   if (add_mode) {
 #pragma unroll
-    for (int it = 0; it < TPAIRS; it++) v[it] = fast_at(gb, fast_eoff(b, L, it));
+    for (int it = 0; it < STEPS; it++) v[it] = fast_at(gb, fast_eoff<STEPS>(b, L, it));
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
-  for (int it = 0; it < TPAIRS; it++) {
-    if (!fast_stores(L, it)) continue;
+  for (int it = 0; it < STEPS; it++) {
+    if (!fast_stores<STEPS>(L, it)) continue;
     int y, z;
     fast_row(L, it, y, z);
+    z += z0;
     const bool owny = y < 2 * BE || lasty, ownz = z < 2 * BE || lastz;
     const S val = s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)];
     if (ownx && owny && ownz) {
-      fast_at(gb, fast_eoff(b, L, it)) = add_mode ? T(v[it] + val) : T(val);
+      fast_at(gb, fast_eoff<STEPS>(b, L, it)) = add_mode ? T(v[it] + val) : T(val);
     } else {
       const int slot = !ownx ? z * TN + y : (!owny ? TN * TN + z * TN + L.ii : 2 * TN * TN + y * TN + L.ii);
       fo[3 * slot] = T(val);
@@ -529,13 +546,14 @@ __device__ __forceinline__ void store_tile_own_fast(const Box &b, const BrickId 
 
 // CH: the Chebyshev update of co is applied to every owned node that is final here (see
 // store_tile_own_fast); the others are stored into g for the face pass.
-template <bool CH = false, typename S, typename T>
+// STEPS row pairs from plane z0: the whole tile, or one wave's third of it.
+template <bool CH = false, int STEPS = TPAIRS, typename S, typename T>
 __device__ __forceinline__ void store_tile_own(const Box &b, const BrickId &br, const Tile &t, const S *__restrict__ s,
                                                T *__restrict__ g, T *__restrict__ face, bool add_mode, int lane,
-                                               const ChebOut<T> *co = nullptr) {
+                                               const ChebOut<T> *co = nullptr, int z0 = 0) {
   asm volatile("" : "+v"(lane));  // see store_tile
   if (tile_fast(b, t)) {
-    store_tile_own_fast<CH>(b, br, t, s, g, face, add_mode, lane, co);
+    store_tile_own_fast<CH, STEPS>(b, br, t, s, g, face, add_mode, lane, co, z0);
     return;
   }
   const TileLane L = tile_lane(b, t, br, lane);
@@ -544,20 +562,23 @@ __device__ __forceinline__ void store_tile_own(const Box &b, const BrickId &br, 
   const bool ownx = ii < 2 * BE || br.bx == b.nbx - 1;
   const bool lasty = br.by == b.nby - 1, lastz = br.bz == b.nbz - 1;
   T *fo = face + (int64_t)br.lin * FACEVALS + c;
-  T v[TPAIRS];
+  T v[STEPS];
   if (add_mode) {
 #pragma unroll
-    for (int it = 0; it < TPAIRS; it++) {
+    for (int it = 0; it < STEPS; it++) {
       int y, z;
       tile_row(it, L, y, z);
+      z += z0;
       v[it] = g[tile_gidx(t, L, y, z)];
     }
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
-  for (int it = 0; it < TPAIRS; it++) {
+  for (int it = 0; it < STEPS; it++) {
     int y, z;
     tile_row(it, L, y, z);
+    if (STEPS < TPAIRS && z >= WPLANES) continue;
+    z += z0;
     if (!(L.col_ok && y < t.tny && z < t.tnz)) continue;
     const bool owny = y < 2 * BE || lasty, ownz = z < 2 * BE || lastz;
     const S val = s[L.lds_col + TRS * y + TPS * z];

@@ -14,7 +14,7 @@ struct ChebOut;
 constexpr int BATCH_MAX = 16;
 template <typename T>
 struct BatchArgs {
-  int n, add;
+  int n, mode;  // mode: OutMode
   int start[BATCH_MAX + 1];
   Box box[BATCH_MAX];
   const T *u[BATCH_MAX];
@@ -26,6 +26,10 @@ struct BatchArgs {
 };
 template <typename T>
 hipError_t launch_a11_batch(const BatchArgs<T> &a, hipStream_t s);
+
+// what an A11 or block launch does to y: y = sum, y += sum, or y = sum with y = u on the Dirichlet
+// dofs of the mask (MatMult semantics)
+enum OutMode { OUT_SET = 0, OUT_ADD = 1, OUT_BC = 2 };
 
 // error bits raised by validation kernels into a device int
 constexpr int ERRBIT_MESH = 1;
@@ -39,13 +43,13 @@ constexpr int ERRBIT_NONFINITE = 4;
 // co (one-launch path only): the owned nodes that no face slot adds to get the Chebyshev update
 // of co instead of being stored into y (the face pass updates the rest)
 hipError_t launch_a11_fp64(const Box &b, const double *coords, const double *u, const uint8_t *mask,
-                           const double *eta_bm, double *y, bool add, hipStream_t s, double *facebuf = nullptr,
+                           const double *eta_bm, double *y, OutMode mode, hipStream_t s, double *facebuf,
                            bool gather = true, const ChebOut<double> *co = nullptr);
 // the full block [A11 A12; A21 0] in one element pass (FP64); fp (27 per element, may be null)
 // subtracts the continuity source from yp
 hipError_t launch_stokes_fp64(const Box &b, const double *coords, const double *u, const double *p,
                               const uint8_t *mask, const double *eta_bm, double *yu, double *yp, const double *fp,
-                              bool add, hipStream_t s, double *facebuf = nullptr);
+                              bool add, hipStream_t s, double *facebuf);
 hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, const float *fac, float *y, bool add,
                            hipStream_t s, float *facebuf = nullptr, bool gather = true,
                            const ChebOut<float> *co = nullptr);
@@ -60,7 +64,8 @@ hipError_t launch_a11_fp32_split(const Box &b, const float *u, const uint8_t *ma
 // (ptq2_mfma.hip); one-launch output path only
 hipError_t launch_a11_fp32_mfma(const Box &b, const float *u, const uint8_t *mask, const float *fac, float *y,
                                 bool add, hipStream_t s, float *facebuf, bool gather = true);
-// the face pass alone (adds the face slots of facebuf into their owners)
+// the face pass alone (adds the face slots of facebuf into their owners; not into the dofs of mask,
+// if given)
 hipError_t launch_gather_faces(const Box &b, const float *face, float *y, hipStream_t s);
 hipError_t launch_gather_faces(const Box &b, const double *face, double *y, hipStream_t s);
 hipError_t launch_build_fac32(const Box &b, const double *coords, const double *eta_bm, float *fac, float *facb,
@@ -72,7 +77,8 @@ hipError_t launch_stokes_fp32(const Box &b, const float *u, const float *p, cons
                               const float *facb, float *yu, float *yp, bool add, hipStream_t s,
                               float *facebuf = nullptr);
 hipError_t launch_eta_to_bm(const Box &b, const double *eta, double *eta_bm, int *err, hipStream_t s);
-hipError_t launch_check_mesh(const Box &b, const double *coords, int *err, hipStream_t s);
+// validates the mesh and, if xtile is not null, writes the resident coordinate tiles (Box::xtile)
+hipError_t launch_check_mesh(const Box &b, const double *coords, double *xtile, int *err, hipStream_t s);
 hipError_t launch_a21(const Box &b, const double *coords, const double *u, const uint8_t *mask, double *yp, bool add,
                       hipStream_t s);
 hipError_t launch_a12(const Box &b, const double *coords, const double *p, double *y, bool add, hipStream_t s);

@@ -6,6 +6,7 @@
 // element per lane (see ptq2_device.h for the brick/tile decomposition).
 #include "ptq2_device.h"
 #include "ptq2_kernels.h"
+#include "ptq2_comp.h"
 
 #include <algorithm>
 
@@ -164,19 +165,18 @@ __device__ __forceinline__ void load3(const double *__restrict__ ep, int row, do
   for (int q = 0; q < 3; q++) e3[q] = ep[(3 * row + q) * BEL];
 }
 
-// BLK = false: the A11 apply.  BLK = true: the full block [A11 A12; A21 0] in the same single
-// element pass (MFStokesWrapper_A_AVX, src/stokes_operators_avx.c:439-636): y gets A11 u + A12 p,
-// yp gets A21 u (and, with fp, minus the continuity source: FormFunctionLocal_P's
-// -int N^p fp, src/stokes_form_function.c:478-580).
-// CH: store with the fused Chebyshev update of co (store_tile_own<true>).
-// The brick br of box b (one wave); k_a11_fp64_t and the batched k_a11_fp64_batch resolve br.
-template <bool BLK, bool CH>
-__device__ __forceinline__ void a11_fp64_brick(const Box &b, const BrickId &br, int color,
-                                               const double *__restrict__ coords, const double *__restrict__ u,
-                                               const uint8_t *__restrict__ mask, const double *__restrict__ eta_bm,
-                                               double *__restrict__ y, int add_mode, double *__restrict__ facebuf,
-                                               const double *__restrict__ p, double *__restrict__ yp,
-                                               const double *__restrict__ fp, const ChebOut<double> &co) {
+// The full block [A11 A12; A21 0] in one element pass, one wave per brick
+// (MFStokesWrapper_A_AVX, src/stokes_operators_avx.c:439-636): yu gets A11 u + A12 p, yp gets A21 u
+// (and, with fp, minus the continuity source: FormFunctionLocal_P's -int N^p fp,
+// src/stokes_form_function.c:478-580).
+__global__ __launch_bounds__(BEL) void k_stokes_fp64(Box b, const double *__restrict__ coords,
+                                                     const double *__restrict__ u, const uint8_t *__restrict__ mask,
+                                                     const double *__restrict__ eta_bm, double *__restrict__ y,
+                                                     int add_mode, double *__restrict__ facebuf,
+                                                     const double *__restrict__ p, double *__restrict__ yp,
+                                                     const double *__restrict__ fp) {
+  constexpr bool BLK = true;
+  const BrickId br = brick_xcd(b, blockIdx.x);
   __shared__ double Xs[3 * TCS];
   __shared__ double Us[3 * TCS];
   const int lane = threadIdx.x;
@@ -199,7 +199,7 @@ __device__ __forceinline__ void a11_fp64_brick(const Box &b, const BrickId &br, 
         for (int i = 0; i < 3; i++) Y[c][k][j][i] = 0.0;
   BlockState bs;
   int64_t e = 0;
-  if constexpr (BLK) {
+  {
     bs.Yp[0] = bs.Yp[1] = bs.Yp[2] = bs.Yp[3] = 0.0;
     bs.pe[0] = bs.pe[1] = bs.pe[2] = bs.pe[3] = 0.0;
     bs.fp = nullptr;
@@ -214,66 +214,33 @@ __device__ __forceinline__ void a11_fp64_brick(const Box &b, const BrickId &br, 
   if (active) {
     double ca[9], cb9[9];
     ld_col(Xs, base, 0, ca);
-    if constexpr (!BLK) {
-      // slab form of the y/z transposes (the full block keeps the per-row form: with its
-      // pressure state the slab sums would spill)
 #pragma nounroll
-      for (int qc = 0; qc < 3; qc++) {
-        double RB[3][3][3], RD[3][3][3];
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-#pragma unroll
-          for (int j = 0; j < 3; j++)
-#pragma unroll
-            for (int i = 0; i < 3; i++) RB[c][j][i] = RD[c][j][i] = 0.0;
-#pragma nounroll
-        for (int qb = 0; qb < 3; qb++) {
-          const int row = qb + 3 * qc;
-          double e3[3] = {en[0], en[1], en[2]};
-          if (row < 8) load3(ep, row + 1, en);
-          a11_row64<BLK, true>(Xs, Us, base, coef1(qb), coef1(qc), c_gw[qb] * c_gw[qc], e3, ca, cb9, Y, row, &bs,
-                               RB, RD);
-        }
-        acc_slab_rt(coef1(qc), RB, RD, Y);
-        row_fence();
-      }
-    } else {
-#pragma nounroll
-      for (int row = 0; row < 9; row++) {
-        const int qb = row % 3, qc = row / 3;
-        double e3[3] = {en[0], en[1], en[2]};
-        if (row < 8) load3(ep, row + 1, en);
-        a11_row64<BLK>(Xs, Us, base, coef1(qb), coef1(qc), c_gw[qb] * c_gw[qc], e3, ca, cb9, Y, row, &bs);
-      }
+    for (int row = 0; row < 9; row++) {
+      const int qb = row % 3, qc = row / 3;
+      double e3[3] = {en[0], en[1], en[2]};
+      if (row < 8) load3(ep, row + 1, en);
+      a11_row64<BLK>(Xs, Us, base, coef1(qb), coef1(qc), c_gw[qb] * c_gw[qc], e3, ca, cb9, Y, row, &bs);
     }
-    if constexpr (BLK) {
-      double *o = yp + 4 * e;
+    double *o = yp + 4 * e;
 #pragma unroll
-      for (int i = 0; i < 4; i++) o[i] = add_mode ? o[i] + bs.Yp[i] : bs.Yp[i];
-    }
+    for (int i = 0; i < 4; i++) o[i] = add_mode ? o[i] + bs.Yp[i] : bs.Yp[i];
   }
   __syncthreads();
   zero_tile(Xs, lane);
   __syncthreads();
   if (active) emit_element(Xs, base, Y);
   __syncthreads();
-  if (color >= 0)
-    store_tile(b, br, t, Xs, y, add_mode != 0, lane);
-  else if constexpr (CH)
-    store_tile_own<true>(b, br, t, Xs, y, facebuf, false, lane, &co);
-  else
-    store_tile_own(b, br, t, Xs, y, facebuf, add_mode != 0, lane);
+  store_tile_own(b, br, t, Xs, y, facebuf, add_mode != 0, lane);
 }
 
-template <bool BLK, bool CH>
-__global__ __launch_bounds__(BEL) void k_a11_fp64_t(Box b, int color, const double *__restrict__ coords,
-                                                    const double *__restrict__ u, const uint8_t *__restrict__ mask,
-                                                    const double *__restrict__ eta_bm, double *__restrict__ y,
-                                                    int add_mode, double *__restrict__ facebuf,
-                                                    const double *__restrict__ p, double *__restrict__ yp,
-                                                    const double *__restrict__ fp, ChebOut<double> co) {
-  const BrickId br = color >= 0 ? brick_of(b, color, blockIdx.x) : brick_xcd(b, blockIdx.x);
-  a11_fp64_brick<BLK, CH>(b, br, color, coords, u, mask, eta_bm, y, add_mode, facebuf, p, yp, fp, co);
+template <bool CH>
+__global__ __launch_bounds__(CWAVES * BEL, 2) void k_a11_fp64_t(Box b, const double *__restrict__ coords,
+                                                                const double *__restrict__ u,
+                                                                const uint8_t *__restrict__ mask,
+                                                                const double *__restrict__ eta_bm,
+                                                                double *__restrict__ y, int mode,
+                                                                double *__restrict__ facebuf, ChebOut<double> co) {
+  a11_fp64_brick<CH>(b, brick_xcd(b, blockIdx.x), coords, u, mask, eta_bm, y, mode, facebuf, co);
 }
 
 // Several problems in one launch: block i belongs to the problem p with start[p] <= i <
@@ -286,13 +253,13 @@ __device__ __forceinline__ int batch_problem(const int *start, int n, int bid) {
   return p;
 }
 
-__global__ __launch_bounds__(BEL) void k_a11_fp64_batch(BatchArgs<double> a) {
+__global__ __launch_bounds__(CWAVES * BEL, 2) void k_a11_fp64_batch(BatchArgs<double> a) {
   const int p = batch_problem(a.start, a.n, blockIdx.x);
   const Box b = a.box[p];
   const int local = (int)blockIdx.x - a.start[p];
   if (local >= b.nbx * b.nby * b.nbz) return;
-  a11_fp64_brick<false, false>(b, brick_xcd(b, local), -1, a.coords[p], a.u[p], a.mask[p], a.fac[p], a.y[p], a.add,
-                               a.face[p], nullptr, nullptr, nullptr, ChebOut<double>{});
+  a11_fp64_brick<false>(b, brick_xcd(b, local), a.coords[p], a.u[p], a.mask[p], a.fac[p], a.y[p], a.mode, a.face[p],
+                        ChebOut<double>{});
 }
 
 // ----------------------------------------------------------------- A11 FP32
@@ -455,7 +422,7 @@ __global__ __launch_bounds__(BEL) void k_a11_fp32_batch(BatchArgs<float> a) {
   const Box b = a.box[p];
   const int local = (int)blockIdx.x - a.start[p];
   if (local >= b.nbx * b.nby * b.nbz) return;
-  a11_fp32_brick<false>(b, brick_xcd(b, local), -1, a.u[p], a.mask[p], a.fac[p], a.y[p], a.add, a.face[p],
+  a11_fp32_brick<false>(b, brick_xcd(b, local), -1, a.u[p], a.mask[p], a.fac[p], a.y[p], a.mode == OUT_ADD, a.face[p],
                         ChebOut<float>{});
 }
 
@@ -932,13 +899,21 @@ __device__ __forceinline__ void check_row(const double *Xs, int base, int &bad) 
   row_fence();
 }
 
-__global__ __launch_bounds__(BEL) void k_check_mesh(Box b, const double *__restrict__ coords, int *__restrict__ err) {
+// It has every brick's coordinate tile in LDS: with xtile it also writes them out in that layout
+// (Box::xtile), for the tile copies of the FP64 passes.
+__global__ __launch_bounds__(BEL) void k_check_mesh(Box b, const double *__restrict__ coords,
+                                                    double *__restrict__ xtile, int *__restrict__ err) {
   __shared__ double Xs[3 * TCS];
   const int lane = threadIdx.x;
   const BrickId br = brick_lin(b, blockIdx.x);
   const Tile t = tile_of(b, br);
+  zero_tile(Xs, lane);  // the layout's gaps
   load_tile(b, t, br, coords, (const uint8_t *)nullptr, Xs, lane);
   __syncthreads();
+  if (xtile) {
+    double *o = xtile + (int64_t)br.lin * 3 * TCS;
+    for (int n = lane; n < 3 * TCS; n += BEL) o[n] = Xs[n];
+  }
   if (!lane_active(t, lane)) return;
   const int base = lane_base(lane);
   int bad = 0;
@@ -1336,15 +1311,17 @@ static inline int nbricks(const Box &b) { return b.nbx * b.nby * b.nbz; }
 // LDS by one batch of independent loads (the XCD-aware brick order keeps most of them on the
 // same L2 as their writer); then each thread takes up to 3 of the brick's at most 3 x 3 x TN x TN
 // face values.
+// mask: the Dirichlet dofs, which keep their y (OUT_BC), or null.
 template <typename T>
 __device__ __forceinline__ void gather_faces_brick(const Box &b, const BrickId &br, const T *__restrict__ face,
-                                                   T *__restrict__ y) {
+                                                   T *__restrict__ y, const uint8_t *__restrict__ mask) {
   constexpr int F2 = TN * TN, UP = 2 * BE;
   constexpr int OFX = 0, OFY = 3 * F2, OFZ = 6 * F2, OXY = 9 * F2, OXZ = OXY + 3 * TN, OYZ = OXZ + 3 * TN,
                 OC = OYZ + 3 * TN, NS = OC + 3;
   __shared__ T sh[NS];
   const bool hx = br.bx > 0, hy = br.by > 0, hz = br.bz > 0;
   if (!(hx || hy || hz)) return;
+  if (mask && b.bdir && !b.bdir[br.lin]) mask = nullptr;
   const Tile t = tile_of(b, br);
   const int tid = threadIdx.x;
   const int64_t fx = FACEVALS, fy = (int64_t)b.nbx * FACEVALS, fz = (int64_t)b.nbx * b.nby * FACEVALS;
@@ -1380,7 +1357,7 @@ __device__ __forceinline__ void gather_faces_brick(const Box &b, const BrickId &
   const int nX = hx ? oy * oz : 0, nY = hy ? (ox - x0) * oz : 0, nZ = hz ? (ox - x0) * (oy - y0) : 0;
   const int nval = 3 * (nX + nY + nZ);
   int64_t gi[3];
-  int ix[3], iy[3], iz[3], cc[3];
+  int ix[3], iy[3], iz[3], cc[3], dir[3] = {0, 0, 0};
   T own[3];
 #pragma unroll
   for (int m = 0; m < 3; m++) {
@@ -1398,6 +1375,7 @@ __device__ __forceinline__ void gather_faces_brick(const Box &b, const BrickId &
     }
     gi[m] = 3 * (t.node0 + ix[m] + (int64_t)b.NX * (iy[m] + (int64_t)b.NY * iz[m])) + cc[m];
     own[m] = y[gi[m]];
+    if (mask) dir[m] = mask[gi[m]];
   }
 #pragma unroll
   for (int m = 0; m < 3; m++) {
@@ -1412,13 +1390,14 @@ __device__ __forceinline__ void gather_faces_brick(const Box &b, const BrickId &
     if (ny && nx) acc += sh[OXY + c * TN + Z];
     if (ny) acc += sh[OFY + c * F2 + Z * TN + X];
     if (nx) acc += sh[OFX + c * F2 + Z * TN + Y];
-    y[gi[m]] = acc;
+    if (!dir[m]) y[gi[m]] = acc;
   }
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_gather_faces(Box b, const T *__restrict__ face, T *__restrict__ y) {
-  gather_faces_brick(b, brick_xcd(b, blockIdx.x), face, y);
+__global__ __launch_bounds__(256) void k_gather_faces(Box b, const T *__restrict__ face, T *__restrict__ y,
+                                                     const uint8_t *__restrict__ mask) {
+  gather_faces_brick(b, brick_xcd(b, blockIdx.x), face, y, mask);
 }
 
 template <typename T>
@@ -1427,37 +1406,26 @@ __global__ __launch_bounds__(256) void k_gather_faces_batch(BatchArgs<T> a) {
   const Box b = a.box[p];
   const int local = (int)blockIdx.x - a.start[p];
   if (local >= b.nbx * b.nby * b.nbz) return;
-  gather_faces_brick(b, brick_xcd(b, local), (const T *)a.face[p], a.y[p]);
+  gather_faces_brick(b, brick_xcd(b, local), (const T *)a.face[p], a.y[p], a.mode == OUT_BC ? a.mask[p] : nullptr);
 }
 
 template <typename T>
-hipError_t launch_gather(const Box &b, const T *face, T *y, hipStream_t s) {
-  hipLaunchKernelGGL(k_gather_faces<T>, dim3(nbricks(b)), dim3(256), 0, s, b, face, y);
+hipError_t launch_gather(const Box &b, const T *face, T *y, hipStream_t s, const uint8_t *mask = nullptr) {
+  hipLaunchKernelGGL(k_gather_faces<T>, dim3(nbricks(b)), dim3(256), 0, s, b, face, y, mask);
   return hipGetLastError();
 }
 
 hipError_t launch_a11_fp64(const Box &b, const double *coords, const double *u, const uint8_t *mask,
-                           const double *eta_bm, double *y, bool add, hipStream_t s, double *facebuf, bool gather,
+                           const double *eta_bm, double *y, OutMode mode, hipStream_t s, double *facebuf, bool gather,
                            const ChebOut<double> *co) {
-  if (facebuf) {
-    if (co) {
-      hipLaunchKernelGGL((k_a11_fp64_t<false, true>), dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, coords, u, mask, eta_bm,
-                         y, 0, facebuf, (const double *)nullptr, (double *)nullptr, (const double *)nullptr, *co);
-      return hipGetLastError();
-    }
-    hipLaunchKernelGGL((k_a11_fp64_t<false, false>), dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, coords, u, mask, eta_bm, y,
-                       add ? 1 : 0, facebuf, (const double *)nullptr, (double *)nullptr, (const double *)nullptr,
-                       ChebOut<double>{});
-    return gather ? launch_gather(b, (const double *)facebuf, y, s) : hipGetLastError();
+  const dim3 grid(nbricks(b)), block(CWAVES * BEL);
+  if (co) {
+    hipLaunchKernelGGL(k_a11_fp64_t<true>, grid, block, 0, s, b, coords, u, mask, eta_bm, y, (int)OUT_SET, facebuf, *co);
+    return hipGetLastError();
   }
-  for (int c = 0; c < 8; c++) {
-    int nb = nbricks_color(b, c);
-    if (nb == 0) continue;
-    hipLaunchKernelGGL((k_a11_fp64_t<false, false>), dim3(nb), dim3(BEL), 0, s, b, c, coords, u, mask, eta_bm, y, add ? 1 : 0,
-                       (double *)nullptr, (const double *)nullptr, (double *)nullptr, (const double *)nullptr,
-                       ChebOut<double>{});
-  }
-  return hipGetLastError();
+  hipLaunchKernelGGL(k_a11_fp64_t<false>, grid, block, 0, s, b, coords, u, mask, eta_bm, y, (int)mode, facebuf,
+                     ChebOut<double>{});
+  return gather ? launch_gather(b, (const double *)facebuf, y, s, mode == OUT_BC ? mask : nullptr) : hipGetLastError();
 }
 
 hipError_t launch_gather_faces(const Box &b, const float *face, float *y, hipStream_t s) {
@@ -1488,7 +1456,7 @@ template <typename T>
 hipError_t launch_a11_batch(const BatchArgs<T> &a, hipStream_t s) {
   const int nb = a.start[a.n];
   if constexpr (sizeof(T) == 8)
-    hipLaunchKernelGGL(k_a11_fp64_batch, dim3(nb), dim3(BEL), 0, s, a);
+    hipLaunchKernelGGL(k_a11_fp64_batch, dim3(nb), dim3(CWAVES * BEL), 0, s, a);
   else
     hipLaunchKernelGGL(k_a11_fp32_batch, dim3(nb), dim3(BEL), 0, s, a);
   hipError_t e = hipGetLastError();
@@ -1502,18 +1470,9 @@ template hipError_t launch_a11_batch<float>(const BatchArgs<float> &, hipStream_
 hipError_t launch_stokes_fp64(const Box &b, const double *coords, const double *u, const double *p,
                               const uint8_t *mask, const double *eta_bm, double *yu, double *yp, const double *fp,
                               bool add, hipStream_t s, double *facebuf) {
-  if (facebuf) {
-    hipLaunchKernelGGL((k_a11_fp64_t<true, false>), dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, coords, u, mask, eta_bm, yu,
-                       add ? 1 : 0, facebuf, p, yp, fp, ChebOut<double>{});
-    return launch_gather(b, (const double *)facebuf, yu, s);
-  }
-  for (int c = 0; c < 8; c++) {
-    int nb = nbricks_color(b, c);
-    if (nb == 0) continue;
-    hipLaunchKernelGGL((k_a11_fp64_t<true, false>), dim3(nb), dim3(BEL), 0, s, b, c, coords, u, mask, eta_bm, yu,
-                       add ? 1 : 0, (double *)nullptr, p, yp, fp, ChebOut<double>{});
-  }
-  return hipGetLastError();
+  hipLaunchKernelGGL(k_stokes_fp64, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, u, mask, eta_bm, yu, add ? 1 : 0,
+                     facebuf, p, yp, fp);
+  return launch_gather(b, (const double *)facebuf, yu, s);
 }
 
 hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, const float *fac, float *y, bool add,
@@ -1586,8 +1545,8 @@ hipError_t launch_eta_to_bm(const Box &b, const double *eta, double *eta_bm, int
   return hipGetLastError();
 }
 
-hipError_t launch_check_mesh(const Box &b, const double *coords, int *err, hipStream_t s) {
-  hipLaunchKernelGGL(k_check_mesh, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, err);
+hipError_t launch_check_mesh(const Box &b, const double *coords, double *xtile, int *err, hipStream_t s) {
+  hipLaunchKernelGGL(k_check_mesh, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, xtile, err);
   return hipGetLastError();
 }
 

@@ -1264,8 +1264,8 @@ hipError_t level_launch(ptq2_mg *mg, int l, const double *x, double *y, bool gat
   if (mg->tune[l].split == 1 && !mg->f32)
     return ptq2::launch_a11_fp64_split(b, c->coords, x, c->mask, c->eta_bm, y, false, mg->stream,
                                        (double *)c->facebuf, gather);
-  return ptq2::launch_a11_fp64(b, c->coords, x, c->mask, c->eta_bm, y, false, mg->stream, (double *)c->facebuf,
-                               gather);
+  return ptq2::launch_a11_fp64(b, c->coords, x, c->mask, c->eta_bm, y, ptq2::OUT_SET, mg->stream,
+                               (double *)c->facebuf, gather);
 }
 hipError_t level_launch(ptq2_mg *mg, int l, const float *x, float *y, bool gather) {
   ptq2_ctx *c = mg->ctx[l];
@@ -1334,8 +1334,8 @@ int level_apply_cheb(ptq2_mg *mg, int l, const T *x, T *y, const ptq2::ChebOut<T
 template <>
 int level_apply_cheb<double>(ptq2_mg *mg, int l, const double *x, double *y, const ptq2::ChebOut<double> &co) {
   ptq2_ctx *c = mg->ctx[l];
-  MGCHK(ptq2::launch_a11_fp64(mg->lbox[l], c->coords, x, c->mask, c->eta_bm, y, false, mg->stream, (double *)c->facebuf,
-                              false, &co));
+  MGCHK(ptq2::launch_a11_fp64(mg->lbox[l], c->coords, x, c->mask, c->eta_bm, y, ptq2::OUT_SET, mg->stream,
+                              (double *)c->facebuf, false, &co));
   return PTQ2_OK;
 }
 template <>

@@ -1,0 +1,55 @@
+"""Element passes on several waves per brick: meshes at the edges of the 4x4x4 bricks, scattered
+Dirichlet masks, and the resident coordinate tiles of large meshes, against the oracle.
+
+Tolerance: an output node sums up to 8 elements x 27 points x ~30 rounded products of FP64, whose
+errors add like a random walk to well below 1e-14 of the result; 1e-12 (the operators' bar)
+leaves room for cancellation between the elements of a stiff inclusion."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+import ptq2
+from ptq2 import _lib
+from ptq2 import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+DEV = torch.device("cuda:0")
+
+EDGES = [(1, 1, 1), (4, 4, 4), (5, 4, 4), (4, 9, 3), (8, 8, 8), (12, 5, 8), (3, 13, 17)]
+
+
+def problem(dims, seed=5, mask_share=0.05):
+    mx, my, mz = dims
+    c = M.jitter(mx, my, mz, M.q2_uniform(mx, my, mz), 0.1, 1.0 / (2 * max(dims)), seed)
+    eta = 10.0 ** M.uniform(seed + 1, 27 * mx * my * mz, -2.0, 2.0)
+    n = 3 * M.nnodes(mx, my, mz)
+    # whole Dirichlet faces in x, and single dofs anywhere (inside bricks, on their faces and edges)
+    mask = (M.uniform(seed + 2, n) < mask_share).astype(np.uint8)
+    mask.reshape(-1, 2 * mx + 1, 3)[:, 0, :] = 1
+    return M.Problem(mx, my, mz, M.affine(c, M.SHEAR, [0.0, 0.0, 0.0]), mask, eta)
+
+
+def rel(a, b):
+    return float(np.linalg.norm(np.asarray(a, dtype=np.float64) - b) / np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("dims", EDGES + [(128, 128, 32)])
+def test_a11_fp64(dims):
+    """Raw, ADD and MatMult applies; Dirichlet rows are u's bit for bit, ADD adds to what is there."""
+    print("case: A11 FP64", dims, flush=True)
+    P = problem(dims)
+    A = ptq2.MatA11MF("hip")
+    A.setup(P)
+    u = M.uniform(3, P.nvel, -1.0, 1.0)
+    ud = torch.from_numpy(u).to(DEV)
+    ref = O.a11_tensor(*dims, P.coords, P.eta, u, threads=8)
+    y = A.ctx.a11(ud)
+    assert rel(y.cpu().numpy(), ref) <= 1e-12
+    y0 = torch.full_like(ud, 0.5)
+    assert rel(A.ctx.a11(ud, y0.clone(), _lib.ADD).cpu().numpy(), ref + 0.5) <= 1e-12
+    ym = A.mult(ud).cpu().numpy()
+    assert rel(ym, O.matmult_a11(*dims, P.coords, P.eta, P.mask, u)) <= 1e-12
+    d = P.mask > 0
+    assert np.array_equal(ym[d], u[d])
