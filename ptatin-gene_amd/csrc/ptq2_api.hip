@@ -376,6 +376,9 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   b.xtile = c->xtile;
   c->box = b;
   c->nnodes = nn; c->nvel = 3 * nn; c->nel = ne; c->npres = 4 * ne; c->nbricks = nb;
+  // the face slots now, so that no operator's first call allocates (it may be under capture); where they
+  // do not fit, that call says so
+  (void)ptq2_internal_facebuf(c, &rc);
   if ((rc = clear_err(c))) return rc;
   HIPCHK(c, ptq2::launch_check_mesh(b, c->coords, c->xtile, c->err, c->stream));
   int bits = 0;
@@ -627,7 +630,9 @@ int ptq2_a11_diag(ptq2_ctx *c, double *d, unsigned flags) {
     if (add) HIPCHK(c, hipMemcpyAsync(c->sy, d, sizeof(double) * (size_t)n, hipMemcpyHostToDevice, c->stream));
     dd = (double *)c->sy;
   }
-  HIPCHK(c, ptq2::launch_diag(c->box, c->coords, c->eta_bm, dd, add, c->stream));
+  void *fb = ptq2_internal_facebuf(c, &rc);
+  if (rc) return rc;
+  HIPCHK(c, ptq2::launch_diag(c->box, c->coords, c->eta_bm, dd, add, (double *)fb, c->stream));
   if (mm) HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, (const double *)nullptr, dd, 2, c->stream));
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(d, dd, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, c->stream));
@@ -654,7 +659,9 @@ int ptq2_a12_apply(ptq2_ctx *c, const double *p, double *yu, unsigned flags) {
     dp = c->sp;
     dy = (double *)c->sy;
   }
-  HIPCHK(c, ptq2::launch_a12(c->box, c->coords, dp, dy, add, c->stream));
+  void *fb = ptq2_internal_facebuf(c, &rc);
+  if (rc) return rc;
+  HIPCHK(c, ptq2::launch_a12(c->box, c->coords, dp, dy, add, (double *)fb, c->stream));
   if (mm) HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, (const double *)nullptr, dy, 1, c->stream));
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(yu, dy, sizeof(double) * (size_t)c->nvel, hipMemcpyDeviceToHost, c->stream));
@@ -776,7 +783,7 @@ int ptq2_stokes_apply(ptq2_ctx *c, const void *u, const void *p, void *yu, void 
       // resident geometry: the A11 kernel of that form, then A12 and A21
       HIPCHK(c, ptq2::launch_a11_fp64g(c->box, (const double *)du, mask, c->geo64, c->eta_bm, (double *)dyu, add,
                                        c->stream, (double *)fb));
-      HIPCHK(c, ptq2::launch_a12(c->box, c->coords, (const double *)dp, (double *)dyu, true, c->stream));
+      HIPCHK(c, ptq2::launch_a12(c->box, c->coords, (const double *)dp, (double *)dyu, true, (double *)fb, c->stream));
       HIPCHK(c, ptq2::launch_a21(c->box, c->coords, (const double *)du, mask, (double *)dyp, add, c->stream));
     }
     if (mm)

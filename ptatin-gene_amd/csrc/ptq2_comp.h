@@ -106,10 +106,11 @@ __device__ __forceinline__ void modal27(double v[27]) {
 // slab: g[d][qa].  v[0..8] holds the slab's values along z and
 // v[9..17] its derivatives, per modal (x, y) coefficient: in slab 1 (z = 0), which runs first, these
 // are m and b themselves; fold_slab0 and fold_slab2 turn them into those of the next slab.
+// r0: the row's values (no derivative) per modal x coefficient.
 template <int QB>
-__device__ __forceinline__ void row_grad(const double v[18], double g[3][3]) {
+__device__ __forceinline__ void row_grad(const double v[18], double g[3][3], double r0[3]) {
   constexpr double sy = QB == 0 ? -1.0 : 1.0;
-  double r0[3], r1[3], r2[3];
+  double r1[3], r2[3];
 #pragma unroll
   for (int i = 0; i < 3; i++) {
     const double *ZB = v + i, *ZD = v + 9 + i;  // stride 3 in y
@@ -134,6 +135,11 @@ __device__ __forceinline__ void row_grad(const double v[18], double g[3][3]) {
   const double p2 = fma(MOD_V2, r2[2], r2[0]);
   g[2][0] = fma(-MOD_V1, r2[1], p2);
   g[2][2] = fma(MOD_V1, r2[1], p2);
+}
+template <int QB>
+__device__ __forceinline__ void row_grad(const double v[18], double g[3][3]) {
+  double r0[3];
+  row_grad<QB>(v, g, r0);
 }
 // slab 1 -> slab 0; a[n] gets the z direction's a, which slab 2 needs (u0: layer 0, still nodal)
 __device__ __forceinline__ void fold_slab0(double v[18], double u0[9], double a[9]) {
@@ -681,69 +687,18 @@ __device__ __forceinline__ void load_tiles_full(const Box &b, const BrickId &br,
   }
 }
 
-// The owner-writes store of a full tile.  A row's nodes go to y, except the last column (the X plane of
-// the face slot, slot number = row number), the row y = 8 (Y plane) and the plane z = 8 (Z plane)
-// where a neighbour owns them; each lane's target is one of two bases and the row's offset from it.
-// U wave w stores the planes 3 w .. 3 w + 2 up to 7, the G wave the plane 8.
-template <int STEPS, int ROWS>
-__device__ __forceinline__ void store_rows_full(const Box &b, const BrickId &br, const Tile &t,
-                                                const double *__restrict__ s, double *__restrict__ g,
-                                                double *__restrict__ face, bool add_mode, int z0, int lane) {
-  constexpr int E = ROWS % 2 ? STEPS : STEPS + 1;  // an even row count has no half-empty last pair
-  const FastLane L = fast_lane(b, lane);
-  const bool ownx = L.ii < 2 * BE || br.bx == b.nbx - 1;
-  const bool lasty = br.by == b.nby - 1, ownz = z0 < 2 * BE || br.bz == b.nbz - 1;
-  double *gb = g + 3 * (t.node0 + (int64_t)b.NX * b.NY * z0);
-  double *fo = face + (int64_t)br.lin * FACEVALS;
-  s += TPS * z0;
-  double val[STEPS];
-#pragma unroll
-  for (int it = 0; it < STEPS; it++) val[it] = s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)];
-  if (add_mode && ownz) {
-    double old[STEPS];
-#pragma unroll
-    for (int it = 0; it < STEPS; it++) old[it] = fast_at(gb, fast_eoff<E>(b, L, it));
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int it = 0; it < STEPS; it++) {
-      int y, z;
-      fast_row(L, it, y, z);
-      if (ownx && (y < 2 * BE || lasty)) val[it] += old[it];
-    }
-  }
-  if (L.p > 1) return;
-  const int odd = L.p;
-  double *by = fo + 3 * TN * (TN + z0) + L.col;
-  // One store per row pair and no branches: a lane's base is y or, in a last column that a neighbour
-  // owns, the X plane (row r of the group at 3 r + c); the rows y = 8 of an inner brick go to the Y plane.
-  char *base = reinterpret_cast<char *>(ownx ? gb : fo + 3 * TN * z0 + L.c);
-  double *bz = ownx ? fo + 3 * TN * 2 * TN + L.col : fo + 3 * TN * z0 + L.c;
-#pragma unroll
-  for (int it = 0; it < STEPS; it++) {
-    const int r0 = 2 * it;                                                // the even lanes' row of the group
-    const bool top0 = r0 % TN == 2 * BE, top1 = (r0 + 1) % TN == 2 * BE;  // rows y = 8
-    double *at;
-    if (ownz)
-      at = reinterpret_cast<double *>(base + (ownx ? 8u * fast_eoff<E>(b, L, it) : 24u * (uint32_t)(r0 + odd)));
-    else
-      at = bz + (ownx ? 3 * TN * (r0 + odd) : 3 * (r0 + odd));  // the plane z = 8: Z plane [y][x]
-    if ((top0 || top1) && !lasty) {
-      const bool toy = ownx && (top0 ? odd == 0 : odd == 1);
-      at = toy ? by + 3 * TN * ((top0 ? r0 : r0 + 1) / TN) : at;
-    }
-    if (2 * it + 1 < ROWS || odd == 0) *at = val[it];
-  }
-}
+// The owner-writes store of a full tile: U wave w stores the planes 3 w .. 3 w + 2 up to 7, the G wave the
+// plane 8.
 __device__ __forceinline__ void store_tile_full(const Box &b, const BrickId &br, const Tile &t,
                                                 const double *__restrict__ s, double *__restrict__ g,
                                                 double *__restrict__ face, bool add_mode, int w, int lane) {
   asm volatile("" : "+v"(lane));  // see store_tile
   if (w < 2)
-    store_rows_full<WSTEPS, 3 * TN>(b, br, t, s, g, face, add_mode, WPLANES * w, lane);
+    store_rows_full<3 * TN>(b, br, t, s, g, face, add_mode, WPLANES * w, lane);
   else if (w == 2)
-    store_rows_full<TN, 2 * TN>(b, br, t, s, g, face, add_mode, 2 * WPLANES, lane);
+    store_rows_full<2 * TN>(b, br, t, s, g, face, add_mode, 2 * WPLANES, lane);
   else
-    store_rows_full<(TN + 1) / 2, TN>(b, br, t, s, g, face, add_mode, 2 * BE, lane);
+    store_rows_full<TN>(b, br, t, s, g, face, add_mode, 2 * BE, lane);
 }
 
 __device__ __forceinline__ void g_wave(double *lds, int lane) {

@@ -223,9 +223,8 @@ __host__ __device__ __forceinline__ void fast_row(const FastLane &L, int it, int
   y = fast_wrap(it) ? (odd ? 0 : y0) : y0 + odd;
   z = fast_wrap(it) ? z0 + odd : z0;
 }
-template <int STEPS = TPAIRS>
 __host__ __device__ __forceinline__ bool fast_stores(const FastLane &L, int it) {
-  return L.p == 0 || (L.p == 1 && it < STEPS - 1);
+  return L.p == 0 || (L.p == 1 && it < TPAIRS - 1);
 }
 // element e of a field from a wave-uniform base: the byte offset is formed in 32 bits, so the
 // access is one global instruction with a scalar base and a 32-bit vector offset
@@ -458,94 +457,123 @@ __host__ __device__ __forceinline__ T cheb_update(const ChebOut<T> &co, int64_t 
   return cheb_value(co, co.dinv[i], co.b[i], y, co.x[i], co.pkm1 ? co.pkm1[i] : T(0), co.pkm1 != nullptr);
 }
 
-// the full-tile case with the addressing of load_tile2_fast; STEPS row pairs from plane z0
-template <bool CH, int STEPS, typename S, typename T>
-__device__ __forceinline__ void store_tile_own_fast(const Box &b, const BrickId &br, const Tile &t,
-                                                    const S *__restrict__ s, T *__restrict__ g,
-                                                    T *__restrict__ face, bool add_mode, int lane,
-                                                    const ChebOut<T> *co, int z0) {
+// The owner-writes store of ROWS rows of a full tile from plane z0 on; they lie below the plane z = 8 or
+// are that plane.  A row's nodes go to y, except the last column (the X plane of the face slot, slot
+// number = row number), the row y = 8 (Y plane) and the plane z = 8 (Z plane) where a neighbour owns them.
+// One store per row pair and no branches: a lane's base is y or, in a last column that a neighbour owns,
+// the X plane, and the row's offset from it is added.  A third of the instructions of a loop that
+// decides node by node, which a wave alone on its SIMD waits for one by one.
+template <int ROWS, typename S, typename T>
+__device__ __forceinline__ void store_rows_full(const Box &b, const BrickId &br, const Tile &t,
+                                                const S *__restrict__ s, T *__restrict__ g, T *__restrict__ face,
+                                                bool add_mode, int z0, int lane) {
+  constexpr int STEPS = (ROWS + 1) / 2, E = ROWS % 2 ? STEPS : STEPS + 1;  // even: no half-empty last pair
+  const FastLane L = fast_lane(b, lane);
+  const bool ownx = L.ii < 2 * BE || br.bx == b.nbx - 1;
+  const bool lasty = br.by == b.nby - 1, ownz = z0 < 2 * BE || br.bz == b.nbz - 1;
+  T *gb = g + 3 * (t.node0 + (int64_t)b.NX * b.NY * z0);
+  T *fo = face + (int64_t)br.lin * FACEVALS;
+  s += TPS * z0;
+  T val[STEPS];
+#pragma unroll
+  for (int it = 0; it < STEPS; it++) val[it] = T(s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)]);
+  if (add_mode && ownz) {
+    T old[STEPS];
+#pragma unroll
+    for (int it = 0; it < STEPS; it++) old[it] = fast_at(gb, fast_eoff<E>(b, L, it));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int it = 0; it < STEPS; it++) {
+      int y, z;
+      fast_row(L, it, y, z);
+      if (ownx && (y < 2 * BE || lasty)) val[it] += old[it];
+    }
+  }
+  if (L.p > 1) return;
+  const int odd = L.p;
+  T *by = fo + 3 * TN * (TN + z0) + L.col;
+  char *base = reinterpret_cast<char *>(ownx ? gb : fo + 3 * TN * z0 + L.c);
+  T *bz = ownx ? fo + 3 * TN * 2 * TN + L.col : fo + 3 * TN * z0 + L.c;
+  constexpr uint32_t SZ = sizeof(T);
+#pragma unroll
+  for (int it = 0; it < STEPS; it++) {
+    const int r0 = 2 * it;                                                // the even lanes' row of the group
+    const bool top0 = r0 % TN == 2 * BE, top1 = (r0 + 1) % TN == 2 * BE;  // rows y = 8
+    T *at;
+    if (ownz)
+      at = reinterpret_cast<T *>(base + (ownx ? SZ * fast_eoff<E>(b, L, it) : 3 * SZ * (uint32_t)(r0 + odd)));
+    else
+      at = bz + (ownx ? 3 * TN * (r0 + odd) : 3 * (r0 + odd));  // the plane z = 8: Z plane [y][x]
+    if ((top0 || top1) && !lasty) {
+      const bool toy = ownx && (top0 ? odd == 0 : odd == 1);
+      at = toy ? by + 3 * TN * ((top0 ? r0 : r0 + 1) / TN) : at;
+    }
+    if (2 * it + 1 < ROWS || odd == 0) *at = val[it];
+  }
+}
+
+// the Chebyshev store of a full tile, with the addressing of load_tile2_fast
+template <typename S, typename T>
+__device__ __forceinline__ void store_tile_cheb_fast(const Box &b, const BrickId &br, const Tile &t,
+                                                     const S *__restrict__ s, T *__restrict__ g,
+                                                     T *__restrict__ face, int lane, const ChebOut<T> *co) {
+  constexpr int STEPS = TPAIRS;
   const FastLane L = fast_lane(b, lane);
   const bool ownx = L.ii < 2 * BE || br.bx == b.nbx - 1;
   const bool lasty = br.by == b.nby - 1, lastz = br.bz == b.nbz - 1;
-  const int64_t node0 = t.node0 + (int64_t)b.NX * b.NY * z0;
-  s += TPS * z0;
+  const int64_t node0 = t.node0;
   T *gb = g + 3 * node0;
   T *fo = face + (int64_t)br.lin * FACEVALS + L.c;
-  if constexpr (CH) {
-    // the update's operands of a chunk of steps are all loaded before the first is used (one
-    // exposed memory latency per chunk, not per step); every tile address is inside the box
-    constexpr int CHUNK = sizeof(T) == 4 ? STEPS : 14;
-    const T *bb = co->b + 3 * node0, *bd = co->dinv + 3 * node0, *bx = co->x + 3 * node0;
-    const T *bp = co->pkm1 ? co->pkm1 + 3 * node0 : nullptr;
-    const uint8_t *bm = co->mask ? co->mask + 3 * node0 : nullptr;
-    T *bo = co->out + 3 * node0;
+  // the update's operands of a chunk of steps are all loaded before the first is used (one
+  // exposed memory latency per chunk, not per step); every tile address is inside the box
+  constexpr int CHUNK = sizeof(T) == 4 ? STEPS : 14;
+  const T *bb = co->b + 3 * node0, *bd = co->dinv + 3 * node0, *bx = co->x + 3 * node0;
+  const T *bp = co->pkm1 ? co->pkm1 + 3 * node0 : nullptr;
+  const uint8_t *bm = co->mask ? co->mask + 3 * node0 : nullptr;
+  T *bo = co->out + 3 * node0;
 #pragma unroll
-    for (int c0 = 0; c0 < STEPS; c0 += CHUNK) {
-      T vb[CHUNK], vd[CHUNK], vx[CHUNK], vp[CHUNK];
-      int vm[CHUNK];
+  for (int c0 = 0; c0 < STEPS; c0 += CHUNK) {
+    T vb[CHUNK], vd[CHUNK], vx[CHUNK], vp[CHUNK];
+    int vm[CHUNK];
 #pragma unroll
-      for (int k = 0; k < CHUNK; k++) {
-        const int it = c0 + k;
-        if (it >= STEPS) break;
-        const uint32_t e = fast_eoff<STEPS>(b, L, it);
-        vb[k] = fast_at(bb, e);
-        vd[k] = fast_at(bd, e);
-        vx[k] = fast_at(bx, e);
-        vp[k] = bp ? fast_at(bp, e) : T(0);
-        vm[k] = bm ? (int)fast_at(bm, e) : 0;
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int k = 0; k < CHUNK; k++) {
-        const int it = c0 + k;
-        if (it >= STEPS) break;
-        if (!fast_stores<STEPS>(L, it)) continue;
-        int y, z;
-        fast_row(L, it, y, z);
-    z += z0;
-        const bool owny = y < 2 * BE || lasty, ownz = z < 2 * BE || lastz;
-        const S val = s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)];
-        const uint32_t e = fast_eoff<STEPS>(b, L, it);
-        if (ownx && owny && ownz) {
-          const bool lower = (L.ii == 0 && br.bx > 0) || (y == 0 && br.by > 0) || (z == 0 && br.bz > 0);
-          if (vm[k] || !lower) {
-            fast_at(bo, e) = cheb_value(*co, vd[k], vb[k], vm[k] ? vx[k] : T(val), vx[k], vp[k], bp != nullptr);
-          } else {
-            fast_at(gb, e) = T(val);
-          }
-        } else {
-          const int slot = !ownx ? z * TN + y : (!owny ? TN * TN + z * TN + L.ii : 2 * TN * TN + y * TN + L.ii);
-          fo[3 * slot] = T(val);
-        }
-      }
+    for (int k = 0; k < CHUNK; k++) {
+      const int it = c0 + k;
+      if (it >= STEPS) break;
+      const uint32_t e = fast_eoff(b, L, it);
+      vb[k] = fast_at(bb, e);
+      vd[k] = fast_at(bd, e);
+      vx[k] = fast_at(bx, e);
+      vp[k] = bp ? fast_at(bp, e) : T(0);
+      vm[k] = bm ? (int)fast_at(bm, e) : 0;
     }
-    return;
-  }
-  T v[STEPS];
-  if (add_mode) {
-#pragma unroll
-    for (int it = 0; it < STEPS; it++) v[it] = fast_at(gb, fast_eoff<STEPS>(b, L, it));
     __builtin_amdgcn_sched_barrier(0);
-  }
 #pragma unroll
-  for (int it = 0; it < STEPS; it++) {
-    if (!fast_stores<STEPS>(L, it)) continue;
-    int y, z;
-    fast_row(L, it, y, z);
-    z += z0;
-    const bool owny = y < 2 * BE || lasty, ownz = z < 2 * BE || lastz;
-    const S val = s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)];
-    if (ownx && owny && ownz) {
-      fast_at(gb, fast_eoff<STEPS>(b, L, it)) = add_mode ? T(v[it] + val) : T(val);
-    } else {
-      const int slot = !ownx ? z * TN + y : (!owny ? TN * TN + z * TN + L.ii : 2 * TN * TN + y * TN + L.ii);
-      fo[3 * slot] = T(val);
+    for (int k = 0; k < CHUNK; k++) {
+      const int it = c0 + k;
+      if (it >= STEPS) break;
+      if (!fast_stores(L, it)) continue;
+      int y, z;
+      fast_row(L, it, y, z);
+      const bool owny = y < 2 * BE || lasty, ownz = z < 2 * BE || lastz;
+      const S val = s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)];
+      const uint32_t e = fast_eoff(b, L, it);
+      if (ownx && owny && ownz) {
+        const bool lower = (L.ii == 0 && br.bx > 0) || (y == 0 && br.by > 0) || (z == 0 && br.bz > 0);
+        if (vm[k] || !lower) {
+          fast_at(bo, e) = cheb_value(*co, vd[k], vb[k], vm[k] ? vx[k] : T(val), vx[k], vp[k], bp != nullptr);
+        } else {
+          fast_at(gb, e) = T(val);
+        }
+      } else {
+        const int slot = !ownx ? z * TN + y : (!owny ? TN * TN + z * TN + L.ii : 2 * TN * TN + y * TN + L.ii);
+        fo[3 * slot] = T(val);
+      }
     }
   }
 }
 
 // CH: the Chebyshev update of co is applied to every owned node that is final here (see
-// store_tile_own_fast); the others are stored into g for the face pass.
+// store_tile_cheb_fast); the others are stored into g for the face pass.
 // STEPS row pairs from plane z0: the whole tile, or one wave's third of it.
 template <bool CH = false, int STEPS = TPAIRS, typename S, typename T>
 __device__ __forceinline__ void store_tile_own(const Box &b, const BrickId &br, const Tile &t, const S *__restrict__ s,
@@ -553,7 +581,17 @@ __device__ __forceinline__ void store_tile_own(const Box &b, const BrickId &br, 
                                                const ChebOut<T> *co = nullptr, int z0 = 0) {
   asm volatile("" : "+v"(lane));  // see store_tile
   if (tile_fast(b, t)) {
-    store_tile_own_fast<CH, STEPS>(b, br, t, s, g, face, add_mode, lane, co, z0);
+    if constexpr (CH) {
+      store_tile_cheb_fast(b, br, t, s, g, face, lane, co);
+    } else if (STEPS == TPAIRS) {
+      store_rows_full<2 * BE * TN>(b, br, t, s, g, face, add_mode, 0, lane);
+      store_rows_full<TN>(b, br, t, s, g, face, add_mode, 2 * BE, lane);
+    } else if (z0 < 2 * WPLANES) {
+      store_rows_full<WPLANES * TN>(b, br, t, s, g, face, add_mode, z0, lane);
+    } else {
+      store_rows_full<2 * TN>(b, br, t, s, g, face, add_mode, z0, lane);
+      store_rows_full<TN>(b, br, t, s, g, face, add_mode, 2 * BE, lane);
+    }
     return;
   }
   const TileLane L = tile_lane(b, t, br, lane);

@@ -81,8 +81,10 @@ hipError_t launch_eta_to_bm(const Box &b, const double *eta, double *eta_bm, int
 hipError_t launch_check_mesh(const Box &b, const double *coords, double *xtile, int *err, hipStream_t s);
 hipError_t launch_a21(const Box &b, const double *coords, const double *u, const uint8_t *mask, double *yp, bool add,
                       hipStream_t s);
-hipError_t launch_a12(const Box &b, const double *coords, const double *p, double *y, bool add, hipStream_t s);
-hipError_t launch_diag(const Box &b, const double *coords, const double *eta_bm, double *d, bool add, hipStream_t s);
+hipError_t launch_a12(const Box &b, const double *coords, const double *p, double *y, bool add, double *facebuf,
+                      hipStream_t s);
+hipError_t launch_diag(const Box &b, const double *coords, const double *eta_bm, double *d, bool add, double *facebuf,
+                       hipStream_t s);
 // y (+)= the body-force load of fu (3 per quadrature point, element-major)
 // one launch with owner-writes output into facebuf (nbricks * FACEVALS doubles) plus the face pass
 hipError_t launch_body_force(const Box &b, const double *coords, const double *fu, double *y, bool add,

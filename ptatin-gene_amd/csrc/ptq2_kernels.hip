@@ -488,7 +488,8 @@ __global__ __launch_bounds__(3 * BEL) void k_a11_fp64_split(Box b, const double 
     if (w == k && active) emit_element(Xs, base, Y);
     __syncthreads();
   }
-  if (w == 0) store_tile_own(b, br, t, Xs, y, facebuf, add_mode != 0, lane);
+  store_tile_own<false, WSTEPS>(b, br, t, Xs, y, facebuf, add_mode != 0, lane, (const ChebOut<double> *)nullptr,
+                                WPLANES * w);
 }
 
 __global__ __launch_bounds__(3 * BEL) void k_a11_fp32_split(Box b, const float *__restrict__ u,
@@ -523,7 +524,8 @@ __global__ __launch_bounds__(3 * BEL) void k_a11_fp32_split(Box b, const float *
     if (w == k && active) emit_element(Ts, base, Y);
     __syncthreads();
   }
-  if (w == 0) store_tile_own(b, br, t, Ts, y, facebuf, add_mode != 0, lane);
+  store_tile_own<false, WSTEPS>(b, br, t, Ts, y, facebuf, add_mode != 0, lane, (const ChebOut<float> *)nullptr,
+                                WPLANES * w);
 }
 
 // ------------------------------------------------------ A11 FP64, stored geometry
@@ -923,38 +925,117 @@ __global__ __launch_bounds__(BEL) void k_check_mesh(Box b, const double *__restr
   if (bad) atomicOr(err, ERRBIT_MESH);
 }
 
-// ------------------------------------------------------------------ A21
-// y_p[4e+i] += -sum_q w det N^p_i (div u)_q ; div u = trace(M)/det.
+// --------------------------------------------------------- A21 and A12
+// One wave per brick, the contractions in the modal form of ptq2_comp.h, slab by slab in the order 1, 0, 2
+// of the quadrature points' z.  A wave is alone on its SIMD (all 512 registers), so what bounds both is
+// the number of instructions and every latency between them: 3.1k FP64 operations of 5-6k instructions
+// per wave (5.3k of 8-11k with the nodal tables and a row's data read from the tile).  64^3 elements:
+// A21 114 -> 79 us; A12 in one launch with the face pass 119 us, against 218 us in 8 coloured ones
+// (512 waves each, half the chip's SIMDs) with nodal tables.
 
-template <int qa, int qb, int qc>
-__device__ __forceinline__ void a21_qp(const double xr0[3][3], const double xr1[3][3], const double xr2[3][3],
-                                       const double ur0[3][3], const double ur1[3][3], const double ur2[3][3],
-                                       const PBasis &pb, double Yp[4]) {
-  double J[3][3], A[3][3], g[3][3], x[3];
-  qp_grad<qa>(xr0, xr1, xr2, J);
-  adjugate(J, A);
-  qp_grad<qa>(ur0, ur1, ur2, g);
-  qp_value<qa>(xr0, x);
-  // trace(M) = sum_k sum_m g[m][k] A[k][m] = det * div u
-  double tr = 0.0;
+// The lane's element values of tile component c at node layer K along z, modal in x and y.
+template <int K>
+__device__ __forceinline__ void load_layer(const double *s, int base, int c, double shift, double v[9]) {
 #pragma unroll
-  for (int k = 0; k < 3; k++) tr += g[0][k] * A[k][0] + g[1][k] * A[k][1] + g[2][k] * A[k][2];
-  constexpr double w = gw1(qa) * gw1(qb) * gw1(qc);
-  double f = -w * tr;
-  Yp[0] += f;
+  for (int j = 0; j < 3; j++)
 #pragma unroll
-  for (int d = 0; d < 3; d++) Yp[1 + d] += f * ((x[d] - pb.avg[d]) * pb.inv[d]);
+    for (int i = 0; i < 3; i++) v[i + 3 * j] = s[base + c * TCS + xo(i) + j * TRS + K * TPS];
+  modal_layer(v);
+  v[0] -= shift;
+}
+// One field's values and derivatives along z (row_grad) for the slab of row R, when R opens a slab;
+// field values are taken relative to shift.  The third z coefficient a, which slab 1 does not need,
+// is formed again in the other two from a layer read from the tile: kept, it would cost 54 registers of the
+// three (or six) fields.  Slab 0 has v = m + V2 a - V1 b, d = b - D2 a, and u2 = m + (b + a) / 2 gives
+// a (1/2 - V2 + (1/2 + V1) D2) = u2 - v - (1/2 + V1) d.
+template <int R>
+__device__ __forceinline__ void to_row_slab(const double *s, int base, int c, double shift, double v[18]) {
+  if (R == 0) {
+    double u0[9], u2[9];
+    load_layer<0>(s, base, c, 0.0, u0);
+    load_layer<1>(s, base, c, shift, v);
+    load_layer<2>(s, base, c, 0.0, u2);
+#pragma unroll
+    for (int n = 0; n < 9; n++) v[9 + n] = u2[n] - u0[n];
+  } else if (R == 3) {
+    double u0[9];
+    load_layer<0>(s, base, c, shift, u0);
+#pragma unroll
+    for (int n = 0; n < 9; n++) {
+      const double a = fma(2.0, u0[n] - v[n], v[n + 9]);
+      v[n] = fma(-MOD_V1, v[n + 9], fma(MOD_V2, a, v[n]));
+      v[n + 9] = fma(-MOD_D2, a, v[n + 9]);
+    }
+  } else if (R == 6) {
+    constexpr double e = 0.5 + MOD_V1, f = 1.0 / (0.5 - MOD_V2 + e * MOD_D2);
+    double u2[9];
+    load_layer<2>(s, base, c, shift, u2);
+#pragma unroll
+    for (int n = 0; n < 9; n++) {
+      const double a = f * fma(-e, v[n + 9], u2[n] - v[n]);
+      const double b = fma(MOD_D2, a, v[n + 9]);
+      v[n] = fma(2.0 * MOD_V1, b, v[n]);
+      v[n + 9] = fma(MOD_D2, a, b);
+    }
+  }
+  if (R % 3 == 0) {
+    pin<18>(v);
+    row_fence();
+  }
 }
 
-template <int qb, int qc>
-__device__ __forceinline__ void a21_row(const double *Xs, const double *Us, int base, const PBasis &pb, double Yp[4]) {
-  double xr0[3][3], xr1[3][3], xr2[3][3], ur0[3][3], ur1[3][3], ur2[3][3];
-  row_data<qb, qc>(Xs, base, xr0, xr1, xr2);
-  row_data<qb, qc>(Us, base, ur0, ur1, ur2);
-  a21_qp<0, qb, qc>(xr0, xr1, xr2, ur0, ur1, ur2, pb, Yp);
-  a21_qp<1, qb, qc>(xr0, xr1, xr2, ur0, ur1, ur2, pb, Yp);
-  a21_qp<2, qb, qc>(xr0, xr1, xr2, ur0, ur1, ur2, pb, Yp);
+// values at a row's three points from its modal x coefficients
+__device__ __forceinline__ void row_values(const double r[3], double v[3]) {
+  const double s = fma(MOD_V2, r[2], r[0]);
+  v[0] = fma(-MOD_V1, r[1], s);
+  v[1] = r[0];
+  v[2] = fma(MOD_V1, r[1], s);
+}
+template <int R, int Q>
+constexpr double w8() {
+  return gw1(Q) * gw1(row_qb(R)) * gw1(row_qc(R)) * 0.125;
+}
+
+// y_p[4e+i] += -sum_q w det N^p_i (div u)_q ; div u = trace(M)/det, trace(M) = sum_kc g[k][c] A[c][k].
+// x: coordinates relative to the basis' centre; its scale is applied at the end.
+template <int R>
+__device__ __forceinline__ void a21_rows(const double *Xs, const double *Us, int base, const PBasis &pb,
+                                         double x[3][18], double u[3][18], double Yp[4]) {
+  double Jc[3][3][3], r0[3][3];  // [component][d][qa]
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    to_row_slab<R>(Xs, base, c, pb.avg[c], x[c]);
+    row_grad<row_qb(R)>(x[c], Jc[c], r0[c]);
+  }
+  double tr[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    double g[3][3];
+    to_row_slab<R>(Us, base, c, 0.0, u[c]);
+    row_grad<row_qb(R)>(u[c], g);
+    // column c of the adjugate: the cross product of the other two components' gradients
+    const int a = (c + 1) % 3, b = (c + 2) % 3;
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const int d1 = (d + 1) % 3, d2 = (d + 2) % 3;
+        tr[q] = fma(g[d][q], fma(Jc[a][d1][q], Jc[b][d2][q], -Jc[a][d2][q] * Jc[b][d1][q]), tr[q]);
+      }
+  }
+  tr[0] *= w8<R, 0>();
+  tr[1] *= w8<R, 1>();
+  tr[2] *= w8<R, 2>();
+  Yp[0] += tr[0] + tr[1] + tr[2];
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    double v[3];
+    row_values(r0[c], v);
+    Yp[1 + c] = fma(tr[0], v[0], fma(tr[1], v[1], fma(tr[2], v[2], Yp[1 + c])));
+  }
+  pin<4>(Yp);
   row_fence();
+  if constexpr (R < 8) a21_rows<R + 1>(Xs, Us, base, pb, x, u, Yp);
 }
 
 __global__ __launch_bounds__(BEL) void k_a21(Box b, const double *__restrict__ coords, const double *__restrict__ u,
@@ -969,99 +1050,90 @@ __global__ __launch_bounds__(BEL) void k_a21(Box b, const double *__restrict__ c
   if (!lane_active(t, lane)) return;
   const int base = lane_base(lane);
   const PBasis pb = pbasis_setup(Xs, base);
-  double Yp[4] = {0.0, 0.0, 0.0, 0.0};
-  a21_row<0, 0>(Xs, Us, base, pb, Yp); a21_row<1, 0>(Xs, Us, base, pb, Yp); a21_row<2, 0>(Xs, Us, base, pb, Yp);
-  a21_row<0, 1>(Xs, Us, base, pb, Yp); a21_row<1, 1>(Xs, Us, base, pb, Yp); a21_row<2, 1>(Xs, Us, base, pb, Yp);
-  a21_row<0, 2>(Xs, Us, base, pb, Yp); a21_row<1, 2>(Xs, Us, base, pb, Yp); a21_row<2, 2>(Xs, Us, base, pb, Yp);
-  const int64_t e = lane_element(b, t, lane);
-  double *o = yp + 4 * e;
+  double xm[3][18], um[3][18], Yp[4] = {0.0, 0.0, 0.0, 0.0};
+  a21_rows<0>(Xs, Us, base, pb, xm, um, Yp);
+  double *o = yp + 4 * lane_element(b, t, lane);
+  double r[4] = {-Yp[0], 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int i = 0; i < 4; i++) o[i] = add_mode ? o[i] + Yp[i] : Yp[i];
+  for (int d = 0; d < 3; d++) r[1 + d] = -Yp[1 + d] * pb.inv[d];
+#pragma unroll
+  for (int i = 0; i < 4; i++) o[i] = add_mode ? o[i] + r[i] : r[i];
 }
 
-// ------------------------------------------------------------------ A12
-// y_u[n,l] += -sum_q w p_q (A^T)... : dv[k][l] = -w p A[l][k] (QuadratureAction_A12_AVX).
-
-template <int qa, int qb, int qc>
-__device__ __forceinline__ void a12_qp(const double xr0[3][3], const double xr1[3][3], const double xr2[3][3],
-                                       const PBasis &pb, const double pe[4], double RB[3][3][3], double RD[3][3][3]) {
-  double J[3][3], A[3][3], x[3], dv[3][3];
-  qp_grad<qa>(xr0, xr1, xr2, J);
-  adjugate(J, A);
-  qp_value<qa>(xr0, x);
-  double pq = pe[0];
+// y_u[n,l] += -sum_q w p_q A[l][.] . grad N_n (QuadratureAction_A12_AVX).
+template <int R>
+__device__ __forceinline__ void a12_rows(const double *Xs, int base, const PBasis &pb, const double ps[4],
+                                         double x[3][18], double RB[3][9], double RD[3][9], double Y[3][27]) {
+  constexpr int QB = row_qb(R);
+  double Jc[3][3][3], rp[3];  // [component][d][qa]
 #pragma unroll
-  for (int d = 0; d < 3; d++) pq += pe[1 + d] * ((x[d] - pb.avg[d]) * pb.inv[d]);
-  constexpr double w = gw1(qa) * gw1(qb) * gw1(qc);
-  double f = -w * pq;
+  for (int c = 0; c < 3; c++) {
+    double r0[3];
+    to_row_slab<R>(Xs, base, c, pb.avg[c], x[c]);
+    row_grad<QB>(x[c], Jc[c], r0);
+    // the pressure is linear in the coordinates relative to the basis' centre
 #pragma unroll
-  for (int k = 0; k < 3; k++)
+    for (int i = 0; i < 3; i++) rp[i] = c == 0 ? ps[1] * r0[i] : fma(ps[1 + c], r0[i], rp[i]);
+  }
+  rp[0] += ps[0];
+  double f[3];
+  row_values(rp, f);
+  f[0] *= -w8<R, 0>();
+  f[1] *= -w8<R, 1>();
+  f[2] *= -w8<R, 2>();
 #pragma unroll
-    for (int l = 0; l < 3; l++) dv[k][l] = f * A[l][k];
-  acc_direct<qa, qb>(dv, RB, RD);
+  for (int l = 0; l < 3; l++) {
+    const int a = (l + 1) % 3, b = (l + 2) % 3;
+    double dv[3][3];
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const int d1 = (d + 1) % 3, d2 = (d + 2) % 3;
+        dv[d][q] = f[q] * fma(Jc[a][d1][q], Jc[b][d2][q], -Jc[a][d2][q] * Jc[b][d1][q]);
+      }
+    row_dual<QB>(dv, RB[l], RD[l]);
+    if (R % 3 == 2) slab_dual<row_qc(R)>(RB[l], RD[l], Y[l]);
+    row_fence();
+  }
+  if constexpr (R < 8) a12_rows<R + 1>(Xs, base, pb, ps, x, RB, RD, Y);
 }
 
-template <int qb, int qc>
-__device__ __forceinline__ void a12_row(const double *Xs, int base, const PBasis &pb, const double pe[4],
-                                        double RB[3][3][3], double RD[3][3][3]) {
-  double xr0[3][3], xr1[3][3], xr2[3][3];
-  row_data<qb, qc>(Xs, base, xr0, xr1, xr2);
-  a12_qp<0, qb, qc>(xr0, xr1, xr2, pb, pe, RB, RD);
-  a12_qp<1, qb, qc>(xr0, xr1, xr2, pb, pe, RB, RD);
-  a12_qp<2, qb, qc>(xr0, xr1, xr2, pb, pe, RB, RD);
-  row_fence();
-}
-
-template <int qc>
-__device__ __forceinline__ void a12_slab(const double *Xs, int base, const PBasis &pb, const double pe[4],
-                                         double Y[3][3][3][3]) {
-  double RB[3][3][3], RD[3][3][3];
-#pragma unroll
-  for (int c = 0; c < 3; c++)
-#pragma unroll
-    for (int j = 0; j < 3; j++)
-#pragma unroll
-      for (int i = 0; i < 3; i++) RB[c][j][i] = RD[c][j][i] = 0.0;
-  a12_row<0, qc>(Xs, base, pb, pe, RB, RD);
-  a12_row<1, qc>(Xs, base, pb, pe, RB, RD);
-  a12_row<2, qc>(Xs, base, pb, pe, RB, RD);
-  acc_elem<qc>(RB, RD, Y);
-  row_fence();
-}
-
-__global__ __launch_bounds__(BEL) void k_a12(Box b, int color, const double *__restrict__ coords,
-                                             const double *__restrict__ p, double *__restrict__ y, int add_mode) {
+__global__ __launch_bounds__(BEL) void k_a12(Box b, const double *__restrict__ coords, const double *__restrict__ p,
+                                             double *__restrict__ y, int add_mode, double *__restrict__ facebuf) {
   __shared__ double Xs[3 * TCS];
   const int lane = threadIdx.x;
-  const BrickId br = brick_of(b, color, blockIdx.x);
+  const BrickId br = brick_xcd(b, blockIdx.x);
   const Tile t = tile_of(b, br);
+  const bool active = lane_active(t, lane);
+  const double *pe = p + 4 * (active ? lane_element(b, t, lane) : 0);
+  double ps[4] = {pe[0], pe[1], pe[2], pe[3]};
   load_tile(b, t, br, coords, (const uint8_t *)nullptr, Xs, lane);
   __syncthreads();
   const int base = lane_base(lane);
-  const bool active = lane_active(t, lane);
-  double Y[3][3][3][3];
+  // lanes without an element run too (on whatever the tile holds) and emit nothing
+  const PBasis pb = pbasis_setup(Xs, base);
 #pragma unroll
-  for (int c = 0; c < 3; c++)
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-#pragma unroll
-      for (int j = 0; j < 3; j++)
-#pragma unroll
-        for (int i = 0; i < 3; i++) Y[c][k][j][i] = 0.0;
-  if (active) {
-    const PBasis pb = pbasis_setup(Xs, base);
-    const int64_t e = lane_element(b, t, lane);
-    double pe[4] = {p[4 * e], p[4 * e + 1], p[4 * e + 2], p[4 * e + 3]};
-    a12_slab<0>(Xs, base, pb, pe, Y);
-    a12_slab<1>(Xs, base, pb, pe, Y);
-    a12_slab<2>(Xs, base, pb, pe, Y);
-  }
-  __syncthreads();
+  for (int d = 0; d < 3; d++) ps[1 + d] *= pb.inv[d];
+  double x[3][18], RB[3][9], RD[3][9], Y[3][27];
+  a12_rows<0>(Xs, base, pb, ps, x, RB, RD, Y);
+  __syncthreads();  // the coordinates are read: their LDS becomes the output tile
   zero_tile(Xs, lane);
   __syncthreads();
-  if (active) emit_element(Xs, base, Y);
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    dual_to_nodal27(Y[c]);
+    if (active) {
+#pragma unroll
+      for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+#pragma unroll
+          for (int i = 0; i < 3; i++) lds_add(&Xs[base + toff(c, i, j, k)], Y[c][i + 3 * j + 9 * k]);
+    }
+  }
   __syncthreads();
-  store_tile(b, br, t, Xs, y, add_mode != 0, lane);
+  store_tile_own(b, br, t, Xs, y, facebuf, add_mode != 0, lane);
 }
 
 // ---------------------------------------------------------------- body force
@@ -1195,7 +1267,9 @@ __global__ __launch_bounds__(BEL) void k_body_force(Box b, const double *__restr
 // ---------------------------------------------------------------- diagonal
 // diag(n,x) += sum_q w det eta (2 Nx^2 + Ny^2 + Nz^2) (cyclic for y, z), the form of
 // MatMultMF_Stokes_MixedFEM3d_diagB11 (src/stokes_q2p1_mf_operators_diag_def.c:120-205).
-// With h = A grad_xi N = det grad_x N: w det eta Nx^2 = (w eta / det) h_x^2.
+// With h = A grad_xi N = det grad_x N: w det eta Nx^2 = (w eta / det) h_x^2.  17k VALU instructions of one
+// wave per brick bound it; 40x36x44 elements take 56 + 6 us (face pass) in one launch, 355 us in 8 coloured
+// launches of 125 waves, each one brick's latency.
 
 template <int qa, int qb, int qc>
 __device__ __forceinline__ void diag_qp(const double xr0[3][3], const double xr1[3][3], const double xr2[3][3],
@@ -1238,11 +1312,12 @@ __device__ __forceinline__ void diag_row(const double *Xs, int base, const doubl
   row_fence();
 }
 
-__global__ __launch_bounds__(BEL) void k_diag(Box b, int color, const double *__restrict__ coords,
-                                              const double *__restrict__ eta_bm, double *__restrict__ d, int add_mode) {
+__global__ __launch_bounds__(BEL) void k_diag(Box b, const double *__restrict__ coords,
+                                              const double *__restrict__ eta_bm, double *__restrict__ d, int add_mode,
+                                              double *__restrict__ facebuf) {
   __shared__ double Xs[3 * TCS];
   const int lane = threadIdx.x;
-  const BrickId br = brick_of(b, color, blockIdx.x);
+  const BrickId br = brick_xcd(b, blockIdx.x);
   const Tile t = tile_of(b, br);
   load_tile(b, t, br, coords, (const uint8_t *)nullptr, Xs, lane);
   __syncthreads();
@@ -1272,7 +1347,7 @@ __global__ __launch_bounds__(BEL) void k_diag(Box b, int color, const double *__
   __syncthreads();
   if (active) emit_element(Xs, base, Y);
   __syncthreads();
-  store_tile(b, br, t, Xs, d, add_mode != 0, lane);
+  store_tile_own(b, br, t, Xs, d, facebuf, add_mode != 0, lane);
 }
 
 // ------------------------------------------------------------- BC helpers
@@ -1556,13 +1631,10 @@ hipError_t launch_a21(const Box &b, const double *coords, const double *u, const
   return hipGetLastError();
 }
 
-hipError_t launch_a12(const Box &b, const double *coords, const double *p, double *y, bool add, hipStream_t s) {
-  for (int c = 0; c < 8; c++) {
-    int nb = nbricks_color(b, c);
-    if (nb == 0) continue;
-    hipLaunchKernelGGL(k_a12, dim3(nb), dim3(BEL), 0, s, b, c, coords, p, y, add ? 1 : 0);
-  }
-  return hipGetLastError();
+hipError_t launch_a12(const Box &b, const double *coords, const double *p, double *y, bool add, double *facebuf,
+                      hipStream_t s) {
+  hipLaunchKernelGGL(k_a12, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, p, y, add ? 1 : 0, facebuf);
+  return launch_gather(b, (const double *)facebuf, y, s);
 }
 
 hipError_t launch_body_force(const Box &b, const double *coords, const double *fu, double *y, bool add,
@@ -1572,13 +1644,10 @@ hipError_t launch_body_force(const Box &b, const double *coords, const double *f
   return e != hipSuccess ? e : launch_gather(b, (const double *)facebuf, y, s);
 }
 
-hipError_t launch_diag(const Box &b, const double *coords, const double *eta_bm, double *d, bool add, hipStream_t s) {
-  for (int c = 0; c < 8; c++) {
-    int nb = nbricks_color(b, c);
-    if (nb == 0) continue;
-    hipLaunchKernelGGL(k_diag, dim3(nb), dim3(BEL), 0, s, b, c, coords, eta_bm, d, add ? 1 : 0);
-  }
-  return hipGetLastError();
+hipError_t launch_diag(const Box &b, const double *coords, const double *eta_bm, double *d, bool add, double *facebuf,
+                       hipStream_t s) {
+  hipLaunchKernelGGL(k_diag, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, eta_bm, d, add ? 1 : 0, facebuf);
+  return launch_gather(b, (const double *)facebuf, d, s);
 }
 
 template <typename T>

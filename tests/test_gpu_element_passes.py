@@ -53,3 +53,25 @@ def test_a11_fp64(dims):
     assert rel(ym, O.matmult_a11(*dims, P.coords, P.eta, P.mask, u)) <= 1e-12
     d = P.mask > 0
     assert np.array_equal(ym[d], u[d])
+
+
+@pytest.mark.parametrize("dims", EDGES)
+def test_gradient_divergence_diagonal(dims):
+    """A12, A21 and the A11 diagonal, set and ADD; the mesh sits 50 edge lengths from the origin, where
+    the pressure basis works with differences of coordinates: a point's position, a sum of 27 rounded
+    terms on either side, is off by up to 27 x 50 x 2^-53 against an element's edge of 1 / max(dims)."""
+    tol = max(1e-12, 2 * 27 * 50 * max(dims) * 2.0 ** -53)
+    print("case: A12, A21, diagonal", dims, flush=True)
+    P = problem(dims)
+    P = M.Problem(*dims, P.coords + 50.0, P.mask, P.eta)
+    A = ptq2.MatA11MF("hip")
+    A.setup(P)
+    u, p = M.uniform(3, P.nvel, -1.0, 1.0), M.uniform(4, 4 * int(np.prod(dims)), -1.0, 1.0)
+    ud, pd = torch.from_numpy(u).to(DEV), torch.from_numpy(p).to(DEV)
+    c = A.ctx
+    for ref, y, again in (
+            (O.a12(*dims, P.coords, p), c.a12(pd), lambda y0: c.a12(pd, y0, _lib.ADD)),
+            (O.a21(*dims, P.coords, u), c.a21(ud), lambda y0: c.a21(ud, y0, _lib.ADD)),
+            (O.diag_a11(*dims, P.coords, P.eta), c.a11_diag(device=DEV), lambda y0: c.a11_diag(y0, _lib.ADD))):
+        assert rel(y.cpu().numpy(), ref) <= tol
+        assert rel(again(torch.full_like(y, 0.5)).cpu().numpy(), ref + 0.5) <= tol
