@@ -160,10 +160,11 @@ int ptq2_stokes_residual(ptq2_ctx *ctx, const double *u, const double *p, const 
    (0 <= wil < n_elements: the xi/wil fields of MPntStd) and values eta_p[p], rho_p[p] (the
    eta/rho of MPntPStokes; rho_p may be NULL).  Writes eta_qp and rho_qp (27 per element, q =
    a+3b+9c; rho_qp is NULL exactly when rho_p is), as the reference writes .eta/.rho of
-   QPntVolCoefStokes.  Every node sums the points of its adjacent elements in a fixed order
-   (ascending element, then point index), so the result is bitwise reproducible; it equals the
+   QPntVolCoefStokes.  Every element sums its points in index order and every node its adjacent
+   elements in ascending order, so the result is bitwise reproducible; it equals the
    reference's point-order sums to rounding.  flags: PTQ2_DEVICE (every array a device pointer).
-   Synchronous (device scratch is allocated and freed inside).  Needs a single-rank box
+   Synchronous.  A workspace of about 350 bytes per element (more with more than 8 points per element,
+   750 at most) stays with the context until its next mesh set-up or its end.  Needs a single-rank box
    (ptq2_setup_mesh, or ptq2_setup_mesh_box without a ghost layer); a box with a ghost layer is
    PTQ2_ERR_UNSUPPORTED.  An element index out of range is PTQ2_ERR_INVALID_ARG, a non-finite
    coordinate or value PTQ2_ERR_NONFINITE.  Pass eta_qp to ptq2_set_viscosity to use it. */

@@ -248,6 +248,7 @@ int ptq2_destroy(ptq2_ctx **pc) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   dev_free(c->coords); dev_free(c->mask); dev_free(c->dir_idx); dev_free(c->eta_bm);
   dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf);
+  dev_free(c->pwork);
   dev_free(c->err); dev_free(c->su); dev_free(c->sy); dev_free(c->sp); dev_free(c->syp); dev_free(c->ures);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   if (c->ev) (void)hipEventDestroy(c->ev);
@@ -325,9 +326,11 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   c->gen++;
   dev_free(c->coords); dev_free(c->mask); dev_free(c->dir_idx); dev_free(c->eta_bm);
   dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf);
+  dev_free(c->pwork);
   c->coords = nullptr; c->mask = nullptr; c->dir_idx = nullptr; c->eta_bm = nullptr;
   c->xtile = nullptr; c->bdir = nullptr;
   c->fac32 = nullptr; c->facb32 = nullptr; c->geo64 = nullptr; c->facebuf = nullptr;
+  c->pwork = nullptr; c->pwork_bytes = 0;
   c->mesh_ready = c->eta_ready = c->fac32_valid = c->facb32_valid = c->geo64_valid = c->has_state = false;
   c->ndir = 0;
 

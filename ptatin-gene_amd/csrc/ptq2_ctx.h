@@ -43,6 +43,9 @@ struct ptq2_ctx {
   // u with the Dirichlet values inserted, for the residual (allocated on first use)
   double *ures = nullptr;
   size_t ures_bytes = 0;
+  // workspace of the point projection (allocated on first use)
+  void *pwork = nullptr;
+  size_t pwork_bytes = 0;
   // stream ordering of the batched apply (created on first use)
   hipEvent_t ev = nullptr;
   // staging for host-pointer calls

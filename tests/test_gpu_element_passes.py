@@ -75,3 +75,41 @@ def test_gradient_divergence_diagonal(dims):
             (O.diag_a11(*dims, P.coords, P.eta), c.a11_diag(device=DEV), lambda y0: c.a11_diag(y0, _lib.ADD))):
         assert rel(y.cpu().numpy(), ref) <= tol
         assert rel(again(torch.full_like(y, 0.5)).cpu().numpy(), ref + 0.5) <= tol
+
+
+@pytest.mark.parametrize("dims,ppe,crowd,rho", [((1, 1, 1), 1, 0, True), ((5, 3, 9), 8, 0, True),
+                                                ((8, 4, 1), 56, 0, False), ((4, 4, 3), 57, 0, True),
+                                                ((6, 5, 2), 2, 400, True), ((3, 3, 3), 0, 7, False)])
+def test_point_buckets(dims, ppe, crowd, rho):
+    """Points that fit the elements' slots (up to 56 on average), that do not, and one element
+    crowded by `crowd` more: against the oracle at the projection's bars or, if larger, the rounding of
+    two weighted means of a node's n points (n 2^-53 each), and away from the crowded element bit for bit
+    what the same points give without the crowd."""
+    sums = 2 * (8 * ppe + crowd) * 2.0 ** -53
+    print("case: point buckets", dims, ppe, crowd, flush=True)
+    mx, my, mz = dims
+    ne = mx * my * mz
+    c = M.q2_uniform(mx, my, mz)
+    wil = np.repeat(np.arange(ne), ppe)
+    wil = np.concatenate([wil[np.argsort(M.uniform(9, wil.size))], np.full(crowd, ne - 1)]).astype(np.int32)
+    xi = M.uniform(10, 3 * wil.size, -1.0, 1.0).reshape(-1, 3)
+    eta_p, rho_p = 10.0 ** M.uniform(11, wil.size, -2.0, 3.0), M.uniform(12, wil.size, -1.0, 1.0)
+    ctx = ptq2.Context(0)
+    ctx.setup_mesh(mx, my, mz, c)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+    def run(n):
+        out = ctx.project_points(dev(xi[:n]), dev(wil[:n]), dev(eta_p[:n]), dev(rho_p[:n]) if rho else None)
+        return [o.cpu().numpy() for o in (out if rho else [out])]
+
+    got = run(wil.size)
+    ref = O.project_q1(mx, my, mz, xi, wil, eta_p, rho_p)
+    assert np.max(np.abs(got[0] - ref[0]) / np.maximum(np.abs(ref[0]), 1e-300)) <= max(1e-13, sums)
+    if rho:
+        assert np.max(np.abs(got[1] - ref[1])) <= max(1e-14, sums)
+    if crowd and ppe:
+        far = np.ones((mz, my, mx), dtype=bool)
+        far[-2:, -2:, -2:] = False
+        for a, b in zip(got, run(wil.size - crowd)):
+            assert np.array_equal(a.reshape(ne, 27)[far.reshape(-1)], b.reshape(ne, 27)[far.reshape(-1)])
+    ctx.destroy()
