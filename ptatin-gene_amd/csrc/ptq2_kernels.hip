@@ -155,11 +155,6 @@ __device__ __forceinline__ void emit_element(S *Ys, int base, const T Y[3][3][3]
         for (int i = 0; i < 3; i++) lds_add(&Ys[base + toff(c, i, j, k)], S(Y[c][k][j][i]));
 }
 
-__device__ __forceinline__ void load9(const double *__restrict__ ep, int qc, double *e9) {
-#pragma unroll
-  for (int q = 0; q < 9; q++) e9[q] = ep[(9 * qc + q) * BEL];
-}
-
 __device__ __forceinline__ void load3(const double *__restrict__ ep, int row, double *e3) {
 #pragma unroll
   for (int q = 0; q < 3; q++) e3[q] = ep[(3 * row + q) * BEL];
@@ -1267,49 +1262,65 @@ __global__ __launch_bounds__(BEL) void k_body_force(Box b, const double *__restr
 // ---------------------------------------------------------------- diagonal
 // diag(n,x) += sum_q w det eta (2 Nx^2 + Ny^2 + Nz^2) (cyclic for y, z), the form of
 // MatMultMF_Stokes_MixedFEM3d_diagB11 (src/stokes_q2p1_mf_operators_diag_def.c:120-205).
-// With h = A grad_xi N = det grad_x N: w det eta Nx^2 = (w eta / det) h_x^2.  17k VALU instructions of one
-// wave per brick bound it; 40x36x44 elements take 56 + 6 us (face pass) in one launch, 355 us in 8 coloured
-// launches of 125 waves, each one brick's latency.
+// With h = A grad_xi N = det grad_x N: w det eta Nx^2 = (w eta / det) h_x^2.
+// The VALU instructions of one wave per brick bound it: 12k with the sums of h^2 below (17.8k with the three
+// weighted sums per point and node).  40x36x44 elements: 36 us (55 us) and 6 us of face pass; 355 us in
+// 8 coloured launches of 125 waves, each one brick's latency.
 
+// At a point, with r = sqrt(w eta / det) and A = r adj(J), h_c(n) = D_i p + B_i q at node (i,j,k) with
+// p = A[c][0] B_j B_k and q = A[c][1] D_j B_k + A[c][2] B_j D_k, and X_c(n) sums h_c^2 over the points;
+// the diagonal is X_c + (X_0 + X_1 + X_2).
 template <int qa, int qb, int qc>
-__device__ __forceinline__ void diag_qp(const double xr0[3][3], const double xr1[3][3], const double xr2[3][3],
-                                        const double *eta9, double Y[3][3][3][3]) {
+__device__ __forceinline__ void diag_qp(const double Jc[3][3][3], double eta, double X[3][27]) {
   double J[3][3], A[3][3];
-  qp_grad<qa>(xr0, xr1, xr2, J);
-  double det = adjugate(J, A);
-  constexpr double w = gw1(qa) * gw1(qb) * gw1(qc);
-  double s = (w * eta9[qa + 3 * qb]) * rcp64(det);
 #pragma unroll
-  for (int k = 0; k < 3; k++)
+  for (int d = 0; d < 3; d++)
 #pragma unroll
-    for (int j = 0; j < 3; j++)
+    for (int c = 0; c < 3; c++) J[d][c] = Jc[c][d][qa];
+  const double det = adjugate(J, A);
+  // twice the derivatives (modal form): adj' = 4 adj, det' = 8 det
+  constexpr double w = gw1(qa) * gw1(qb) * gw1(qc) * 0.5;
+  const double r = sqrt((w * eta) * rcp64(det));
 #pragma unroll
-      for (int i = 0; i < 3; i++) {
-        const double n0 = gD(qa, i) * gB(qb, j) * gB(qc, k);
-        const double n1 = gB(qa, i) * gD(qb, j) * gB(qc, k);
-        const double n2 = gB(qa, i) * gB(qb, j) * gD(qc, k);
-        if (n0 != 0.0 || n1 != 0.0 || n2 != 0.0) {
-          double hx = A[0][0] * n0 + A[0][1] * n1 + A[0][2] * n2;
-          double hy = A[1][0] * n0 + A[1][1] * n1 + A[1][2] * n2;
-          double hz = A[2][0] * n0 + A[2][1] * n1 + A[2][2] * n2;
-          double ax = hx * hx, ay = hy * hy, az = hz * hz, sum = ax + ay + az;
-          Y[0][k][j][i] += s * (sum + ax);
-          Y[1][k][j][i] += s * (sum + ay);
-          Y[2][k][j][i] += s * (sum + az);
+  for (int c = 0; c < 3; c++) {
+    const double a0 = r * A[c][0], a1 = r * A[c][1], a2 = r * A[c][2];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+      for (int j = 0; j < 3; j++) {
+        const double c0 = gB(qb, j) * gB(qc, k), c1 = gD(qb, j) * gB(qc, k), c2 = gB(qb, j) * gD(qc, k);
+        const double p = c0 != 0.0 ? c0 * a0 : 0.0;
+        const double q = c1 != 0.0 ? (c2 != 0.0 ? fma(c2, a2, c1 * a1) : c1 * a1) : (c2 != 0.0 ? c2 * a2 : 0.0);
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+          const bool up = gD(qa, i) != 0.0 && c0 != 0.0, uq = gB(qa, i) != 0.0 && (c1 != 0.0 || c2 != 0.0);
+          if (!up && !uq) continue;
+          const double h = up ? (uq ? fma(gB(qa, i), q, gD(qa, i) * p) : gD(qa, i) * p) : gB(qa, i) * q;
+          double &x = X[c][i + 3 * j + 9 * k];
+          x = fma(h, h, x);
         }
       }
+  }
+  row_fence();
 }
 
-template <int qb, int qc>
-__device__ __forceinline__ void diag_row(const double *Xs, int base, const double *eta9, double Y[3][3][3][3]) {
-  double xr0[3][3], xr1[3][3], xr2[3][3];
-  row_data<qb, qc>(Xs, base, xr0, xr1, xr2);
-  diag_qp<0, qb, qc>(xr0, xr1, xr2, eta9, Y);
+template <int R>
+__device__ __forceinline__ void diag_rows(const double *Xs, int base, const double *__restrict__ ep, double x[3][18],
+                                          double X[3][27]) {
+  constexpr int QB = row_qb(R), QC = row_qc(R);
+  double Jc[3][3][3], e[3];
+#pragma unroll
+  for (int q = 0; q < 3; q++) e[q] = ep[(q + 3 * QB + 9 * QC) * BEL];
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    to_row_slab<R>(Xs, base, c, 0.0, x[c]);
+    row_grad<QB>(x[c], Jc[c]);
+  }
   row_fence();
-  diag_qp<1, qb, qc>(xr0, xr1, xr2, eta9, Y);
-  row_fence();
-  diag_qp<2, qb, qc>(xr0, xr1, xr2, eta9, Y);
-  row_fence();
+  diag_qp<0, QB, QC>(Jc, e[0], X);
+  diag_qp<1, QB, QC>(Jc, e[1], X);
+  diag_qp<2, QB, QC>(Jc, e[2], X);
+  if constexpr (R < 8) diag_rows<R + 1>(Xs, base, ep, x, X);
 }
 
 __global__ __launch_bounds__(BEL) void k_diag(Box b, const double *__restrict__ coords,
@@ -1322,30 +1333,27 @@ __global__ __launch_bounds__(BEL) void k_diag(Box b, const double *__restrict__ 
   load_tile(b, t, br, coords, (const uint8_t *)nullptr, Xs, lane);
   __syncthreads();
   const int base = lane_base(lane);
-  const bool active = lane_active(t, lane);
-  double Y[3][3][3][3];
-#pragma unroll
-  for (int c = 0; c < 3; c++)
+  double X[3][27] = {};
+  if (lane_active(t, lane)) {
+    double x[3][18];
+    diag_rows<0>(Xs, base, eta_bm + (int64_t)br.lin * 27 * BEL + lane, x, X);
+  }
+  __syncthreads();
+  zero_tile(Xs, lane);
+  __syncthreads();
+  if (lane_active(t, lane)) {
 #pragma unroll
     for (int k = 0; k < 3; k++)
 #pragma unroll
       for (int j = 0; j < 3; j++)
 #pragma unroll
-        for (int i = 0; i < 3; i++) Y[c][k][j][i] = 0.0;
-  if (active) {
-    const double *ep = eta_bm + (int64_t)br.lin * 27 * BEL + lane;
-    double e9[9];
-    load9(ep, 0, e9);
-    diag_row<0, 0>(Xs, base, e9, Y); diag_row<1, 0>(Xs, base, e9, Y); diag_row<2, 0>(Xs, base, e9, Y);
-    load9(ep, 1, e9);
-    diag_row<0, 1>(Xs, base, e9, Y); diag_row<1, 1>(Xs, base, e9, Y); diag_row<2, 1>(Xs, base, e9, Y);
-    load9(ep, 2, e9);
-    diag_row<0, 2>(Xs, base, e9, Y); diag_row<1, 2>(Xs, base, e9, Y); diag_row<2, 2>(Xs, base, e9, Y);
+        for (int i = 0; i < 3; i++) {
+          const int n = i + 3 * j + 9 * k;
+          const double sum = X[0][n] + X[1][n] + X[2][n];
+#pragma unroll
+          for (int c = 0; c < 3; c++) lds_add(&Xs[base + toff(c, i, j, k)], sum + X[c][n]);
+        }
   }
-  __syncthreads();
-  zero_tile(Xs, lane);
-  __syncthreads();
-  if (active) emit_element(Xs, base, Y);
   __syncthreads();
   store_tile_own(b, br, t, Xs, d, facebuf, add_mode != 0, lane);
 }
