@@ -1161,7 +1161,7 @@ struct DevBuf {
 
 // launch shape of a level's smoother apply, picked at set-up by timing (autotune)
 struct LevelTune {
-  int split = 0;              // kernel: 0 one wave per brick, 1 row-split (3 waves per brick),
+  int split = 0;              // kernel: 0 one wave per brick, 1 row-split (3 or 9 waves per brick),
                               // 2 matrix-core form (FP32 smoothing only)
   int fast = 0;               // tile addressing of full tiles: 1 = 32-bit fast path, 0 = general
   double ms = 0.0, ms_default = 0.0;  // measured time per apply: chosen shape, default shape
@@ -1519,7 +1519,7 @@ int time_level(ptq2_mg *mg, int l, int reps, double *ms) {
 }
 
 // Autotuner of the smoother apply, per level: times each launch shape (one wave per brick, the
-// row-split kernel's three, and for FP32 smoothing the matrix-core form; fast or general tile
+// row-split kernel's three or nine, and for FP32 smoothing the matrix-core form; fast or general tile
 // addressing where the tiles are full) and keeps the fastest, the default shape unless another
 // is at least 3% faster.  Levels with few bricks (e.g. 16^3: 64 bricks for 1,024 SIMDs) are
 // latency-bound in the one-wave kernel.
