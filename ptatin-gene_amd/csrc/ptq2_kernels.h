@@ -58,6 +58,12 @@ hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, co
 hipError_t launch_a11_fp64_split(const Box &b, const double *coords, const double *u, const uint8_t *mask,
                                  const double *eta_bm, double *y, bool add, hipStream_t s, double *facebuf,
                                  bool gather = true);
+// The FP32 apply in overlapping blocks (nine waves each), complete in one launch: y = A x with y = x on the mask's
+// dofs or, with co, its Chebyshev update (co->mask is mask, co->x is x; y unused, and out is none of the
+// inputs).  For boxes without ghost layers whose blocks get a CU each (own_blocks_fit).
+bool own_blocks_fit(const Box &b);
+hipError_t launch_a11_fp32_own(const Box &b, const float *x, const uint8_t *mask, const float *fac, float *y,
+                               hipStream_t s, const ChebOut<float> *co = nullptr);
 hipError_t launch_a11_fp32_split(const Box &b, const float *u, const uint8_t *mask, const float *fac, float *y,
                                  bool add, hipStream_t s, float *facebuf, bool gather = true);
 // The FP32 smoother operator with the reference gradient as a dense GEMM on the matrix cores

@@ -531,6 +531,14 @@ __global__ __launch_bounds__(RWAVES * BEL) void k_a11_fp32_rows(Box b, const flo
   a11_rows32_brick(b, brick_xcd(b, blockIdx.x), u, mask, fac, y, add_mode, facebuf);
 }
 
+template <bool CH>
+__global__ __launch_bounds__(RWAVES * BEL) void k_a11_fp32_own(Box b, const float *__restrict__ x,
+                                                               const uint8_t *__restrict__ mask,
+                                                               const float *__restrict__ fac, float *__restrict__ y,
+                                                               ChebOut<float> co) {
+  a11_rows32_own<CH>(b, blockIdx.x, x, mask, fac, y, co);
+}
+
 // ------------------------------------------------------ A11 FP64, stored geometry
 // The same operator with the per-point geometry G = sqrt(w/det) adj(J) resident in HBM
 // (FP64, built once per mesh by k_build_geo64) and eta applied at run time:
@@ -1547,6 +1555,20 @@ hipError_t launch_a11_fp32_split(const Box &b, const float *u, const uint8_t *ma
   else
     hipLaunchKernelGGL(k_a11_fp32_split, dim3(nb), dim3(3 * BEL), 0, s, b, u, mask, fac, y, add ? 1 : 0, facebuf);
   return gather ? launch_gather(b, (const float *)facebuf, y, s) : hipGetLastError();
+}
+
+bool own_blocks_fit(const Box &b) {
+  const bool single = !b.i0 && !b.j0 && !b.k0 && b.NX == 2 * b.mx + 1 && b.NY == 2 * b.my + 1 && b.NZ == 2 * b.mz + 1;
+  return single && (int64_t)own_blocks(b.mx) * own_blocks(b.my) * own_blocks(b.mz) <= NUM_CUS;
+}
+hipError_t launch_a11_fp32_own(const Box &b, const float *x, const uint8_t *mask, const float *fac, float *y,
+                               hipStream_t s, const ChebOut<float> *co) {
+  const dim3 grid(own_blocks(b.mx) * own_blocks(b.my) * own_blocks(b.mz)), block(RWAVES * BEL);
+  if (co)
+    hipLaunchKernelGGL(k_a11_fp32_own<true>, grid, block, 0, s, b, x, mask, fac, y, *co);
+  else
+    hipLaunchKernelGGL(k_a11_fp32_own<false>, grid, block, 0, s, b, x, mask, fac, y, ChebOut<float>{});
+  return hipGetLastError();
 }
 
 template <typename T>

@@ -213,20 +213,17 @@ __device__ __forceinline__ void row_stress(const float F[27], const float g[3][3
   }
 }
 
-// The FP32 pass.  LDS: the velocity tile, later the output tile (FP64 sums) in its place, and the rows'
+// LDS of the FP32 pass: the velocity tile, later the output tile (FP64 sums) in its place, and the rows'
 // values.
-__device__ __forceinline__ void a11_rows32_brick(const Box &b, const BrickId &br, const float *__restrict__ u,
-                                                 const uint8_t *__restrict__ mask, const float *__restrict__ fac,
-                                                 float *__restrict__ y, int add_mode, float *__restrict__ facebuf) {
-  __shared__ double Ts[3 * TCS];
-  __shared__ float Ex[RWAVES * ROWVALS * BEL];
-  float *Us = reinterpret_cast<float *>(Ts);
-  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / BEL), lane = (int)threadIdx.x - BEL * w;
-  const Tile t = tile_of(b, br);
-  float v[PSTEPS], F[27];
-  plane_load_masked(b, t, u, mask, w, lane, v);
-  // the slots of lanes without an element hold something, and nobody takes their outputs
-  const float *fs = fac + ((int64_t)br.lin * 243 + 27 * w) * BEL + lane;
+struct RowsLds32 {
+  double Ts[3 * TCS];
+  float Ex[RWAVES * ROWVALS * BEL];
+};
+// The pass from wave w's plane v of the velocity tile to the output tile L.Ts; fs: the lane's factors of row w.
+__device__ __forceinline__ void a11_rows32(RowsLds32 &L, const float v[PSTEPS], const float *__restrict__ fs,
+                                           bool active, int w, int lane) {
+  float *Us = reinterpret_cast<float *>(L.Ts);
+  float F[27];
 #pragma unroll
   for (int n = 0; n < 27; n++) F[n] = fs[n * BEL];
   plane_put(v, Us, w, lane);
@@ -242,16 +239,15 @@ __device__ __forceinline__ void a11_rows32_brick(const Box &b, const BrickId &br
     }
     row_stress(F, g, dv);
 #pragma unroll
-    for (int c = 0; c < 3; c++) row_hand_over(dv[c], Ex + (ROWVALS * w + 8 * c) * BEL, lane);
+    for (int c = 0; c < 3; c++) row_hand_over(dv[c], L.Ex + (ROWVALS * w + 8 * c) * BEL, lane);
   }
   lds_barrier();  // the velocities are read, the rows' values written
-  for (int n = threadIdx.x; n < 3 * TCS; n += RWAVES * BEL) Ts[n] = 0.0;
+  for (int n = threadIdx.x; n < 3 * TCS; n += RWAVES * BEL) L.Ts[n] = 0.0;
   float Y[9];
   const int c = w % 3, k = w / 3;
-  gather_rows(Ex, lane, c, k, Y);
+  gather_rows(L.Ex, lane, c, k, Y);
   lds_barrier();
-  double *o = Ts + base + c * TCS + TPS * k;
-  const bool active = lane_active(t, lane);
+  double *o = L.Ts + base + c * TCS + TPS * k;
 #pragma unroll
   for (int half = 0; half < 2; half++) {
     if (active && (k == 2) == (half == 1)) {
@@ -262,7 +258,74 @@ __device__ __forceinline__ void a11_rows32_brick(const Box &b, const BrickId &br
     }
     lds_barrier();
   }
-  plane_store(b, br, t, Ts, y, facebuf, add_mode != 0, w, lane);
+}
+
+__device__ __forceinline__ void a11_rows32_brick(const Box &b, const BrickId &br, const float *__restrict__ u,
+                                                 const uint8_t *__restrict__ mask, const float *__restrict__ fac,
+                                                 float *__restrict__ y, int add_mode, float *__restrict__ facebuf) {
+  __shared__ RowsLds32 L;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / BEL), lane = (int)threadIdx.x - BEL * w;
+  const Tile t = tile_of(b, br);
+  float v[PSTEPS];
+  plane_load_masked(b, t, u, mask, w, lane, v);
+  // the factor slots of lanes without an element hold something, and nobody takes their outputs
+  a11_rows32(L, v, fac + ((int64_t)br.lin * 243 + 27 * w) * BEL + lane, lane_active(t, lane), w, lane);
+  plane_store(b, br, t, L.Ts, y, facebuf, add_mode != 0, w, lane);
+}
+
+// Overlapping blocks: 4x4x4 elements each, three elements apart, so that every node is complete in
+// one block (of the nodes 0 .. 8 along an axis an inner block has 1 .. 7 and owns 1 .. 6).  With 64 / 27 of the work
+// there are no face slots, and an apply with its Chebyshev update or its Dirichlet rows is one launch.
+__host__ __device__ constexpr int own_blocks(int m) { return m <= BE ? 1 : (m - BE + 2) / 3 + 1; }
+struct OwnAxis {
+  int e0, lo, hi;  // first element; owned tile nodes lo .. hi
+  __device__ __forceinline__ OwnAxis(int k, int m)
+      : e0(3 * k), lo(k > 0 ? 1 : 0), hi(3 * k + BE < m ? 6 : 2 * (m - 3 * k)) {}
+};
+// y = A x with y = x on the mask's dofs (CH: the Chebyshev update of co instead); single-rank boxes
+template <bool CH>
+__device__ __forceinline__ void a11_rows32_own(const Box &b, int bid, const float *__restrict__ x,
+                                               const uint8_t *__restrict__ mask, const float *__restrict__ fac,
+                                               float *__restrict__ y, const ChebOut<float> &co) {
+  __shared__ RowsLds32 L;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / BEL), lane = (int)threadIdx.x - BEL * w;
+  const int nx = own_blocks(b.mx), ny = own_blocks(b.my);
+  const OwnAxis ax(bid % nx, b.mx), ay(bid / nx % ny, b.my), az(bid / (nx * ny), b.mz);
+  Tile t;
+  t.ex0 = ax.e0; t.ey0 = ay.e0; t.ez0 = az.e0;
+  t.nex = min(BE, b.mx - t.ex0); t.ney = min(BE, b.my - t.ey0); t.nez = min(BE, b.mz - t.ez0);
+  t.tnx = 2 * t.nex + 1; t.tny = 2 * t.ney + 1; t.tnz = 2 * t.nez + 1;
+  t.node0 = 2 * (t.ex0 + (int64_t)b.NX * (t.ey0 + (int64_t)b.NY * t.ez0));
+  float v[PSTEPS], xv[PSTEPS], bv[PSTEPS], dv[PSTEPS], pv[PSTEPS] = {};
+  uint8_t mk[PSTEPS] = {};
+  plane_load(b, t, x, w, lane, xv);
+  if (mask) plane_load(b, t, mask, w, lane, mk);
+  if (CH) {  // the update's operands travel behind the tile
+    plane_load(b, t, co.b, w, lane, bv);
+    plane_load(b, t, co.dinv, w, lane, dv);
+    if (co.pkm1) plane_load(b, t, co.pkm1, w, lane, pv);
+  }
+#pragma unroll
+  for (int it = 0; it < PSTEPS; it++) v[it] = mk[it] ? 0.0f : xv[it];  // BCListInsertLocalZero, src/dmda_bcs.c:581-608
+  const LaneElem e = lane_elem(lane);
+  const int ex = min(t.ex0 + e.lx, b.mx - 1), ey = min(t.ey0 + e.ly, b.my - 1), ez = min(t.ez0 + e.lz, b.mz - 1);
+  const int64_t brick = ex / BE + (int64_t)b.nbx * (ey / BE + (int64_t)b.nby * (ez / BE));
+  a11_rows32(L, v, fac + (brick * 243 + 27 * w) * BEL + elem_lane(ex % BE, ey % BE, ez % BE), lane_active(t, lane), w,
+             lane);
+  const RowLane R(lane);
+  if (R.p > 1 || R.ii < ax.lo || R.ii > ax.hi || w < az.lo || w > az.hi) return;
+  const int64_t col = 3 * (t.node0 + R.ii + (int64_t)b.NX * b.NY * w) + R.c;
+#pragma unroll
+  for (int it = 0; it < PSTEPS; it++) {
+    const int yy = 2 * it + R.p;
+    if (yy < ay.lo || yy > ay.hi) continue;
+    const int64_t gi = col + 3 * (int64_t)b.NX * yy;
+    const float val = mk[it] ? xv[it] : (float)L.Ts[R.lds_col + TRS * yy + TPS * w];
+    if (CH)
+      co.out[gi] = cheb_value(co, dv[it], bv[it], val, xv[it], pv[it], co.pkm1 != nullptr);
+    else
+      y[gi] = val;
+  }
 }
 
 }  // namespace ptq2

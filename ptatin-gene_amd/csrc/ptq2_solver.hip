@@ -1248,6 +1248,11 @@ int level_matmult(ptq2_mg *mg, int l, const T *x, T *y);
 template <typename T>
 hipError_t galerkin_mf(ptq2_mg *mg, int l, const T *x, T *y);
 
+// the row-split FP32 kernel in overlapping blocks, complete without face pass and Dirichlet rows
+bool level_own(const ptq2_mg *mg, int l) {
+  return mg->f32 && mg->tune[l].split == 1 && !mg->gal[l] && ptq2::own_blocks_fit(mg->lbox[l]);
+}
+
 // (the row-split choice is made for the smoothing precision and applies to it only)
 hipError_t level_launch(ptq2_mg *mg, int l, const double *x, double *y, bool gather) {
   ptq2_ctx *c = mg->ctx[l];
@@ -1276,6 +1281,7 @@ hipError_t level_launch(ptq2_mg *mg, int l, const float *x, float *y, bool gathe
                        (const float *)mg->gst32[l], x, y);
     return hipGetLastError();
   }
+  if (level_own(mg, l)) return ptq2::launch_a11_fp32_own(b, x, c->mask, c->fac32, y, mg->stream);
   if (mg->tune[l].split == 1 && mg->f32)
     return ptq2::launch_a11_fp32_split(b, x, c->mask, c->fac32, y, false, mg->stream, (float *)c->facebuf, gather);
   if (mg->tune[l].split == 2 && mg->f32)
@@ -1316,6 +1322,7 @@ template <>
 int level_matmult<float>(ptq2_mg *mg, int l, const float *x, float *y) {
   ptq2_ctx *c = mg->ctx[l];
   MGCHK(level_launch(mg, l, x, y, true));
+  if (level_own(mg, l)) return PTQ2_OK;
   MGCHK(ptq2::launch_bc_rows<float>(c->ndir, c->dir_idx, x, y, 0, mg->stream));
   return PTQ2_OK;
 }
@@ -1370,6 +1377,12 @@ int chebyshev(ptq2_mg *mg, int l, bool zero_guess) {
   auto step = [&](const T *xin, const T *pkm1, T *out, double cr, double ck, double cx) -> int {
     const ptq2::ChebOut<T> co{(const T *)b, (const T *)dinv, xin, pkm1, out, (const uint8_t *)lc->mask, (T)cr, (T)ck,
                               (T)cx};
+    if constexpr (sizeof(T) == 4) {
+      if (level_own(mg, l)) {
+        MGCHK(ptq2::launch_a11_fp32_own(mg->lbox[l], xin, lc->mask, lc->fac32, (float *)nullptr, mg->stream, &co));
+        return PTQ2_OK;
+      }
+    }
     if (fz)
       MGRC(level_apply_cheb<T>(mg, l, xin, y, co));
     else
