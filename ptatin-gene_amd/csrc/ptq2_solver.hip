@@ -73,14 +73,13 @@ __global__ void k_vout(const VcIO *__restrict__ io, int64_t n, const T *__restri
 }
 
 
-// p1 = scale * Dinv * r0 + x, with r0 = b (zero guess) or b - y
+// the first step from a zero guess: p1 = scale * Dinv * b, and the guess itself
 template <typename T>
-__global__ void k_cheb_first(int64_t n, const T *__restrict__ b, const T *__restrict__ y, const T *__restrict__ dinv,
-                             const T *__restrict__ x, T *__restrict__ p, T scale) {
+__global__ void k_cheb_first(int64_t n, const T *__restrict__ b, const T *__restrict__ dinv, T *__restrict__ guess,
+                             T *__restrict__ p, T scale) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    T r = y ? b[i] - y[i] : b[i];
-    T xi = x ? x[i] : T(0);
-    p[i] = scale * dinv[i] * r + xi;
+    p[i] = scale * dinv[i] * b[i] + T(0);
+    guess[i] = T(0);
   }
 }
 
@@ -242,13 +241,17 @@ __global__ void k_restrict(int NXc, int NYc, int NZc, int NXf, int NYf, int NZf,
   }
 }
 
-// x_f += P x_c (trilinear), not on fine Dirichlet dofs
+// x_f = x_s + P x_c (trilinear), x_s alone on fine Dirichlet dofs; x_s may be x_f, and null is zero
 template <typename T>
 __global__ void k_prolong_add(int NXc, int NYc, int NXf, int NYf, int NZf, const T *__restrict__ xc,
-                              const uint8_t *__restrict__ fmask, T *__restrict__ xf) {
+                              const uint8_t *__restrict__ fmask, const T *xs, T *xf) {
   int64_t nf = 3 * (int64_t)NXf * NYf * NZf;
   for (int64_t d = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; d < nf; d += (int64_t)gridDim.x * blockDim.x) {
-    if (fmask && fmask[d]) continue;
+    const T x0 = xs ? xs[d] : T(0);
+    if (fmask && fmask[d]) {
+      xf[d] = x0;
+      continue;
+    }
     int comp = (int)(d % 3);
     int64_t node = d / 3;
     int i = (int)(node % NXf), j = (int)((node / NXf) % NYf), k = (int)(node / ((int64_t)NXf * NYf));
@@ -275,7 +278,7 @@ __global__ void k_prolong_add(int NXc, int NYc, int NXf, int NYf, int NZf, const
       }
       s = (s + s3) * wk;
     }
-    xf[d] += s;
+    xf[d] = x0 + s;
   }
 }
 
@@ -460,13 +463,38 @@ constexpr int MD = 8;      // vectors per pass over w
 constexpr int MDB = 2048;  // blocks of the reduction kernels (partials per product)
 constexpr int MDU = 4;     // grid strides per loop iteration (independent loads in flight)
 
-template <int NR>
-__device__ __forceinline__ void block_partials(double (&s)[NR], double (*red)[TPB / 64]) {
+// The wave sums of NR values per lane.  A step that adds lane l + OFF to lane l leaves half the lanes
+// idle, so two values share it: the lower lanes get the first's sums and the upper lanes the second's, in
+// the order a value alone would be summed.  NR + NR / 2 + ... exchanges instead of 6 NR, which is what
+// a projection of 16 vectors (35 values) waits for.  Lane l ends with value number wave_row(l).
+template <int NR, int OFF>
+__device__ __forceinline__ double wave_sums(const double (&s)[NR]) {
+  constexpr int H = (NR + 1) / 2;
+  const bool up = (threadIdx.x & OFF) != 0;
+  double r[H];
 #pragma unroll
-  for (int m = 0; m < NR; m++) {
-    for (int off = 32; off > 0; off >>= 1) s[m] += __shfl_down(s[m], off, 64);
-    if ((threadIdx.x & 63) == 0) red[m][threadIdx.x / 64] = s[m];
+  for (int k = 0; k < H; k++) {
+    const double a = s[2 * k], b = 2 * k + 1 < NR ? s[2 * k + 1] : 0.0;
+    r[k] = (up ? b : a) + __shfl_xor(up ? a : b, OFF, 64);
   }
+  if constexpr (OFF > 1)
+    return wave_sums<H, OFF / 2>(r);
+  else
+    return r[0];
+}
+__device__ __forceinline__ int wave_row(int lane) { return (int)(__brev((unsigned)lane) >> 26); }
+template <int NR>
+__device__ __forceinline__ void block_partials(const double (&s)[NR], double (*red)[TPB / 64]) {
+  static_assert(NR <= 64, "one value per lane");
+  const double v = wave_sums<NR, 32>(s);
+  const int row = wave_row(threadIdx.x & 63);
+  if (row < NR) red[row][threadIdx.x / 64] = v;
+}
+// A block whose share of n elements is empty: zeros for its rows of part, nothing to sum
+__device__ __forceinline__ bool idle_block(int64_t n, int rows, double *__restrict__ part) {
+  if ((int64_t)blockIdx.x * TPB < n || blockIdx.x == 0) return false;
+  for (int r = threadIdx.x; r < rows; r += TPB) part[(int64_t)r * MDB + blockIdx.x] = 0.0;
+  return true;
 }
 
 // part[v * MDB + block]: partial of V[v].w for v < nv; with self, part[nv * MDB + block]:
@@ -475,6 +503,7 @@ template <typename VT>
 __global__ __launch_bounds__(TPB) void k_mdot(int64_t n, const VT *const *__restrict__ V, int nv,
                                               const double *__restrict__ w, int self, double *__restrict__ part) {
   __shared__ double red[MD + 1][TPB / 64];
+  if (idle_block(n, nv + (self ? 1 : 0), part)) return;
   const int64_t stride = (int64_t)MDB * TPB;
   const int64_t i0 = (int64_t)blockIdx.x * TPB + threadIdx.x;
   const int ngroups = nv > 0 ? (nv + MD - 1) / MD : 1;
@@ -541,6 +570,7 @@ __global__ __launch_bounds__(TPB) void k_maxpy_norm(int64_t n, const VT *const *
                                                     const double *__restrict__ h, double *__restrict__ w,
                                                     double *__restrict__ part) {
   __shared__ double red[1][TPB / 64];
+  if (idle_block(n, 1, part)) return;
   double acc[1] = {0.0};
   for (int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x; i < n; i += (int64_t)MDB * TPB) {
     double s = w[i];
@@ -565,6 +595,7 @@ __global__ __launch_bounds__(TPB) void k_mdot2(int64_t n, const VT *const *__res
                                                double *__restrict__ part) {
   constexpr int NR = 2 * MD2 + 3;
   __shared__ double red[NR][TPB / 64];
+  if (idle_block(n, 2 * nv + 3, part)) return;
   const int64_t stride = (int64_t)MDB * TPB;
   const int64_t i0 = (int64_t)blockIdx.x * TPB + threadIdx.x;
   const int ngroups = nv > 0 ? (nv + MD2 - 1) / MD2 : 1;
@@ -642,6 +673,7 @@ __global__ __launch_bounds__(TPB) void k_dcgs_update(int64_t n, const VT *const 
                                                      const double *u, VT *vo, const double *__restrict__ w,
                                                      double *__restrict__ wo, double *__restrict__ part) {
   __shared__ double red[1][TPB / 64];
+  if (idle_block(n, 1, part)) return;
   double acc[1] = {0.0};
   for (int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x; i < n; i += (int64_t)MDB * TPB) {
     double sa = 0.0, sb = 0.0;
@@ -670,6 +702,7 @@ __global__ __launch_bounds__(TPB) void k_mdot2_f32(int64_t n, const float *const
   constexpr int NR = 2 * MD2 + 3;
   __shared__ double red[NR][TPB / 64];
   const int64_t np = n >> 1;
+  if (idle_block(np, 2 * nv + 3, part)) return;
   const int64_t stride = (int64_t)MDB * TPB;
   const int64_t i0 = (int64_t)blockIdx.x * TPB + threadIdx.x;
   const bool tail = (n & 1) && i0 == 0;
@@ -765,6 +798,7 @@ __global__ __launch_bounds__(TPB) void k_dcgs_update_f32(int64_t n, const float 
                                                          float *__restrict__ vo, const double *__restrict__ w,
                                                          double *__restrict__ wo, double *__restrict__ part) {
   __shared__ double red[1][TPB / 64];
+  if (idle_block(n >> 1, 1, part)) return;
   double acc[1] = {0.0};
   const int64_t np = n >> 1;
   const double2 *u2 = (const double2 *)u, *w2 = (const double2 *)w;
@@ -1299,9 +1333,8 @@ hipError_t galerkin_mf(ptq2_mg *mg, int l, const T *x, T *y) {
   const int *mc = &mg->m[3 * l], *mf = &mg->m[3 * (l - 1)];
   const int NXc = 2 * mc[0] + 1, NYc = 2 * mc[1] + 1, NZc = 2 * mc[2] + 1;
   const int NXf = 2 * mf[0] + 1, NYf = 2 * mf[1] + 1, NZf = 2 * mf[2] + 1;
-  hipLaunchKernelGGL(k_fill<T>, dim3(nblk(nf)), dim3(TPB), 0, mg->stream, nf, gp, T(0));
   hipLaunchKernelGGL(k_prolong_add<T>, dim3(nblk(nf)), dim3(TPB), 0, mg->stream, NXc, NYc, NXf, NYf, NZf, x,
-                     (const uint8_t *)f->mask, gp);
+                     (const uint8_t *)f->mask, (const T *)nullptr, gp);
   hipError_t e = level_launch(mg, l - 1, (const T *)gp, ga, true);
   if (e == hipSuccess) e = ptq2::launch_bc_rows<T>(f->ndir, f->dir_idx, (const T *)gp, ga, 0, mg->stream);
   if (e != hipSuccess) return e;
@@ -1353,12 +1386,30 @@ int level_apply_cheb<float>(ptq2_mg *mg, int l, const float *x, float *y, const 
   return PTQ2_OK;
 }
 
-// ChebychevRN on level l: x <- smoothed solution of A x = b; zero_guess skips the first residual
+// The three vectors of the Chebyshev recurrence on level l in the order guess, first step, second step; the
+// steps go round them, and the order is such that the last one writes vx.
+template <typename T>
+void cheb_buffers(const ptq2_mg *mg, int l, T *buf[3]) {
+  const int last = (1 + mg->opt.smooth_its) % 3;
+  buf[last] = (T *)mg->vx[l];
+  buf[(last + 1) % 3] = (T *)mg->vp1[l];
+  buf[(last + 2) % 3] = (T *)mg->vp2[l];
+}
+// where a smoothing of level l with an initial guess expects it
+template <typename T>
+T *cheb_guess(const ptq2_mg *mg, int l) {
+  T *buf[3];
+  cheb_buffers(mg, l, buf);
+  return buf[0];
+}
+
+// ChebychevRN on level l: vx <- smoothed solution of A x = b from the guess in cheb_guess, or from zero
 template <typename T>
 int chebyshev(ptq2_mg *mg, int l, bool zero_guess) {
   const int64_t n = mg->n[l];
-  T *b = (T *)mg->vb[l], *x = (T *)mg->vx[l], *y = (T *)mg->vy[l], *dinv = (T *)mg->vdinv[l];
-  T *buf[3] = {x, (T *)mg->vp1[l], (T *)mg->vp2[l]};
+  T *b = (T *)mg->vb[l], *y = (T *)mg->vy[l], *dinv = (T *)mg->vdinv[l];
+  T *buf[3];
+  cheb_buffers(mg, l, buf);
   const double emax = mg->emax[l], emin = mg->emin[l];
   const double scale = 2.0 / (emax + emin);
   const double alpha = 1.0 - scale * emin;
@@ -1393,11 +1444,10 @@ int chebyshev(ptq2_mg *mg, int l, bool zero_guess) {
     return PTQ2_OK;
   };
   if (zero_guess) {
-    hipLaunchKernelGGL(k_cheb_first<T>, dim3(nblk(n)), dim3(TPB), 0, mg->stream, n, (const T *)b, (const T *)nullptr,
-                       (const T *)dinv, (const T *)nullptr, buf[k], (T)scale);
-    hipLaunchKernelGGL(k_fill<T>, dim3(nblk(n)), dim3(TPB), 0, mg->stream, n, x, T(0));
+    hipLaunchKernelGGL(k_cheb_first<T>, dim3(nblk(n)), dim3(TPB), 0, mg->stream, n, (const T *)b, (const T *)dinv,
+                       buf[km1], buf[k], (T)scale);
   } else {
-    MGRC(step(x, nullptr, buf[k], scale, 0.0, 1.0));
+    MGRC(step(buf[km1], nullptr, buf[k], scale, 0.0, 1.0));
   }
   for (int i = 0; i < mg->opt.smooth_its; i++) {
     c[kp1] = 2.0 * mu * c[k] - c[km1];
@@ -1408,7 +1458,6 @@ int chebyshev(ptq2_mg *mg, int l, bool zero_guess) {
     k = kp1;
     kp1 = t;
   }
-  if (k != 0) MGCHK(hipMemcpyAsync(x, buf[k], sizeof(T) * n, hipMemcpyDeviceToDevice, mg->stream));
   return hipGetLastError() == hipSuccess ? PTQ2_OK : mgfail(mg, PTQ2_ERR_DEVICE, "chebyshev launch");
 }
 
@@ -1440,7 +1489,7 @@ int vcycle_level(ptq2_mg *mg, int l) {
   MGRC(vcycle_level<T>(mg, l + 1));
   prof_mark(mg, l, 2);
   hipLaunchKernelGGL(k_prolong_add<T>, dim3(nblk(n)), dim3(TPB), 0, mg->stream, NXc, NYc, NXf, NYf, NZf,
-                     (const T *)mg->vx[l + 1], (const uint8_t *)mg->ctx[l]->mask, x);
+                     (const T *)mg->vx[l + 1], (const uint8_t *)mg->ctx[l]->mask, (const T *)x, cheb_guess<T>(mg, l));
   MGRC(chebyshev<T>(mg, l, false));
   prof_mark(mg, l, 3);
   return hipGetLastError() == hipSuccess ? PTQ2_OK : mgfail(mg, PTQ2_ERR_DEVICE, "v-cycle launch");
@@ -1473,9 +1522,8 @@ int build_galerkin_level(ptq2_mg *mg, int l) {
         for (int comp = 0; comp < 3 && !rc; comp++) {
           hipLaunchKernelGGL(k_probe_vec, dim3(nblk(nc)), dim3(TPB), 0, mg->stream, NXc, NYc, NZc, 5, cx, cy, cz,
                              comp, (const uint8_t *)c->mask, e);
-          hipLaunchKernelGGL(k_fill<double>, dim3(nblk(nf)), dim3(TPB), 0, mg->stream, nf, vf, 0.0);
           hipLaunchKernelGGL(k_prolong_add<double>, dim3(nblk(nf)), dim3(TPB), 0, mg->stream, NXc, NYc, NXf, NYf,
-                             NZf, (const double *)e, (const uint8_t *)f->mask, vf);
+                             NZf, (const double *)e, (const uint8_t *)f->mask, (const double *)nullptr, vf);
           rc = level_matmult<double>(mg, l - 1, vf, wf);
           hipLaunchKernelGGL(k_restrict<double>, dim3(nblk(nc)), dim3(TPB), 0, mg->stream, NXc, NYc, NZc, NXf, NYf,
                              NZf, (const double *)wf, (const double *)nullptr, (const uint8_t *)c->mask, w);
@@ -2437,9 +2485,9 @@ int ptq2_mg_create(ptq2_mg **out, ptq2_ctx *fine, const ptq2_mg_opts *opts) {
               // restriction writes zeros there)
               const int *mf = &mg->m[3 * lf];
               const int NXf = 2 * mf[0] + 1, NYf = 2 * mf[1] + 1, NZf = 2 * mf[2] + 1;
-              hipLaunchKernelGGL(k_fill<double>, dim3(nblk(nf)), dim3(TPB), 0, mg->stream, nf, vf, 0.0);
               hipLaunchKernelGGL(k_prolong_add<double>, dim3(nblk(nf)), dim3(TPB), 0, mg->stream, NXc, NYc, NXf, NYf,
-                                 NZf, (const double *)e, (const uint8_t *)mg->ctx[lf]->mask, vf);
+                                 NZf, (const double *)e, (const uint8_t *)mg->ctx[lf]->mask, (const double *)nullptr,
+                                 vf);
               rc = level_matmult<double>(mg, lf, vf, wf);
               hipLaunchKernelGGL(k_restrict<double>, dim3(nblk(nc)), dim3(TPB), 0, mg->stream, NXc, NYc, NZc, NXf,
                                  NYf, NZf, (const double *)wf, (const double *)nullptr, cmask, w);
