@@ -86,6 +86,12 @@ void dev_free(void *p) {
   if (p) (void)hipFree(p);
 }
 
+// the Dirichlet rows of a MatMult-like call for its face pass (mode as in launch_bc_rows), none unless mm
+template <typename T>
+ptq2::BcRows<T> bc_of(const ptq2_ctx *c, bool mm, int mode, const T *x = nullptr, const T *v = nullptr) {
+  return ptq2::BcRows<T>{mm ? c->ndir : 0, c->dir_idx, c->mask, x, v, mode};
+}
+
 int ensure(ptq2_ctx *c, void **buf, size_t *have, size_t need) {
   if (*have >= need) return PTQ2_OK;
   dev_free(*buf);
@@ -141,7 +147,10 @@ int ptq2_internal_build_fac32(ptq2_ctx *c, bool block) {
 
 void *ptq2_internal_facebuf(ptq2_ctx *c, int *rc) {
   *rc = PTQ2_OK;
-  if (!c->facebuf) *rc = dev_alloc(c, &c->facebuf, sizeof(double) * (size_t)c->nbricks * ptq2::FACEVALS);
+  if (!c->facebuf) {
+    *rc = dev_alloc(c, &c->facebuf_own, sizeof(double) * (size_t)c->nbricks * ptq2::FACEVALS);
+    c->facebuf = c->facebuf_own;
+  }
   return c->facebuf;
 }
 
@@ -247,7 +256,7 @@ int ptq2_destroy(ptq2_ctx **pc) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   dev_free(c->coords); dev_free(c->mask); dev_free(c->dir_idx); dev_free(c->eta_bm);
-  dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf);
+  dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf_own);
   dev_free(c->pwork);
   dev_free(c->err); dev_free(c->su); dev_free(c->sy); dev_free(c->sp); dev_free(c->syp); dev_free(c->ures);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
@@ -325,11 +334,11 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->gen++;
   dev_free(c->coords); dev_free(c->mask); dev_free(c->dir_idx); dev_free(c->eta_bm);
-  dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf);
+  dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf_own);
   dev_free(c->pwork);
   c->coords = nullptr; c->mask = nullptr; c->dir_idx = nullptr; c->eta_bm = nullptr;
   c->xtile = nullptr; c->bdir = nullptr;
-  c->fac32 = nullptr; c->facb32 = nullptr; c->geo64 = nullptr; c->facebuf = nullptr;
+  c->fac32 = nullptr; c->facb32 = nullptr; c->geo64 = nullptr; c->facebuf = c->facebuf_own = nullptr;
   c->pwork = nullptr; c->pwork_bytes = 0;
   c->mesh_ready = c->eta_ready = c->fac32_valid = c->facb32_valid = c->geo64_valid = c->has_state = false;
   c->ndir = 0;
@@ -366,22 +375,24 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
       HIPCHK(c, hipMemcpy(c->dir_idx, idx.data(), sizeof(int64_t) * idx.size(), hipMemcpyHostToDevice));
     }
   }
-  // Viscosity and the resident coordinate tiles share an allocation.  The tiles pay where the vectors
-  // come from HBM, not from the 256 MB cache before it: FP64 apply 1113 us with, 1163 us without at
-  // 128^3 elements (32768 bricks), 145 us with and without at 64^3 (4096 bricks), where they would only
-  // make the set-up longer (by a tenth at 33^3).  A mesh that fits the device only without them runs
-  // its FP64 passes from the coordinates too.
-  const size_t neta = (size_t)nb * 27 * ptq2::BEL, nxt = nb >= 8192 ? (size_t)nb * 3 * ptq2::TCS : 0;
-  if (nxt && dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * (neta + nxt)) == PTQ2_OK)
-    c->xtile = c->eta_bm + neta;
-  else if ((rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * neta)))
-    return rc;
+  // Viscosity, face slots and the resident coordinate tiles share an allocation (a hipMalloc of its own for
+  // the slots makes the set-up of a 40^3 mesh a tenth longer, and in an operator's first call it would be
+  // refused under capture).  The tiles pay where the vectors come from HBM, not from the 256 MB cache before it:
+  // FP64 apply 1113 us with, 1163 us without at 128^3 elements (32768 bricks), 145 us with and without at 64^3
+  // (4096 bricks), where they would only make the set-up longer (by a tenth at 33^3).  A mesh that fits
+  // the device only without them runs its FP64 passes from the coordinates too; one that fits only without the
+  // face slots gets them, or the error, in the first call that needs them.
+  const size_t neta = (size_t)nb * 27 * ptq2::BEL, nface = (size_t)nb * ptq2::FACEVALS + 1,
+               nxt = nb >= 8192 ? (size_t)nb * 3 * ptq2::TCS : 0;
+  const size_t oface = neta, oxt = oface + (nface & ~(size_t)1);  // 16-byte aligned parts
+  rc = nxt ? dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * (oxt + nxt)) : PTQ2_ERR_ALLOC;
+  if (rc == PTQ2_OK) c->xtile = c->eta_bm + oxt;
+  if (rc) rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * oxt);
+  if (rc == PTQ2_OK) c->facebuf = c->eta_bm + oface;
+  if (rc && (rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * neta))) return rc;
   b.xtile = c->xtile;
   c->box = b;
   c->nnodes = nn; c->nvel = 3 * nn; c->nel = ne; c->npres = 4 * ne; c->nbricks = nb;
-  // the face slots now, so that no operator's first call allocates (it may be under capture); where they
-  // do not fit, that call says so
-  (void)ptq2_internal_facebuf(c, &rc);
   if ((rc = clear_err(c))) return rc;
   HIPCHK(c, ptq2::launch_check_mesh(b, c->coords, c->xtile, c->err, c->stream));
   int bits = 0;
@@ -486,21 +497,23 @@ int ptq2_a11_apply(ptq2_ctx *c, const void *u, void *y, unsigned flags) {
   void *tb = ptq2_internal_facebuf(c, &rc);
   if (rc) return rc;
   if (f32) {
-    if (flags & PTQ2_MFMA)
+    const auto bc = bc_of(c, mm, 0, (const float *)du);
+    if (flags & PTQ2_MFMA) {
       HIPCHK(c, ptq2::launch_a11_fp32_mfma(c->box, (const float *)du, mask, c->fac32, (float *)dy, add, c->stream,
-                                           (float *)tb));
-    else
+                                           (float *)tb, false));
+      HIPCHK(c, ptq2::launch_gather_faces(c->box, (const float *)tb, (float *)dy, c->stream, &bc));
+    } else {
       HIPCHK(c, ptq2::launch_a11_fp32(c->box, (const float *)du, mask, c->fac32, (float *)dy, add, c->stream,
-                                      (float *)tb));
-    if (mm) HIPCHK(c, ptq2::launch_bc_rows<float>(c->ndir, c->dir_idx, (const float *)du, (float *)dy, 0, c->stream));
+                                      (float *)tb, true, nullptr, &bc));
+    }
   } else {
+    const auto bc = bc_of(c, mm, 0, (const double *)du);
     if (otf)
       HIPCHK(c, ptq2::launch_a11_fp64(c->box, c->coords, (const double *)du, mask, c->eta_bm, (double *)dy,
                                       out_mode(c, mm, add), c->stream, (double *)tb));
     else
       HIPCHK(c, ptq2::launch_a11_fp64g(c->box, (const double *)du, mask, c->geo64, c->eta_bm, (double *)dy, add,
-                                       c->stream, (double *)tb));
-    if (mm && !otf) HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, (const double *)du, (double *)dy, 0, c->stream));
+                                       c->stream, (double *)tb, &bc));
   }
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(y, c->sy, es * (size_t)n, hipMemcpyDeviceToHost, c->stream));
@@ -635,8 +648,8 @@ int ptq2_a11_diag(ptq2_ctx *c, double *d, unsigned flags) {
   }
   void *fb = ptq2_internal_facebuf(c, &rc);
   if (rc) return rc;
-  HIPCHK(c, ptq2::launch_diag(c->box, c->coords, c->eta_bm, dd, add, (double *)fb, c->stream));
-  if (mm) HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, (const double *)nullptr, dd, 2, c->stream));
+  const auto bc = bc_of<double>(c, mm, 2);
+  HIPCHK(c, ptq2::launch_diag(c->box, c->coords, c->eta_bm, dd, add, (double *)fb, c->stream, &bc));
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(d, dd, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -664,8 +677,8 @@ int ptq2_a12_apply(ptq2_ctx *c, const double *p, double *yu, unsigned flags) {
   }
   void *fb = ptq2_internal_facebuf(c, &rc);
   if (rc) return rc;
-  HIPCHK(c, ptq2::launch_a12(c->box, c->coords, dp, dy, add, (double *)fb, c->stream));
-  if (mm) HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, (const double *)nullptr, dy, 1, c->stream));
+  const auto bc = bc_of<double>(c, mm, 1);
+  HIPCHK(c, ptq2::launch_a12(c->box, c->coords, dp, dy, add, (double *)fb, c->stream, &bc));
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(yu, dy, sizeof(double) * (size_t)c->nvel, hipMemcpyDeviceToHost, c->stream));
     int bits = 0;
@@ -696,8 +709,8 @@ int ptq2_body_force(ptq2_ctx *c, const double *fu, double *y, unsigned flags) {
   }
   void *fb = ptq2_internal_facebuf(c, &rc);
   if (rc) return rc;
-  HIPCHK(c, ptq2::launch_body_force(c->box, c->coords, df, dy, add, (double *)fb, c->stream));
-  if (mm) HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, (const double *)nullptr, dy, 1, c->stream));
+  const auto bc = bc_of<double>(c, mm, 1);
+  HIPCHK(c, ptq2::launch_body_force(c->box, c->coords, df, dy, add, (double *)fb, c->stream, 1.0, &bc));
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(y, dy, sizeof(double) * (size_t)c->nvel, hipMemcpyDeviceToHost, c->stream));
     int bits = 0;
@@ -774,23 +787,22 @@ int ptq2_stokes_apply(ptq2_ctx *c, const void *u, const void *p, void *yu, void 
   if (rc) return rc;
   if (f32) {
     // one fused pass (MFStokesWrapper_A_AVX's single element loop), FP32 factors
+    const auto bc = bc_of(c, mm, 0, (const float *)du);
     HIPCHK(c, ptq2::launch_stokes_fp32(c->box, (const float *)du, (const float *)dp, mask, c->fac32, c->facb32,
-                                       (float *)dyu, (float *)dyp, add, c->stream, (float *)fb));
-    if (mm) HIPCHK(c, ptq2::launch_bc_rows<float>(c->ndir, c->dir_idx, (const float *)du, (float *)dyu, 0, c->stream));
+                                       (float *)dyu, (float *)dyp, add, c->stream, (float *)fb, &bc));
   } else {
+    const auto bc = bc_of(c, mm, 0, (const double *)du);
     if (otf) {
       // momentum A11 u + A12 p and continuity A21 u in one element pass (MFStokesWrapper_A_AVX)
       HIPCHK(c, ptq2::launch_stokes_fp64(c->box, c->coords, (const double *)du, (const double *)dp, mask, c->eta_bm,
-                                         (double *)dyu, (double *)dyp, nullptr, add, c->stream, (double *)fb));
+                                         (double *)dyu, (double *)dyp, nullptr, add, c->stream, (double *)fb, &bc));
     } else {
       // resident geometry: the A11 kernel of that form, then A12 and A21
       HIPCHK(c, ptq2::launch_a11_fp64g(c->box, (const double *)du, mask, c->geo64, c->eta_bm, (double *)dyu, add,
                                        c->stream, (double *)fb));
-      HIPCHK(c, ptq2::launch_a12(c->box, c->coords, (const double *)dp, (double *)dyu, true, (double *)fb, c->stream));
+      HIPCHK(c, ptq2::launch_a12(c->box, c->coords, (const double *)dp, (double *)dyu, true, (double *)fb, c->stream, &bc));
       HIPCHK(c, ptq2::launch_a21(c->box, c->coords, (const double *)du, mask, (double *)dyp, add, c->stream));
     }
-    if (mm)
-      HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, (const double *)du, (double *)dyu, 0, c->stream));
   }
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(yu, dyu, es * (size_t)c->nvel, hipMemcpyDeviceToHost, c->stream));
@@ -845,8 +857,7 @@ int ptq2_stokes_residual(ptq2_ctx *c, const double *u, const double *p, const do
   const double *ul = du;
   if (c->ndir) {
     if ((rc = ensure(c, (void **)&c->ures, &c->ures_bytes, sizeof(double) * (size_t)nv))) return rc;
-    HIPCHK(c, hipMemcpyAsync(c->ures, du, sizeof(double) * (size_t)nv, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, dphi, c->ures, dphi ? 0 : 1, c->stream));
+    HIPCHK(c, ptq2::launch_insert_bc(nv, du, c->mask, dphi, c->ures, c->stream));
     ul = c->ures;
   }
   void *fb = ptq2_internal_facebuf(c, &rc);
@@ -854,9 +865,9 @@ int ptq2_stokes_residual(ptq2_ctx *c, const double *u, const double *p, const do
   // Fu = A11 u_loc + A12 p, Fp = A21 u_loc - int N^p fp (one element pass), then Fu -= Be
   HIPCHK(c, ptq2::launch_stokes_fp64(c->box, c->coords, ul, dp, nullptr, c->eta_bm, dFu, dFp, dfp, false, c->stream,
                                      (double *)fb));
-  HIPCHK(c, ptq2::launch_body_force(c->box, c->coords, dfu, dFu, true, (double *)fb, c->stream, -1.0));
   // Dirichlet rows: Fu_D = u_D - phi_D (BCListResidualDirichlet, src/dmda_bcs.c:614-648)
-  HIPCHK(c, ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, du, dFu, 3, c->stream, dphi));
+  const auto bc = bc_of(c, true, 3, du, dphi);
+  HIPCHK(c, ptq2::launch_body_force(c->box, c->coords, dfu, dFu, true, (double *)fb, c->stream, -1.0, &bc));
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(Fu, dFu, sizeof(double) * (size_t)nv, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipMemcpyAsync(Fp, dFp, sizeof(double) * (size_t)np, hipMemcpyDeviceToHost, c->stream));

@@ -39,7 +39,8 @@ struct ptq2_ctx {
   // pass adds the face slots into their owners (ptq2::launch_a11_*).  One launch keeps the
   // memory phases of some bricks overlapped with the arithmetic of others, which 8 coloured
   // launches of a few waves per SIMD do not.
-  void *facebuf = nullptr;
+  void *facebuf = nullptr;      // beside eta_bm, or facebuf_own
+  void *facebuf_own = nullptr;  // allocated on first use where the mesh set-up had no room
   // u with the Dirichlet values inserted, for the residual (allocated on first use)
   double *ures = nullptr;
   size_t ures_bytes = 0;

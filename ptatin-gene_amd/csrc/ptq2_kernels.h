@@ -36,6 +36,17 @@ constexpr int ERRBIT_MESH = 1;
 constexpr int ERRBIT_VISCOSITY = 2;
 constexpr int ERRBIT_NONFINITE = 4;
 
+// Dirichlet rows that an operator writes last (modes of launch_bc_rows); mask marks the same dofs as idx.  The
+// face pass takes them along in blocks of its own and leaves the masked dofs to those.
+template <typename T>
+struct BcRows {
+  int64_t n;
+  const int64_t *idx;
+  const uint8_t *mask;
+  const T *x, *v;
+  int mode;
+};
+
 // A11 launchers: with facebuf (FACEVALS values per brick) all bricks run in one launch,
 // storing the nodes they own, and k_gather_faces adds the shared face values into their
 // owners (gather = false leaves that to the caller's next kernel, which then reads the face
@@ -49,10 +60,10 @@ hipError_t launch_a11_fp64(const Box &b, const double *coords, const double *u, 
 // subtracts the continuity source from yp
 hipError_t launch_stokes_fp64(const Box &b, const double *coords, const double *u, const double *p,
                               const uint8_t *mask, const double *eta_bm, double *yu, double *yp, const double *fp,
-                              bool add, hipStream_t s, double *facebuf);
+                              bool add, hipStream_t s, double *facebuf, const BcRows<double> *bc = nullptr);
 hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, const float *fac, float *y, bool add,
                            hipStream_t s, float *facebuf = nullptr, bool gather = true,
-                           const ChebOut<float> *co = nullptr);
+                           const ChebOut<float> *co = nullptr, const BcRows<float> *bc = nullptr);
 // Row-split variants (3 waves per brick, one slab of quadrature rows each) for levels with few
 // bricks; one-launch output path only (facebuf required)
 hipError_t launch_a11_fp64_split(const Box &b, const double *coords, const double *u, const uint8_t *mask,
@@ -72,29 +83,35 @@ hipError_t launch_a11_fp32_mfma(const Box &b, const float *u, const uint8_t *mas
                                 bool add, hipStream_t s, float *facebuf, bool gather = true);
 // the face pass alone (adds the face slots of facebuf into their owners; not into the dofs of mask,
 // if given)
-hipError_t launch_gather_faces(const Box &b, const float *face, float *y, hipStream_t s);
-hipError_t launch_gather_faces(const Box &b, const double *face, double *y, hipStream_t s);
+hipError_t launch_gather_faces(const Box &b, const float *face, float *y, hipStream_t s,
+                               const BcRows<float> *bc = nullptr);
+hipError_t launch_gather_faces(const Box &b, const double *face, double *y, hipStream_t s,
+                               const BcRows<double> *bc = nullptr);
 hipError_t launch_build_fac32(const Box &b, const double *coords, const double *eta_bm, float *fac, float *facb,
                               int *err, hipStream_t s);
 hipError_t launch_a11_fp64g(const Box &b, const double *u, const uint8_t *mask, const double *geo, const double *eta_bm,
-                            double *y, bool add, hipStream_t s, double *facebuf = nullptr);
+                            double *y, bool add, hipStream_t s, double *facebuf = nullptr,
+                            const BcRows<double> *bc = nullptr);
 hipError_t launch_build_geo64(const Box &b, const double *coords, double *geo, hipStream_t s);
 hipError_t launch_stokes_fp32(const Box &b, const float *u, const float *p, const uint8_t *mask, const float *fac,
                               const float *facb, float *yu, float *yp, bool add, hipStream_t s,
-                              float *facebuf = nullptr);
+                              float *facebuf = nullptr, const BcRows<float> *bc = nullptr);
 hipError_t launch_eta_to_bm(const Box &b, const double *eta, double *eta_bm, int *err, hipStream_t s);
 // validates the mesh and, if xtile is not null, writes the resident coordinate tiles (Box::xtile)
 hipError_t launch_check_mesh(const Box &b, const double *coords, double *xtile, int *err, hipStream_t s);
 hipError_t launch_a21(const Box &b, const double *coords, const double *u, const uint8_t *mask, double *yp, bool add,
                       hipStream_t s);
 hipError_t launch_a12(const Box &b, const double *coords, const double *p, double *y, bool add, double *facebuf,
-                      hipStream_t s);
+                      hipStream_t s, const BcRows<double> *bc = nullptr);
 hipError_t launch_diag(const Box &b, const double *coords, const double *eta_bm, double *d, bool add, double *facebuf,
-                       hipStream_t s);
+                       hipStream_t s, const BcRows<double> *bc = nullptr);
 // y (+)= the body-force load of fu (3 per quadrature point, element-major)
 // one launch with owner-writes output into facebuf (nbricks * FACEVALS doubles) plus the face pass
 hipError_t launch_body_force(const Box &b, const double *coords, const double *fu, double *y, bool add,
-                             double *facebuf, hipStream_t s, double scale = 1.0);
+                             double *facebuf, hipStream_t s, double scale = 1.0, const BcRows<double> *bc = nullptr);
+// out = u with the Dirichlet values of phi (null: zero) on the mask's dofs
+hipError_t launch_insert_bc(int64_t n, const double *u, const uint8_t *mask, const double *phi, double *out,
+                            hipStream_t s);
 template <typename T>
 hipError_t launch_bc_rows(int64_t n, const int64_t *idx, const T *x, T *y, int mode, hipStream_t s,
                           const T *v = nullptr);

@@ -1379,12 +1379,20 @@ __global__ __launch_bounds__(BEL) void k_diag(Box b, const double *__restrict__ 
 // BCListInsertZero), 1 (mode 2, BCListInsertValueIntoDirichletSlot) or x[idx] - v[idx] with v
 // null meaning 0 (mode 3, BCListResidualDirichlet).
 template <typename T>
-__global__ void k_bc_rows(int64_t n, const int64_t *__restrict__ idx, const T *__restrict__ x, T *__restrict__ y,
-                          int mode, const T *__restrict__ v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int64_t k = idx[i];
-  y[k] = mode == 0 ? x[k] : (mode == 1 ? T(0) : (mode == 2 ? T(1) : x[k] - (v ? v[k] : T(0))));
+__device__ __forceinline__ void bc_row(const BcRows<T> &r, int64_t i, T *__restrict__ y) {
+  if (i >= r.n) return;
+  const int64_t k = r.idx[i];
+  y[k] = r.mode == 0 ? r.x[k] : (r.mode == 1 ? T(0) : (r.mode == 2 ? T(1) : r.x[k] - (r.v ? r.v[k] : T(0))));
+}
+template <typename T>
+__global__ void k_bc_rows(BcRows<T> r, T *__restrict__ y) {
+  bc_row(r, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, y);
+}
+
+__global__ void k_insert_bc(int64_t n, const double *__restrict__ u, const uint8_t *__restrict__ mask,
+                            const double *__restrict__ phi, double *__restrict__ out) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    out[i] = mask[i] ? (phi ? phi[i] : 0.0) : u[i];
 }
 
 // Non-finite scan of an input vector (sets ERRBIT_NONFINITE).
@@ -1493,10 +1501,16 @@ __device__ __forceinline__ void gather_faces_brick(const Box &b, const BrickId &
   }
 }
 
+// The blocks past the bricks write the Dirichlet rows: dofs that no brick's block writes (mask), so the
+// launch of their own, 4-5 us however few they are, goes.
 template <typename T>
 __global__ __launch_bounds__(256) void k_gather_faces(Box b, const T *__restrict__ face, T *__restrict__ y,
-                                                     const uint8_t *__restrict__ mask) {
-  gather_faces_brick(b, brick_xcd(b, blockIdx.x), face, y, mask);
+                                                     const uint8_t *__restrict__ mask, BcRows<T> bc) {
+  const int nb = b.nbx * b.nby * b.nbz;
+  if ((int)blockIdx.x >= nb)
+    bc_row(bc, (int64_t)(blockIdx.x - nb) * 256 + threadIdx.x, y);
+  else
+    gather_faces_brick(b, brick_xcd(b, blockIdx.x), face, y, mask);
 }
 
 template <typename T>
@@ -1508,9 +1522,13 @@ __global__ __launch_bounds__(256) void k_gather_faces_batch(BatchArgs<T> a) {
   gather_faces_brick(b, brick_xcd(b, local), (const T *)a.face[p], a.y[p], a.mode == OUT_BC ? a.mask[p] : nullptr);
 }
 
+// mask: Dirichlet dofs to leave alone; bc: Dirichlet rows to write (and to leave alone)
 template <typename T>
-hipError_t launch_gather(const Box &b, const T *face, T *y, hipStream_t s, const uint8_t *mask = nullptr) {
-  hipLaunchKernelGGL(k_gather_faces<T>, dim3(nbricks(b)), dim3(256), 0, s, b, face, y, mask);
+hipError_t launch_gather(const Box &b, const T *face, T *y, hipStream_t s, const uint8_t *mask,
+                         const BcRows<T> *bc = nullptr) {
+  const BcRows<T> r = bc && bc->n ? *bc : BcRows<T>{};
+  hipLaunchKernelGGL(k_gather_faces<T>, dim3((unsigned)(nbricks(b) + (r.n + 255) / 256)), dim3(256), 0, s, b, face, y,
+                     r.n ? r.mask : mask, r);
   return hipGetLastError();
 }
 
@@ -1527,11 +1545,11 @@ hipError_t launch_a11_fp64(const Box &b, const double *coords, const double *u, 
   return gather ? launch_gather(b, (const double *)facebuf, y, s, mode == OUT_BC ? mask : nullptr) : hipGetLastError();
 }
 
-hipError_t launch_gather_faces(const Box &b, const float *face, float *y, hipStream_t s) {
-  return launch_gather(b, face, y, s);
+hipError_t launch_gather_faces(const Box &b, const float *face, float *y, hipStream_t s, const BcRows<float> *bc) {
+  return launch_gather<float>(b, face, y, s, nullptr, bc);
 }
-hipError_t launch_gather_faces(const Box &b, const double *face, double *y, hipStream_t s) {
-  return launch_gather(b, face, y, s);
+hipError_t launch_gather_faces(const Box &b, const double *face, double *y, hipStream_t s, const BcRows<double> *bc) {
+  return launch_gather<double>(b, face, y, s, nullptr, bc);
 }
 
 hipError_t launch_a11_fp64_split(const Box &b, const double *coords, const double *u, const uint8_t *mask,
@@ -1540,7 +1558,7 @@ hipError_t launch_a11_fp64_split(const Box &b, const double *coords, const doubl
   if (!facebuf) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_a11_fp64_split, dim3(nbricks(b)), dim3(3 * BEL), 0, s, b, coords, u, mask, eta_bm, y,
                      add ? 1 : 0, facebuf);
-  return gather ? launch_gather(b, (const double *)facebuf, y, s) : hipGetLastError();
+  return gather ? launch_gather<double>(b, facebuf, y, s, nullptr) : hipGetLastError();
 }
 
 // Nine waves per brick while every brick gets a CU of its own: 8 bricks 8.2 us against 12.5 us with three
@@ -1554,7 +1572,7 @@ hipError_t launch_a11_fp32_split(const Box &b, const float *u, const uint8_t *ma
     hipLaunchKernelGGL(k_a11_fp32_rows, dim3(nb), dim3(RWAVES * BEL), 0, s, b, u, mask, fac, y, add ? 1 : 0, facebuf);
   else
     hipLaunchKernelGGL(k_a11_fp32_split, dim3(nb), dim3(3 * BEL), 0, s, b, u, mask, fac, y, add ? 1 : 0, facebuf);
-  return gather ? launch_gather(b, (const float *)facebuf, y, s) : hipGetLastError();
+  return gather ? launch_gather<float>(b, facebuf, y, s, nullptr) : hipGetLastError();
 }
 
 bool own_blocks_fit(const Box &b) {
@@ -1588,14 +1606,15 @@ template hipError_t launch_a11_batch<float>(const BatchArgs<float> &, hipStream_
 
 hipError_t launch_stokes_fp64(const Box &b, const double *coords, const double *u, const double *p,
                               const uint8_t *mask, const double *eta_bm, double *yu, double *yp, const double *fp,
-                              bool add, hipStream_t s, double *facebuf) {
+                              bool add, hipStream_t s, double *facebuf, const BcRows<double> *bc) {
   hipLaunchKernelGGL(k_stokes_fp64, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, u, mask, eta_bm, yu, add ? 1 : 0,
                      facebuf, p, yp, fp);
-  return launch_gather(b, (const double *)facebuf, yu, s);
+  return launch_gather<double>(b, facebuf, yu, s, nullptr, bc);
 }
 
 hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, const float *fac, float *y, bool add,
-                           hipStream_t s, float *facebuf, bool gather, const ChebOut<float> *co) {
+                           hipStream_t s, float *facebuf, bool gather, const ChebOut<float> *co,
+                           const BcRows<float> *bc) {
   if (facebuf) {
     if (co) {
       hipLaunchKernelGGL(k_a11_fp32<true>, dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, u, mask, fac, y, 0, facebuf, *co);
@@ -1603,7 +1622,7 @@ hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, co
     }
     hipLaunchKernelGGL(k_a11_fp32<false>, dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, u, mask, fac, y, add ? 1 : 0,
                        facebuf, ChebOut<float>{});
-    return gather ? launch_gather(b, (const float *)facebuf, y, s) : hipGetLastError();
+    return gather ? launch_gather<float>(b, facebuf, y, s, nullptr, bc) : hipGetLastError();
   }
   for (int c = 0; c < 8; c++) {
     int nb = nbricks_color(b, c);
@@ -1611,7 +1630,7 @@ hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, co
     hipLaunchKernelGGL(k_a11_fp32<false>, dim3(nb), dim3(BEL), 0, s, b, c, u, mask, fac, y, add ? 1 : 0,
                        (float *)nullptr, ChebOut<float>{});
   }
-  return hipGetLastError();
+  return bc ? launch_bc_rows<float>(bc->n, bc->idx, bc->x, y, bc->mode, s, bc->v) : hipGetLastError();
 }
 
 hipError_t launch_build_fac32(const Box &b, const double *coords, const double *eta_bm, float *fac, float *facb,
@@ -1621,11 +1640,11 @@ hipError_t launch_build_fac32(const Box &b, const double *coords, const double *
 }
 
 hipError_t launch_a11_fp64g(const Box &b, const double *u, const uint8_t *mask, const double *geo, const double *eta_bm,
-                            double *y, bool add, hipStream_t s, double *facebuf) {
+                            double *y, bool add, hipStream_t s, double *facebuf, const BcRows<double> *bc) {
   if (facebuf) {
     hipLaunchKernelGGL(k_a11_fp64g, dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, u, mask, geo, eta_bm, y, add ? 1 : 0,
                        facebuf);
-    return launch_gather(b, (const double *)facebuf, y, s);
+    return launch_gather<double>(b, facebuf, y, s, nullptr, bc);
   }
   for (int c = 0; c < 8; c++) {
     int nb = nbricks_color(b, c);
@@ -1633,7 +1652,7 @@ hipError_t launch_a11_fp64g(const Box &b, const double *u, const uint8_t *mask, 
     hipLaunchKernelGGL(k_a11_fp64g, dim3(nb), dim3(BEL), 0, s, b, c, u, mask, geo, eta_bm, y, add ? 1 : 0,
                        (double *)nullptr);
   }
-  return hipGetLastError();
+  return bc ? launch_bc_rows<double>(bc->n, bc->idx, bc->x, y, bc->mode, s, bc->v) : hipGetLastError();
 }
 
 hipError_t launch_build_geo64(const Box &b, const double *coords, double *geo, hipStream_t s) {
@@ -1642,11 +1661,12 @@ hipError_t launch_build_geo64(const Box &b, const double *coords, double *geo, h
 }
 
 hipError_t launch_stokes_fp32(const Box &b, const float *u, const float *p, const uint8_t *mask, const float *fac,
-                              const float *facb, float *yu, float *yp, bool add, hipStream_t s, float *facebuf) {
+                              const float *facb, float *yu, float *yp, bool add, hipStream_t s, float *facebuf,
+                              const BcRows<float> *bc) {
   if (facebuf) {
     hipLaunchKernelGGL(k_stokes_fp32, dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, u, p, mask, fac, facb, yu, yp,
                        add ? 1 : 0, facebuf);
-    return launch_gather(b, (const float *)facebuf, yu, s);
+    return launch_gather<float>(b, facebuf, yu, s, nullptr, bc);
   }
   for (int c = 0; c < 8; c++) {
     int nb = nbricks_color(b, c);
@@ -1654,7 +1674,7 @@ hipError_t launch_stokes_fp32(const Box &b, const float *u, const float *p, cons
     hipLaunchKernelGGL(k_stokes_fp32, dim3(nb), dim3(BEL), 0, s, b, c, u, p, mask, fac, facb, yu, yp, add ? 1 : 0,
                        (float *)nullptr);
   }
-  return hipGetLastError();
+  return bc ? launch_bc_rows<float>(bc->n, bc->idx, bc->x, yu, bc->mode, s, bc->v) : hipGetLastError();
 }
 
 hipError_t launch_eta_to_bm(const Box &b, const double *eta, double *eta_bm, int *err, hipStream_t s) {
@@ -1676,28 +1696,36 @@ hipError_t launch_a21(const Box &b, const double *coords, const double *u, const
 }
 
 hipError_t launch_a12(const Box &b, const double *coords, const double *p, double *y, bool add, double *facebuf,
-                      hipStream_t s) {
+                      hipStream_t s, const BcRows<double> *bc) {
   hipLaunchKernelGGL(k_a12, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, p, y, add ? 1 : 0, facebuf);
-  return launch_gather(b, (const double *)facebuf, y, s);
+  return launch_gather<double>(b, facebuf, y, s, nullptr, bc);
 }
 
 hipError_t launch_body_force(const Box &b, const double *coords, const double *fu, double *y, bool add,
-                             double *facebuf, hipStream_t s, double scale) {
+                             double *facebuf, hipStream_t s, double scale, const BcRows<double> *bc) {
   hipLaunchKernelGGL(k_body_force, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, fu, y, add ? 1 : 0, scale, facebuf);
   hipError_t e = hipGetLastError();
-  return e != hipSuccess ? e : launch_gather(b, (const double *)facebuf, y, s);
+  return e != hipSuccess ? e : launch_gather<double>(b, facebuf, y, s, nullptr, bc);
+}
+
+hipError_t launch_insert_bc(int64_t n, const double *u, const uint8_t *mask, const double *phi, double *out,
+                            hipStream_t s) {
+  const int64_t blocks = std::min<int64_t>((n + 255) / 256, 16384);
+  hipLaunchKernelGGL(k_insert_bc, dim3((unsigned)blocks), dim3(256), 0, s, n, u, mask, phi, out);
+  return hipGetLastError();
 }
 
 hipError_t launch_diag(const Box &b, const double *coords, const double *eta_bm, double *d, bool add, double *facebuf,
-                       hipStream_t s) {
+                       hipStream_t s, const BcRows<double> *bc) {
   hipLaunchKernelGGL(k_diag, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, eta_bm, d, add ? 1 : 0, facebuf);
-  return launch_gather(b, (const double *)facebuf, d, s);
+  return launch_gather<double>(b, facebuf, d, s, nullptr, bc);
 }
 
 template <typename T>
 hipError_t launch_bc_rows(int64_t n, const int64_t *idx, const T *x, T *y, int mode, hipStream_t s, const T *v) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_bc_rows<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, idx, x, y, mode, v);
+  hipLaunchKernelGGL(k_bc_rows<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
+                     BcRows<T>{n, idx, nullptr, x, v, mode}, y);
   return hipGetLastError();
 }
 template hipError_t launch_bc_rows<double>(int64_t, const int64_t *, const double *, double *, int, hipStream_t,

@@ -1344,19 +1344,17 @@ hipError_t galerkin_mf(ptq2_mg *mg, int l, const T *x, T *y) {
   return e == hipSuccess ? ptq2::launch_bc_rows<T>(c->ndir, c->dir_idx, x, y, 0, mg->stream) : e;
 }
 
-template <>
-int level_matmult<double>(ptq2_mg *mg, int l, const double *x, double *y) {
+template <typename T>
+int level_matmult(ptq2_mg *mg, int l, const T *x, T *y) {
   ptq2_ctx *c = mg->ctx[l];
-  MGCHK(level_launch(mg, l, x, y, true));
-  MGCHK(ptq2::launch_bc_rows<double>(c->ndir, c->dir_idx, x, y, 0, mg->stream));
-  return PTQ2_OK;
-}
-template <>
-int level_matmult<float>(ptq2_mg *mg, int l, const float *x, float *y) {
-  ptq2_ctx *c = mg->ctx[l];
-  MGCHK(level_launch(mg, l, x, y, true));
-  if (level_own(mg, l)) return PTQ2_OK;
-  MGCHK(ptq2::launch_bc_rows<float>(c->ndir, c->dir_idx, x, y, 0, mg->stream));
+  const bool faces = !mg->gal[l] && c->facebuf;  // the face pass takes the Dirichlet rows along
+  MGCHK(level_launch(mg, l, x, y, !faces));
+  if (sizeof(T) == 4 && level_own(mg, l)) return PTQ2_OK;
+  const ptq2::BcRows<T> bc{c->ndir, c->dir_idx, c->mask, x, nullptr, 0};
+  if (faces)
+    MGCHK(ptq2::launch_gather_faces(mg->lbox[l], (const T *)c->facebuf, y, mg->stream, &bc));
+  else
+    MGCHK(ptq2::launch_bc_rows<T>(c->ndir, c->dir_idx, x, y, 0, mg->stream));
   return PTQ2_OK;
 }
 
