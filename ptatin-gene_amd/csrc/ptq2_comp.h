@@ -255,13 +255,16 @@ __device__ __forceinline__ void dual_to_nodal27(double Y[27]) {
 //   A: for each point 10 values per lane, adjugate (9) and determinant;
 //   G: for each pair (point q, velocity component c != q) the three gradients;
 //   S: for each pair (component c, point q != c) the point's three stresses in component c.
-// A component's values at the point with its own number stay in its wave's registers.
+// A component's values at the point with its own number stay in its wave's registers.  The full block (BLK):
+//   P: for each point the pressure, from the G wave;
+//   T: for each point w (det div u + det fp), to the G wave.
+template <bool BLK>
 struct CompLds {
   static constexpr int NA = 10, SLOT = 3 * BEL;  // doubles
-  static constexpr int A = 0, G = A + 3 * NA * BEL, S = G + 6 * SLOT;
-  static constexpr int ROW = S + 6 * SLOT;
-  static constexpr int PARK = 2 * ROW;           // 27 values of the G wave
-  static constexpr int N = 2 * ROW + 27 * BEL;
+  static constexpr int A = 0, G = A + 3 * NA * BEL, S = G + 6 * SLOT, P = S + 6 * SLOT, T = P + SLOT;
+  static constexpr int ROW = BLK ? T + SLOT : P;
+  static constexpr int PARK = 2 * ROW;  // the G wave's own: 27 values (block: 9)
+  static constexpr int N = 2 * ROW + (BLK ? 9 : 27) * BEL;
   static_assert(2 * 3 * TCS <= 2 * ROW, "the tiles fit the exchange buffers");
   static_assert(3 * TCS <= S, "the output tile fits a row's A and G buffers");
 };
@@ -282,13 +285,74 @@ __device__ __forceinline__ void get3(const double *slot, int lane, double &a, do
 __host__ __device__ constexpr int row_qc(int r) { return r / 3 == 0 ? 1 : (r / 3 == 1 ? 0 : 2); }
 __host__ __device__ constexpr int row_qb(int r) { return r % 3 == 0 ? 0 : (r % 3 == 1 ? 2 : 1); }
 
+// slab 0 -> slab 2 from the nodal layer 2 instead of a: v = m + V2 a - V1 b and d = b - D2 a in slab 0, and
+// u2 = m + (b + a) / 2 gives a (1/2 - V2 + (1/2 + V1) D2) = u2 - v - (1/2 + V1) d
+__device__ __forceinline__ void fold_slab2_layer(double v[18], double u2[9]) {
+  constexpr double e = 0.5 + MOD_V1, f = 1.0 / (0.5 - MOD_V2 + e * MOD_D2);
+  modal_layer(u2);
+#pragma unroll
+  for (int n = 0; n < 9; n++) {
+    const double a = f * fma(-e, v[n + 9], u2[n] - v[n]);
+    const double b = fma(MOD_D2, a, v[n + 9]);
+    v[n] = fma(2.0 * MOD_V1, b, v[n]);
+    v[n + 9] = fma(MOD_D2, a, b);
+  }
+}
+
+// values at a row's three points from its modal x coefficients
+__device__ __forceinline__ void row_values(const double r[3], double v[3]) {
+  const double s = fma(MOD_V2, r[2], r[0]);
+  v[0] = fma(-MOD_V1, r[1], s);
+  v[1] = r[0];
+  v[2] = fma(MOD_V1, r[1], s);
+}
+
 // the G wave
+template <bool BLK>
 struct GWave {
-  using L = CompLds;
+  using L = CompLds<BLK>;
   double x[3][18];  // modal coordinates: values and derivatives along z in the current slab
   // The z direction's third coefficients (layer 0, then a) are needed between the slabs only: they wait
-  // in LDS (all 81 coefficients, beside a row's Jacobians, would spill).
+  // in LDS (all 81 coefficients, beside a row's Jacobians, would spill).  The block needs that LDS for
+  // the pressure; there the coordinates' layer 0 or 2 is read again one row ahead (xg, t).
   double *park;
+  // block: coordinates relative to the pressure basis' centre; park holds the previous row's at its points
+  double t[3][9], avg[3], ps[4], Yp[4], r0[3][3];
+  const double *xg;    // the lane's element: its first coordinate
+  int64_t gy, gz;      // steps to the next node row and plane
+
+  __device__ __forceinline__ void read_layer(int k) {
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+#pragma unroll
+      for (int j = 0; j < 3; j++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) t[c][i + 3 * j] = xg[k * gz + j * gy + 3 * i + c];
+  }
+  // the continuity sums of the row whose points are parked, then park the next row's points
+  template <bool PARK_NEXT>
+  __device__ __forceinline__ void continuity(const double *row, int lane, bool first) {
+    if (!first) {
+      double f[3];
+#pragma unroll
+      for (int q = 0; q < 3; q++) f[q] = row[L::T + q * BEL + lane];
+      Yp[0] += f[0] + f[1] + f[2];
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+#pragma unroll
+        for (int q = 0; q < 3; q++) Yp[1 + c] = fma(f[q], park[(3 * c + q) * BEL + lane], Yp[1 + c]);
+      pin<4>(Yp);
+    }
+    if (PARK_NEXT) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        double v[3];
+        row_values(r0[c], v);
+#pragma unroll
+        for (int q = 0; q < 3; q++) park[(3 * c + q) * BEL + lane] = v[q];
+      }
+    }
+  }
 
   // adjugates and determinants of row R's points
   template <int R>
@@ -296,7 +360,15 @@ struct GWave {
     double Jc[3][3][3];  // [component][d][qa]
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      if (R == 3 || R == 6) {
+      if (BLK && (R == 3 || R == 6)) {
+#pragma unroll
+        for (int n = 0; n < 9; n++) t[c][n] -= avg[c];
+        if (R == 3)
+          fold_slab0(x[c], t[c], t[c]);
+        else
+          fold_slab2_layer(x[c], t[c]);
+        pin<18>(x[c]);
+      } else if (R == 3 || R == 6) {
         double t[9];
 #pragma unroll
         for (int n = 0; n < 9; n++) t[n] = park[(9 * c + n) * BEL + lane];
@@ -309,7 +381,21 @@ struct GWave {
         }
         pin<18>(x[c]);
       }
-      row_grad<row_qb(R)>(x[c], Jc[c]);
+      if constexpr (BLK)
+        row_grad<row_qb(R)>(x[c], Jc[c], r0[c]);
+      else
+        row_grad<row_qb(R)>(x[c], Jc[c]);
+    }
+    if constexpr (BLK) {
+      // the pressure is linear in the coordinates relative to the basis' centre
+      double rp[3], pv[3];
+#pragma unroll
+      for (int i = 0; i < 3; i++) rp[i] = fma(ps[3], r0[2][i], fma(ps[2], r0[1][i], ps[1] * r0[0][i]));
+      rp[0] += ps[0];
+      row_values(rp, pv);
+#pragma unroll
+      for (int q = 0; q < 3; q++) row[L::P + q * BEL + lane] = pv[q];
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int q = 0; q < 3; q++) {
@@ -332,8 +418,12 @@ struct GWave {
   template <int R>
   __device__ __forceinline__ void rows(double *buf, int lane) {
     lds_barrier();
+    if constexpr (BLK) continuity<true>(buf + ((R + 1) & 1) * L::ROW, lane, R == 0);
     if constexpr (R < 8) {
+      row_fence();
       forward<R + 1>(buf + ((R + 1) & 1) * L::ROW, lane);
+      if (BLK && R == 1) read_layer(0);
+      if (BLK && R == 4) read_layer(2);
       row_fence();
       rows<R + 1>(buf, lane);
     }
@@ -341,15 +431,17 @@ struct GWave {
 };
 
 // U wave C: velocity component C, output component C and the stress of point C of every row.
-template <int C>
+template <int C, bool BLK>
 struct UWave {
-  using L = CompLds;
+  using L = CompLds<BLK>;
   double u[27];          // modal velocity component C
   double Y[27];          // dual modal output component C
   double RB[9], RD[9];
   double own[3];         // gradient of component C at the wave's point
   double eta, eta_n;     // viscosity at the wave's point of this row and the next
   const double *ep;      // the brick's viscosities (uniform)
+  const double *fe;      // block: the lane's element's continuity source, or null (uniformly)
+  double pq;             // block: the pressure at the wave's point
 
   __device__ __forceinline__ double load_eta(int r, int lane) const {
     return fast_at(ep + (C + 3 * row_qb(r) + 9 * row_qc(r)) * BEL, (uint32_t)lane);
@@ -387,6 +479,7 @@ struct UWave {
 #pragma unroll
     for (int c = 0; c < 3; c++)
       if (c != C) get3(row + L::G + pair_slot(C, c) * L::SLOT, lane, G[0][c], G[1][c], G[2][c]);
+    if (BLK) pq = row[L::P + C * BEL + lane];
   }
   __device__ __forceinline__ void read_stress(const double *row, int lane) {
 #pragma unroll
@@ -402,7 +495,13 @@ struct UWave {
 #pragma unroll
     for (int d = 0; d < 3; d++) G[d][C] = own[d];
     const double s = (w8 * eta) * rcp64(det);
-    stress_action(A, G, s, dv);
+    if constexpr (BLK) {
+      const double tr = stress_action_p(A, G, s, w8 * pq, dv);
+      // det is 8 times the determinant, the trace 8 times det div u
+      row[L::T + C * BEL + lane] = w8 * (fe ? fma(det, fe[C + 3 * row_qb(R) + 9 * row_qc(R)], tr) : tr);
+    } else {
+      stress_action(A, G, s, dv);
+    }
 #pragma unroll
     for (int c = 0; c < 3; c++) {
       if (c == C) {
@@ -701,23 +800,66 @@ __device__ __forceinline__ void store_tile_full(const Box &b, const BrickId &br,
     store_rows_full<TN>(b, br, t, s, g, face, add_mode, 2 * BE, lane);
 }
 
-__device__ __forceinline__ void g_wave(double *lds, int lane) {
-  using L = CompLds;
-  GWave W;
+// The full block's other operands: pressure, continuity output and source (may be null)
+struct BlockArgs {
+  const double *p, *coords;
+  double *yp;
+  const double *fp;
+};
+
+template <bool BLK>
+__device__ __forceinline__ void g_wave(double *lds, const Box &b, const Tile &t, const BlockArgs &ba, bool active,
+                                       bool add_mode, int lane) {
+  using L = CompLds<BLK>;
+  GWave<BLK> W;
   const int base = lane_base(lane);
   W.park = lds + L::PARK;
   double x[3][27];
+  double inv[3];
+  int64_t e = 0;
+  if constexpr (BLK) {
+    // lanes without an element take another's coordinates; nobody takes their outputs
+    const LaneElem le = lane_elem(lane);
+    W.gy = 3 * (int64_t)b.NX;
+    W.gz = W.gy * b.NY;
+    W.xg = ba.coords + 3 * (t.node0 + 2 * min(le.lx, t.nex - 1)) + 2 * min(le.ly, t.ney - 1) * W.gy +
+           2 * min(le.lz, t.nez - 1) * W.gz;
+    if (active) e = lane_element(b, t, lane);
+#pragma unroll
+    for (int n = 0; n < 4; n++) {
+      W.ps[n] = ba.p[4 * e + n];
+      W.Yp[n] = 0.0;
+    }
+  }
   lds_barrier();  // the tiles are in LDS
 #pragma unroll
   for (int c = 0; c < 3; c++) load_modal(lds, base, c, x[c]);
   lds_barrier();  // every wave has read its tile: the LDS becomes the exchange buffers
+  if constexpr (BLK) {
+    // P3D_ConstructNi_P1GRel_3D (src/element_utils_q2.c:183-224): centre and scale of the basis
+    inv[0] = 1.0 / (x[0][14] - x[0][12]);
+    inv[1] = 1.0 / (x[1][16] - x[1][10]);
+    inv[2] = 1.0 / (x[2][22] - x[2][4]);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      double sum = 0.0;
+#pragma unroll
+      for (int n = 0; n < 27; n++) sum += x[c][n];
+      W.avg[c] = sum * (1.0 / 27.0);
+#pragma unroll
+      for (int n = 0; n < 27; n++) x[c][n] -= W.avg[c];
+      W.ps[1 + c] *= inv[c];
+    }
+  }
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     modal27(x[c]);
 #pragma unroll
     for (int n = 0; n < 18; n++) W.x[c][n] = x[c][n];
+    if constexpr (!BLK) {
 #pragma unroll
-    for (int n = 0; n < 9; n++) W.park[(9 * c + n) * BEL + lane] = x[c][18 + n];
+      for (int n = 0; n < 9; n++) W.park[(9 * c + n) * BEL + lane] = x[c][18 + n];
+    }
   }
   W.template forward<0>(lds, lane);
   row_fence();
@@ -733,15 +875,26 @@ __device__ __forceinline__ void g_wave(double *lds, int lane) {
   for (int n = 0; n < N2 / BEL; n++) z[n * BEL] = zero;
   if (l2 < N2 % BEL) z[N2 / BEL * BEL] = zero;
   lds_barrier();
+  if constexpr (BLK) {
+    W.template continuity<false>(lds, lane, false);
+    if (active) {
+      double *o = ba.yp + 4 * e;
+      const double r[4] = {-W.Yp[0], -W.Yp[1] * inv[0], -W.Yp[2] * inv[1], -W.Yp[3] * inv[2]};
+#pragma unroll
+      for (int i = 0; i < 4; i++) o[i] = add_mode ? o[i] + r[i] : r[i];
+    }
+  }
   lds_barrier();
 }
 
-template <int C>
-__device__ __forceinline__ void u_wave(double *lds, const double *__restrict__ ep, bool active, int lane) {
-  using L = CompLds;
-  UWave<C> W;
+template <int C, bool BLK>
+__device__ __forceinline__ void u_wave(double *lds, const double *__restrict__ ep, const double *fe, bool active,
+                                       int lane) {
+  using L = CompLds<BLK>;
+  UWave<C, BLK> W;
   const int base = lane_base(lane);
   W.ep = ep;
+  W.fe = fe;
   W.eta = W.load_eta(0, lane);
   lds_barrier();
   load_modal(lds + 3 * TCS, base, C, W.u);
@@ -777,12 +930,14 @@ __device__ __forceinline__ void load_tiles4(const Box &b, const BrickId &br, con
 
 // The brick br of box b.  mode: OUT_SET, OUT_ADD or OUT_BC (set, and y = u on the mask's Dirichlet dofs).
 // CH: store with the fused Chebyshev update of co (store_tile_own<true>).
-template <bool CH>
+// BLK: the full block [A11 A12; A21 0] of ba's pressure and continuity output.
+template <bool CH, bool BLK = false>
 __device__ __forceinline__ void a11_fp64_brick(const Box &b, const BrickId &br, const double *__restrict__ coords,
                                                const double *__restrict__ u, const uint8_t *__restrict__ mask,
                                                const double *__restrict__ eta_bm, double *__restrict__ y, int mode,
-                                               double *__restrict__ facebuf, const ChebOut<double> &co) {
-  using L = CompLds;
+                                               double *__restrict__ facebuf, const ChebOut<double> &co,
+                                               const BlockArgs &ba = BlockArgs{}) {
+  using L = CompLds<BLK>;
   __shared__ double2 lds2[L::N / 2];
   double *lds = reinterpret_cast<double *>(lds2);
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / BEL), lane = (int)threadIdx.x - BEL * w;
@@ -796,11 +951,12 @@ __device__ __forceinline__ void a11_fp64_brick(const Box &b, const BrickId &br, 
   else
     load_tiles4<false>(b, br, t, coords, lds, u, mask, lds + 3 * TCS, w, lane);
   const double *ep = eta_bm + (int64_t)br.lin * 27 * BEL;
+  const double *fe = BLK && ba.fp ? ba.fp + 27 * (active ? lane_element(b, t, lane) : 0) : nullptr;
   switch (w) {
-    case 0: u_wave<0>(lds, ep, active, lane); break;
-    case 1: u_wave<1>(lds, ep, active, lane); break;
-    case 2: u_wave<2>(lds, ep, active, lane); break;
-    default: g_wave(lds, lane); break;
+    case 0: u_wave<0, BLK>(lds, ep, fe, active, lane); break;
+    case 1: u_wave<1, BLK>(lds, ep, fe, active, lane); break;
+    case 2: u_wave<2, BLK>(lds, ep, fe, active, lane); break;
+    default: g_wave<BLK>(lds, b, t, ba, active, mode == OUT_ADD, lane); break;
   }
   const double *Ys = lds + L::ROW;
   const ChebOut<double> *cp = CH ? &co : nullptr;

@@ -770,8 +770,6 @@ __device__ __forceinline__ double rcp64(double x) {
   e = fma(-x, r, 1.0);
   return fma(r, e, r);
 }
-__device__ __forceinline__ float rcp32(float x) { return 1.0f / x; }
-
 // Stress action at one quadrature point.  With M[k][l] = sum_m g[m][l] A[k][m]
 // (= det * du_l/dx_k) and S = s (M + M^T), s = w eta / det, the test-function
 // coefficient is dv[k][l] = sum_m S[m][l] A[m][k]; this equals w det J^-T (2 eta eps(u))
@@ -835,29 +833,12 @@ __device__ __forceinline__ void acc_row(const T dv[3][3], T P0[3][3], T P1[3][3]
     }
 }
 
-// x- and y-transpose of one quadrature point's dv straight into the slab
-// accumulators (no per-row accumulator kept live):
-//   RB[c][j][i] += B(qb,j) D(qa,i) dv[0][c] + D(qb,j) B(qa,i) dv[1][c]
-//   RD[c][j][i] += B(qb,j) B(qa,i) dv[2][c]
-template <int qa, int qb, typename T>
-__device__ __forceinline__ void acc_direct(const T dv[3][3], T RB[3][3][3], T RD[3][3][3]) {
-#pragma unroll
-  for (int c = 0; c < 3; c++)
-#pragma unroll
-    for (int j = 0; j < 3; j++)
-#pragma unroll
-      for (int i = 0; i < 3; i++) {
-        if (nzB(qb, j) && nzD(qa, i)) RB[c][j][i] = fmac(gB(qb, j) * gD(qa, i), dv[0][c], RB[c][j][i]);
-        if (nzD(qb, j) && nzB(qa, i)) RB[c][j][i] = fmac(gD(qb, j) * gB(qa, i), dv[1][c], RB[c][j][i]);
-        if (nzB(qb, j) && nzB(qa, i)) RD[c][j][i] = fmac(gB(qb, j) * gB(qa, i), dv[2][c], RD[c][j][i]);
-      }
-}
-
 // ---------------------------------------------------------------------------
 // Runtime-row variants.  The quadrature row (qb,qc) is a runtime (wave-uniform) loop
 // index; its 1D coefficients come from constant memory into scalar registers, so the
 // whole element body is one row-sized block of code (a fully unrolled element does
 // not fit the instruction cache).  Inside a row everything is unrolled.
+// keeps the scheduler from hoisting the next row's LDS reads into this one
 __device__ __forceinline__ void row_fence() { __builtin_amdgcn_sched_barrier(0); }
 
 // Asynchronous copy of NB contiguous bytes (a multiple of 16) from global memory into
@@ -906,8 +887,6 @@ __constant__ const double c_gB[3][3] = {
 __constant__ const double c_gD[3][3] = {{-0.77459666924148337704 - 0.5, 2.0 * 0.77459666924148337704, -0.77459666924148337704 + 0.5},
                                          {-0.5, 0.0, 0.5},
                                          {0.77459666924148337704 - 0.5, -2.0 * 0.77459666924148337704, 0.77459666924148337704 + 0.5}};
-__constant__ const double c_gw[3] = {5.0 / 9.0, 8.0 / 9.0, 5.0 / 9.0};
-
 __device__ __forceinline__ Coef1 coef1(int q) {
   Coef1 r;
 #pragma unroll
@@ -978,55 +957,6 @@ __device__ __forceinline__ void acc_row_elem_rt(const Coef1 &cb, const Coef1 &cc
 #pragma unroll
         for (int k = 0; k < 3; k++) Y[c][k][j][i] = fmac(cc.b[k], tb, fmac(cc.d[k], td, Y[c][k][j][i]));
       }
-}
-
-// Slab form of the y/z transposes: the rows of one slab (fixed qc) accumulate their y-transposed
-// pairs into RB (B-weighted in z) and RD (D-weighted), and acc_slab_rt spreads the slab over the
-// three z nodes once:  RB[c][j][i] += B(qb,j) P0 + D(qb,j) P1,  RD += B(qb,j) P2, then
-// Y[c][k][j][i] += B(qc,k) RB + D(qc,k) RD.  81 + 54 / 3 operations per row and output instead
-// of 243 per row.
-template <typename T>
-__device__ __forceinline__ void acc_row_slab_rt(const Coef1 &cb, const T P0[3][3], const T P1[3][3],
-                                                const T P2[3][3], T RB[3][3][3], T RD[3][3][3]) {
-#pragma unroll
-  for (int c = 0; c < 3; c++)
-#pragma unroll
-    for (int j = 0; j < 3; j++)
-#pragma unroll
-      for (int i = 0; i < 3; i++) {
-        RB[c][j][i] = fmac(cb.b[j], P0[c][i], fmac(cb.d[j], P1[c][i], RB[c][j][i]));
-        RD[c][j][i] = fmac(cb.b[j], P2[c][i], RD[c][j][i]);
-      }
-}
-template <typename T>
-__device__ __forceinline__ void acc_slab_rt(const Coef1 &cc, const T RB[3][3][3], const T RD[3][3][3],
-                                            T Y[3][3][3][3]) {
-#pragma unroll
-  for (int c = 0; c < 3; c++)
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-#pragma unroll
-      for (int j = 0; j < 3; j++)
-#pragma unroll
-        for (int i = 0; i < 3; i++) Y[c][k][j][i] = fmac(cc.b[k], RB[c][j][i], fmac(cc.d[k], RD[c][j][i], Y[c][k][j][i]));
-}
-
-// keep the scheduler from hoisting the next row's LDS reads into this one
-
-// z-transpose of a finished slab into the element output Y[c][k][j][i]
-template <int qc, typename T>
-__device__ __forceinline__ void acc_elem(const T RB[3][3][3], const T RD[3][3][3], T Y[3][3][3][3]) {
-#pragma unroll
-  for (int c = 0; c < 3; c++)
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-#pragma unroll
-      for (int j = 0; j < 3; j++)
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-          if (nzB(qc, k)) Y[c][k][j][i] = fmac(gB(qc, k), RB[c][j][i], Y[c][k][j][i]);
-          if (nzD(qc, k)) Y[c][k][j][i] = fmac(gD(qc, k), RD[c][j][i], Y[c][k][j][i]);
-        }
 }
 
 template <typename T>

@@ -66,9 +66,6 @@ hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, co
                            const ChebOut<float> *co = nullptr, const BcRows<float> *bc = nullptr);
 // Row-split variants (3 waves per brick, one slab of quadrature rows each) for levels with few
 // bricks; one-launch output path only (facebuf required)
-hipError_t launch_a11_fp64_split(const Box &b, const double *coords, const double *u, const uint8_t *mask,
-                                 const double *eta_bm, double *y, bool add, hipStream_t s, double *facebuf,
-                                 bool gather = true);
 // The FP32 apply in overlapping blocks (nine waves each), complete in one launch: y = A x with y = x on the mask's
 // dofs or, with co, its Chebyshev update (co->mask is mask, co->x is x; y unused, and out is none of the
 // inputs).  For boxes without ghost layers whose blocks get a CU each (own_blocks_fit).

@@ -42,107 +42,6 @@ __device__ __forceinline__ PBasis pbasis_setup(const double *Xs, int base) {
 
 // ----------------------------------------------------------------- A11 FP64
 
-// geometry of quadrature point qa of the current row: adjugate and s = w eta / det
-template <int qa>
-__device__ __forceinline__ double geo_qp(const double xr0[3][3], const double xr1[3][3], const double xr2[3][3],
-                                         double wbc, double eta, double A[3][3], double &s) {
-  double J[3][3];
-  qp_grad<qa>(xr0, xr1, xr2, J);
-  double det = adjugate(J, A);
-  s = (gw1(qa) * wbc * eta) * rcp64(det);
-  return det;
-}
-
-// Pressure-side state of the full block (BLK): the element's P1GRel basis set-up and
-// pressure, the continuity accumulators and, for the residual (fp != nullptr), the 27
-// quadrature values of the continuity source.
-struct BlockState {
-  PBasis pb;
-  double pe[4];
-  double Yp[4];
-  const double *fp;
-};
-
-// pressure basis values N^p_1..3 at quadrature point qa of the row (x from the B-B row data)
-template <int qa>
-__device__ __forceinline__ void pbasis_qp(const double xr0[3][3], const PBasis &pb, double np[3]) {
-  double x[3];
-  qp_value<qa>(xr0, x);
-#pragma unroll
-  for (int d = 0; d < 3; d++) np[d] = (x[d] - pb.avg[d]) * pb.inv[d];
-}
-
-// one quadrature point of the velocity phase
-template <int qa, bool BLK>
-__device__ __forceinline__ void a11_qp64(const double ur0[3][3], const double ur1[3][3], const double ur2[3][3],
-                                         const double A[3][3], double s, double wbc, const double np[3],
-                                         double wdet, int q, BlockState *bs, double P0[3][3], double P1[3][3],
-                                         double P2[3][3]) {
-  double g[3][3], dv[3][3];
-  qp_grad<qa>(ur0, ur1, ur2, g);
-  if constexpr (BLK) {
-    const double w = gw1(qa) * wbc;
-    const double pq = bs->pe[0] + bs->pe[1] * np[0] + bs->pe[2] * np[1] + bs->pe[3] * np[2];
-    const double f = -w * stress_action_p(A, g, s, w * pq, dv);
-    double fs = 0.0;
-    if (bs->fp) fs = -wdet * bs->fp[q];
-    bs->Yp[0] += f + fs;
-#pragma unroll
-    for (int d = 0; d < 3; d++) bs->Yp[1 + d] += (f + fs) * np[d];
-  } else {
-    stress_action(A, g, s, dv);
-  }
-  acc_row<qa>(dv, P0, P1, P2);
-}
-
-// one quadrature row (runtime qb,qc) of the FP64 A11 element: geometry of its three
-// points from the coordinate tile, velocity gradients from the velocity tile, the
-// stress action and the x-transpose into P, then the y- and z-transposes into Y.
-// On entry ca holds column 0 of the coordinate tile; on exit it holds it again (for
-// the next row), its reads in flight behind the stress work.  BLK adds the pressure and
-// continuity terms of the full block.
-template <bool BLK, bool SLAB = false>
-__device__ __forceinline__ void a11_row64(const double *Xs, const double *Us, int base, const Coef1 &cb,
-                                          const Coef1 &cc, double wbc, const double e3[3], double ca[9],
-                                          double cb9[9], double Y[3][3][3][3], int row, BlockState *bs,
-                                          double (*RB)[3][3] = nullptr, double (*RD)[3][3] = nullptr) {
-  double A0[3][3], A1[3][3], A2[3][3], s0, s1, s2;
-  double np[3][3], wd[3] = {0.0, 0.0, 0.0};
-  {
-    double xr0[3][3], xr1[3][3], xr2[3][3];
-    row_data_pipe(Xs, Us, base, cb, cc, ca, cb9, xr0, xr1, xr2);
-    const double d0 = geo_qp<0>(xr0, xr1, xr2, wbc, e3[0], A0, s0);
-    const double d1 = geo_qp<1>(xr0, xr1, xr2, wbc, e3[1], A1, s1);
-    const double d2 = geo_qp<2>(xr0, xr1, xr2, wbc, e3[2], A2, s2);
-    if constexpr (BLK) {
-      pbasis_qp<0>(xr0, bs->pb, np[0]);
-      pbasis_qp<1>(xr0, bs->pb, np[1]);
-      pbasis_qp<2>(xr0, bs->pb, np[2]);
-      if (bs->fp) {
-        wd[0] = gw1(0) * wbc * d0;
-        wd[1] = gw1(1) * wbc * d1;
-        wd[2] = gw1(2) * wbc * d2;
-      }
-    } else {
-      (void)d0; (void)d1; (void)d2;
-    }
-  }
-  row_fence();
-  double ur0[3][3], ur1[3][3], ur2[3][3];
-  row_data_pipe(Us, Xs, base, cb, cc, cb9, ca, ur0, ur1, ur2);
-  double P0[3][3], P1[3][3], P2[3][3];
-  zero33(P0); zero33(P1); zero33(P2);
-  a11_qp64<0, BLK>(ur0, ur1, ur2, A0, s0, wbc, np[0], wd[0], 3 * row, bs, P0, P1, P2);
-  a11_qp64<1, BLK>(ur0, ur1, ur2, A1, s1, wbc, np[1], wd[1], 3 * row + 1, bs, P0, P1, P2);
-  a11_qp64<2, BLK>(ur0, ur1, ur2, A2, s2, wbc, np[2], wd[2], 3 * row + 2, bs, P0, P1, P2);
-  row_fence();
-  if constexpr (SLAB)
-    acc_row_slab_rt(cb, P0, P1, P2, RB, RD);
-  else
-    acc_row_elem_rt(cb, cc, P0, P1, P2, Y);
-  row_fence();
-}
-
 // add the element's 81 outputs into the LDS output tile (of the element's type or wider)
 template <typename S, typename T>
 __device__ __forceinline__ void emit_element(S *Ys, int base, const T Y[3][3][3][3]) {
@@ -156,77 +55,21 @@ __device__ __forceinline__ void emit_element(S *Ys, int base, const T Y[3][3][3]
         for (int i = 0; i < 3; i++) lds_add(&Ys[base + toff(c, i, j, k)], S(Y[c][k][j][i]));
 }
 
-__device__ __forceinline__ void load3(const double *__restrict__ ep, int row, double *e3) {
-#pragma unroll
-  for (int q = 0; q < 3; q++) e3[q] = ep[(3 * row + q) * BEL];
-}
-
-// The full block [A11 A12; A21 0] in one element pass, one wave per brick
+// The full block [A11 A12; A21 0] in one element pass on the four waves of ptq2_comp.h
 // (MFStokesWrapper_A_AVX, src/stokes_operators_avx.c:439-636): yu gets A11 u + A12 p, yp gets A21 u
 // (and, with fp, minus the continuity source: FormFunctionLocal_P's -int N^p fp,
-// src/stokes_form_function.c:478-580).
-__global__ __launch_bounds__(BEL) void k_stokes_fp64(Box b, const double *__restrict__ coords,
-                                                     const double *__restrict__ u, const uint8_t *__restrict__ mask,
-                                                     const double *__restrict__ eta_bm, double *__restrict__ y,
-                                                     int add_mode, double *__restrict__ facebuf,
-                                                     const double *__restrict__ p, double *__restrict__ yp,
-                                                     const double *__restrict__ fp) {
-  constexpr bool BLK = true;
-  const BrickId br = brick_xcd(b, blockIdx.x);
-  __shared__ double Xs[3 * TCS];
-  __shared__ double Us[3 * TCS];
-  const int lane = threadIdx.x;
-  const Tile t = tile_of(b, br);
-  const double *ep = eta_bm + (int64_t)br.lin * 27 * BEL + lane;
-  double en[3];
-  load3(ep, 0, en);
-  load_tile2(b, t, br, coords, Xs, u, mask, Us, lane);
-  __syncthreads();
-  const int base = lane_base(lane);
-  const bool active = lane_active(t, lane);
-  double Y[3][3][3][3];
-#pragma unroll
-  for (int c = 0; c < 3; c++)
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-#pragma unroll
-      for (int j = 0; j < 3; j++)
-#pragma unroll
-        for (int i = 0; i < 3; i++) Y[c][k][j][i] = 0.0;
-  BlockState bs;
-  int64_t e = 0;
-  {
-    bs.Yp[0] = bs.Yp[1] = bs.Yp[2] = bs.Yp[3] = 0.0;
-    bs.pe[0] = bs.pe[1] = bs.pe[2] = bs.pe[3] = 0.0;
-    bs.fp = nullptr;
-    if (active) {
-      e = lane_element(b, t, lane);
-      bs.pb = pbasis_setup(Xs, base);
-#pragma unroll
-      for (int i = 0; i < 4; i++) bs.pe[i] = p[4 * e + i];
-      if (fp) bs.fp = fp + 27 * e;
-    }
-  }
-  if (active) {
-    double ca[9], cb9[9];
-    ld_col(Xs, base, 0, ca);
-#pragma nounroll
-    for (int row = 0; row < 9; row++) {
-      const int qb = row % 3, qc = row / 3;
-      double e3[3] = {en[0], en[1], en[2]};
-      if (row < 8) load3(ep, row + 1, en);
-      a11_row64<BLK>(Xs, Us, base, coef1(qb), coef1(qc), c_gw[qb] * c_gw[qc], e3, ca, cb9, Y, row, &bs);
-    }
-    double *o = yp + 4 * e;
-#pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = add_mode ? o[i] + bs.Yp[i] : bs.Yp[i];
-  }
-  __syncthreads();
-  zero_tile(Xs, lane);
-  __syncthreads();
-  if (active) emit_element(Xs, base, Y);
-  __syncthreads();
-  store_tile_own(b, br, t, Xs, y, facebuf, add_mode != 0, lane);
+// src/stokes_form_function.c:478-580).  The G wave interpolates the pressure, whose basis is linear in the
+// coordinates it has, and takes each point's divergence back; the U waves add one term to the stress.  Bound as
+// the A11 pass is (256 VGPRs, 78 KB of LDS).  64^3: 151 us against 205 us with one wave per brick and nodal tables;
+// 48^3: 69 us against 107 us.
+__global__ __launch_bounds__(CWAVES * BEL, 2) void k_stokes_fp64(Box b, const double *__restrict__ coords,
+                                                                const double *__restrict__ u,
+                                                                const uint8_t *__restrict__ mask,
+                                                                const double *__restrict__ eta_bm,
+                                                                double *__restrict__ y, int mode,
+                                                                double *__restrict__ facebuf, BlockArgs ba) {
+  a11_fp64_brick<false, true>(b, brick_xcd(b, blockIdx.x), coords, u, mask, eta_bm, y, mode, facebuf,
+                              ChebOut<double>{}, ba);
 }
 
 template <bool CH>
@@ -430,63 +273,6 @@ __global__ __launch_bounds__(BEL) void k_a11_fp32_batch(BatchArgs<float> a) {
 // another order than the one-wave kernels' (rounding differs in the last bits).  One-launch
 // output path only (facebuf).
 __device__ __forceinline__ int split_wave() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x / BEL); }
-
-__global__ __launch_bounds__(3 * BEL) void k_a11_fp64_split(Box b, const double *__restrict__ coords,
-                                                            const double *__restrict__ u,
-                                                            const uint8_t *__restrict__ mask,
-                                                            const double *__restrict__ eta_bm, double *__restrict__ y,
-                                                            int add_mode, double *__restrict__ facebuf) {
-  __shared__ double Xs[3 * TCS];
-  __shared__ double Us[3 * TCS];
-  const int w = split_wave(), lane = (int)threadIdx.x - BEL * w;
-  const BrickId br = brick_xcd(b, blockIdx.x);
-  const Tile t = tile_of(b, br);
-  const double *ep = eta_bm + (int64_t)br.lin * 27 * BEL + lane;
-  double en[3];
-  load3(ep, 3 * w, en);
-  if (w == 0) load_tile2(b, t, br, coords, Xs, u, mask, Us, lane);
-  __syncthreads();
-  const int base = lane_base(lane);
-  const bool active = lane_active(t, lane);
-  double Y[3][3][3][3];
-#pragma unroll
-  for (int c = 0; c < 3; c++)
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-#pragma unroll
-      for (int j = 0; j < 3; j++)
-#pragma unroll
-        for (int i = 0; i < 3; i++) Y[c][k][j][i] = 0.0;
-  BlockState bs;
-  if (active) {
-    double ca[9], cb9[9], RB[3][3][3], RD[3][3][3];
-#pragma unroll
-    for (int c = 0; c < 3; c++)
-#pragma unroll
-      for (int j = 0; j < 3; j++)
-#pragma unroll
-        for (int i = 0; i < 3; i++) RB[c][j][i] = RD[c][j][i] = 0.0;
-    ld_col(Xs, base, 0, ca);
-#pragma nounroll
-    for (int row = 3 * w; row < 3 * w + 3; row++) {
-      const int qb = row % 3;
-      double e3[3] = {en[0], en[1], en[2]};
-      if (row + 1 < 3 * w + 3) load3(ep, row + 1, en);
-      a11_row64<false, true>(Xs, Us, base, coef1(qb), coef1(w), c_gw[qb] * c_gw[w], e3, ca, cb9, Y, row, &bs, RB,
-                             RD);
-    }
-    acc_slab_rt(coef1(w), RB, RD, Y);  // the wave's slab (qc = w) into its outputs
-  }
-  __syncthreads();
-  if (w == 0) zero_tile(Xs, lane);
-  __syncthreads();
-  for (int k = 0; k < 3; k++) {
-    if (w == k && active) emit_element(Xs, base, Y);
-    __syncthreads();
-  }
-  store_tile_own<false, WSTEPS>(b, br, t, Xs, y, facebuf, add_mode != 0, lane, (const ChebOut<double> *)nullptr,
-                                WPLANES * w);
-}
 
 __global__ __launch_bounds__(3 * BEL) void k_a11_fp32_split(Box b, const float *__restrict__ u,
                                                             const uint8_t *__restrict__ mask,
@@ -995,13 +781,6 @@ __device__ __forceinline__ void to_row_slab(const double *s, int base, int c, do
   }
 }
 
-// values at a row's three points from its modal x coefficients
-__device__ __forceinline__ void row_values(const double r[3], double v[3]) {
-  const double s = fma(MOD_V2, r[2], r[0]);
-  v[0] = fma(-MOD_V1, r[1], s);
-  v[1] = r[0];
-  v[2] = fma(MOD_V1, r[1], s);
-}
 template <int R, int Q>
 constexpr double w8() {
   return gw1(Q) * gw1(row_qb(R)) * gw1(row_qc(R)) * 0.125;
@@ -1552,15 +1331,6 @@ hipError_t launch_gather_faces(const Box &b, const double *face, double *y, hipS
   return launch_gather<double>(b, face, y, s, nullptr, bc);
 }
 
-hipError_t launch_a11_fp64_split(const Box &b, const double *coords, const double *u, const uint8_t *mask,
-                                 const double *eta_bm, double *y, bool add, hipStream_t s, double *facebuf,
-                                 bool gather) {
-  if (!facebuf) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_a11_fp64_split, dim3(nbricks(b)), dim3(3 * BEL), 0, s, b, coords, u, mask, eta_bm, y,
-                     add ? 1 : 0, facebuf);
-  return gather ? launch_gather<double>(b, facebuf, y, s, nullptr) : hipGetLastError();
-}
-
 // Nine waves per brick while every brick gets a CU of its own: 8 bricks 8.2 us against 12.5 us with three
 // waves, 48 bricks 8.0 against 10.6.  Beyond, the SIMD that runs three of a brick's nine waves is what
 // a CU waits for: 384 bricks take 16.7 us, 13.8 us with three waves.
@@ -1607,8 +1377,8 @@ template hipError_t launch_a11_batch<float>(const BatchArgs<float> &, hipStream_
 hipError_t launch_stokes_fp64(const Box &b, const double *coords, const double *u, const double *p,
                               const uint8_t *mask, const double *eta_bm, double *yu, double *yp, const double *fp,
                               bool add, hipStream_t s, double *facebuf, const BcRows<double> *bc) {
-  hipLaunchKernelGGL(k_stokes_fp64, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, u, mask, eta_bm, yu, add ? 1 : 0,
-                     facebuf, p, yp, fp);
+  hipLaunchKernelGGL(k_stokes_fp64, dim3(nbricks(b)), dim3(CWAVES * BEL), 0, s, b, coords, u, mask, eta_bm, yu,
+                     (int)(add ? OUT_ADD : OUT_SET), facebuf, BlockArgs{p, coords, yp, fp});
   return launch_gather<double>(b, facebuf, yu, s, nullptr, bc);
 }
 

@@ -1195,8 +1195,8 @@ struct DevBuf {
 
 // launch shape of a level's smoother apply, picked at set-up by timing (autotune)
 struct LevelTune {
-  int split = 0;              // kernel: 0 one wave per brick, 1 row-split (3 or 9 waves per brick),
-                              // 2 matrix-core form (FP32 smoothing only)
+  int split = 0;              // FP32 kernel: 0 one wave per brick, 1 row-split (3 or 9 waves per
+                              // brick), 2 matrix-core form; FP64 has one kernel
   int fast = 0;               // tile addressing of full tiles: 1 = 32-bit fast path, 0 = general
   double ms = 0.0, ms_default = 0.0;  // measured time per apply: chosen shape, default shape
 };
@@ -1300,9 +1300,6 @@ hipError_t level_launch(ptq2_mg *mg, int l, const double *x, double *y, bool gat
   // geometry recomputed from the coordinates (the faster FP64 kernel); the level's face
   // buffer was allocated by its set-up applies (no allocation here: this runs under graph
   // capture)
-  if (mg->tune[l].split == 1 && !mg->f32)
-    return ptq2::launch_a11_fp64_split(b, c->coords, x, c->mask, c->eta_bm, y, false, mg->stream,
-                                       (double *)c->facebuf, gather);
   return ptq2::launch_a11_fp64(b, c->coords, x, c->mask, c->eta_bm, y, ptq2::OUT_SET, mg->stream,
                                (double *)c->facebuf, gather);
 }
@@ -1625,7 +1622,7 @@ int autotune(ptq2_mg *mg) {
     const int reps = (int)std::min(50.0, std::max(2.0, 2.0 / std::max(t0, 1e-3)));  // ~2 ms per batch
     double best = 1e30;
     int bs = 0, bf = c->box.fast32;
-    const int kinds = sizeof(T) == 4 ? 3 : 2;
+    const int kinds = sizeof(T) == 4 ? 3 : 1;  // FP64 has one kernel, on four waves per brick
     for (int split = 0; split < kinds; split++)
       for (int fast = c->box.fast32; fast >= 0; fast--) {
         t.split = split;

@@ -139,3 +139,40 @@ def test_row_split_smoother(dims):
         S.destroy()
         ctx.destroy()
     assert (torch.linalg.norm(z[1] - z[0]) / torch.linalg.norm(z[0])).item() <= 1e-5
+
+
+@pytest.mark.parametrize("dims", EDGES)
+def test_full_block_and_residual(dims):
+    """The full block (set, ADD, MatMult) and the residual with a continuity source, on bricks of all
+    fillings, against the oracle at the operators' bar; parts of the residual by superposition."""
+    print("case: full block", dims, flush=True)
+    P = problem(dims)
+    ne = int(np.prod(dims))
+    A = ptq2.MatA11MF("hip")
+    A.setup(P)
+    u, p = M.uniform(3, P.nvel, -1.0, 1.0), M.uniform(4, 4 * ne, -1.0, 1.0)
+    ud, pd = torch.from_numpy(u).to(DEV), torch.from_numpy(p).to(DEV)
+    ru, rp = O.stokes_a(*dims, P.coords, P.eta, u, p)
+    yu, yp = A.ctx.stokes(ud, pd)
+    assert rel(yu.cpu().numpy(), ru) <= 1e-12 and rel(yp.cpu().numpy(), rp) <= 1e-12
+    au, ap = A.ctx.stokes(ud, pd, torch.full_like(yu, 0.5), torch.full_like(yp, 0.5), _lib.ADD)
+    assert rel(au.cpu().numpy(), ru + 0.5) <= 1e-12 and rel(ap.cpu().numpy(), rp + 0.5) <= 1e-12
+    d = P.mask > 0
+    um = np.where(d, 0.0, u)
+    mu, mp = A.ctx.stokes(ud, pd, flags=_lib.MATMULT)
+    ru, rp = O.stokes_a(*dims, P.coords, P.eta, um, p)
+    assert rel(mu.cpu().numpy(), np.where(d, u, ru)) <= 1e-12 and rel(mp.cpu().numpy(), rp) <= 1e-12
+    fu, phi = M.uniform(7, 81 * ne, -1.0, 1.0), M.uniform(8, P.nvel, -1.0, 1.0)
+    fp = M.uniform(9, 27 * ne, -1.0, 1.0)
+    dev = lambda a: torch.from_numpy(a).to(DEV)
+    Fu, Fp = A.ctx.residual(ud, pd, dev(fu), dev(fp), dev(phi))
+    ul = np.where(d, phi, u)
+    ru, rp = O.stokes_a(*dims, P.coords, P.eta, ul, p)
+    ru -= O.body_force(*dims, P.coords, fu)
+    assert rel(Fu.cpu().numpy(), np.where(d, u - phi, ru)) <= 1e-12
+    # the source alone: fp = 1 integrates the pressure basis
+    z, zp = torch.zeros_like(ud), torch.zeros_like(pd)
+    F1 = A.ctx.residual(z, zp, dev(0.0 * fu), dev(fp), dev(0.0 * phi))[1]
+    F0 = A.ctx.residual(ud, pd, dev(fu), None, dev(phi))[1]
+    assert rel(F0.cpu().numpy(), rp) <= 1e-12
+    assert rel((F0 + F1).cpu().numpy(), Fp.cpu().numpy()) <= 1e-12
