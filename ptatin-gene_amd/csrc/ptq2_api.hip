@@ -864,10 +864,10 @@ int ptq2_stokes_residual(ptq2_ctx *c, const double *u, const double *p, const do
   if (rc) return rc;
   // Fu = A11 u_loc + A12 p, Fp = A21 u_loc - int N^p fp (one element pass), then Fu -= Be
   HIPCHK(c, ptq2::launch_stokes_fp64(c->box, c->coords, ul, dp, nullptr, c->eta_bm, dFu, dFp, dfp, false, c->stream,
-                                     (double *)fb));
+                                     (double *)fb, nullptr, false));
   // Dirichlet rows: Fu_D = u_D - phi_D (BCListResidualDirichlet, src/dmda_bcs.c:614-648)
   const auto bc = bc_of(c, true, 3, du, dphi);
-  HIPCHK(c, ptq2::launch_body_force(c->box, c->coords, dfu, dFu, true, (double *)fb, c->stream, -1.0, &bc));
+  HIPCHK(c, ptq2::launch_body_force(c->box, c->coords, dfu, dFu, true, (double *)fb, c->stream, -1.0, &bc, true));
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(Fu, dFu, sizeof(double) * (size_t)nv, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipMemcpyAsync(Fp, dFp, sizeof(double) * (size_t)np, hipMemcpyDeviceToHost, c->stream));

@@ -463,7 +463,8 @@ __host__ __device__ __forceinline__ T cheb_update(const ChebOut<T> &co, int64_t 
 // One store per row pair and no branches: a lane's base is y or, in a last column that a neighbour owns,
 // the X plane, and the row's offset from it is added.  A third of the instructions of a loop that
 // decides node by node, which a wave alone on its SIMD waits for one by one.
-template <int ROWS, typename S, typename T>
+// ALL: add to the face slots too (what an earlier pass left there for the same face pass).
+template <int ROWS, bool ALL = false, typename S, typename T>
 __device__ __forceinline__ void store_rows_full(const Box &b, const BrickId &br, const Tile &t,
                                                 const S *__restrict__ s, T *__restrict__ g, T *__restrict__ face,
                                                 bool add_mode, int z0, int lane) {
@@ -477,7 +478,7 @@ __device__ __forceinline__ void store_rows_full(const Box &b, const BrickId &br,
   T val[STEPS];
 #pragma unroll
   for (int it = 0; it < STEPS; it++) val[it] = T(s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)]);
-  if (add_mode && ownz) {
+  if (!ALL && add_mode && ownz) {
     T old[STEPS];
 #pragma unroll
     for (int it = 0; it < STEPS; it++) old[it] = fast_at(gb, fast_eoff<E>(b, L, it));
@@ -495,6 +496,7 @@ __device__ __forceinline__ void store_rows_full(const Box &b, const BrickId &br,
   char *base = reinterpret_cast<char *>(ownx ? gb : fo + 3 * TN * z0 + L.c);
   T *bz = ownx ? fo + 3 * TN * 2 * TN + L.col : fo + 3 * TN * z0 + L.c;
   constexpr uint32_t SZ = sizeof(T);
+  T *to[STEPS];
 #pragma unroll
   for (int it = 0; it < STEPS; it++) {
     const int r0 = 2 * it;                                                // the even lanes' row of the group
@@ -508,7 +510,17 @@ __device__ __forceinline__ void store_rows_full(const Box &b, const BrickId &br,
       const bool toy = ownx && (top0 ? odd == 0 : odd == 1);
       at = toy ? by + 3 * TN * ((top0 ? r0 : r0 + 1) / TN) : at;
     }
-    if (2 * it + 1 < ROWS || odd == 0) *at = val[it];
+    to[it] = at;
+    if (!ALL && (2 * it + 1 < ROWS || odd == 0)) *at = val[it];
+  }
+  if constexpr (ALL) {
+    T old[STEPS];
+#pragma unroll
+    for (int it = 0; it < STEPS; it++)
+      if (2 * it + 1 < ROWS || odd == 0) old[it] = *to[it];
+#pragma unroll
+    for (int it = 0; it < STEPS; it++)
+      if (2 * it + 1 < ROWS || odd == 0) *to[it] = old[it] + val[it];
   }
 }
 
@@ -575,7 +587,8 @@ __device__ __forceinline__ void store_tile_cheb_fast(const Box &b, const BrickId
 // CH: the Chebyshev update of co is applied to every owned node that is final here (see
 // store_tile_cheb_fast); the others are stored into g for the face pass.
 // STEPS row pairs from plane z0: the whole tile, or one wave's third of it.
-template <bool CH = false, int STEPS = TPAIRS, typename S, typename T>
+// ALL: with add_mode, the face slots are added to as well.
+template <bool CH = false, int STEPS = TPAIRS, bool ALL = false, typename S, typename T>
 __device__ __forceinline__ void store_tile_own(const Box &b, const BrickId &br, const Tile &t, const S *__restrict__ s,
                                                T *__restrict__ g, T *__restrict__ face, bool add_mode, int lane,
                                                const ChebOut<T> *co = nullptr, int z0 = 0) {
@@ -584,8 +597,8 @@ __device__ __forceinline__ void store_tile_own(const Box &b, const BrickId &br, 
     if constexpr (CH) {
       store_tile_cheb_fast(b, br, t, s, g, face, lane, co);
     } else if (STEPS == TPAIRS) {
-      store_rows_full<2 * BE * TN>(b, br, t, s, g, face, add_mode, 0, lane);
-      store_rows_full<TN>(b, br, t, s, g, face, add_mode, 2 * BE, lane);
+      store_rows_full<2 * BE * TN, ALL>(b, br, t, s, g, face, add_mode, 0, lane);
+      store_rows_full<TN, ALL>(b, br, t, s, g, face, add_mode, 2 * BE, lane);
     } else if (z0 < 2 * WPLANES) {
       store_rows_full<WPLANES * TN>(b, br, t, s, g, face, add_mode, z0, lane);
     } else {
@@ -634,7 +647,7 @@ __device__ __forceinline__ void store_tile_own(const Box &b, const BrickId &br, 
       }
     } else {
       const int slot = !ownx ? z * TN + y : (!owny ? TN * TN + z * TN + ii : 2 * TN * TN + y * TN + ii);
-      fo[3 * slot] = T(val);
+      fo[3 * slot] = ALL ? T(fo[3 * slot] + val) : T(val);
     }
   }
 }
@@ -844,7 +857,9 @@ __device__ __forceinline__ void row_fence() { __builtin_amdgcn_sched_barrier(0);
 // Asynchronous copy of NB contiguous bytes (a multiple of 16) from global memory into
 // LDS with global->LDS loads: lane l moves bytes [16l, 16l+16) of every 1 KiB chunk, and
 // no vector register is held while the copy is in flight.  Every lane of the wave must
-// take part.  Completion: s_waitcnt vmcnt(0) (WAIT_VM0).
+// take part.  Completion: s_waitcnt vmcnt(0) (WAIT_VM0).  AUX_NT: data that one brick reads once, which
+// leaves the caches to what neighbours share (nodal vectors, face slots).
+constexpr int AUX_NT = 2;
 template <typename T>
 __device__ __forceinline__ const T *uniform_ptr(const T *p) {
   const uint64_t v = (uint64_t)p;
@@ -852,7 +867,7 @@ __device__ __forceinline__ const T *uniform_ptr(const T *p) {
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
   return (const T *)(((uint64_t)hi << 32) | lo);
 }
-template <int NB>
+template <int NB, int AUX = 0>
 __device__ __forceinline__ void lds_copy_async(const void *src, void *lds, int lane) {
   static_assert(NB % 16 == 0, "16-byte chunks");
   constexpr int CH = NB / 16, FULL = CH / 64, REM = CH % 64;
@@ -865,11 +880,11 @@ __device__ __forceinline__ void lds_copy_async(const void *src, void *lds, int l
 #pragma unroll
   for (int i = 0; i < FULL; i++)
     __builtin_amdgcn_global_load_lds((const void *)(s0 + i * 1024 + off),
-                                     (__attribute__((address_space(3))) void *)(d0 + i * 1024), 16, 0, 0);
+                                     (__attribute__((address_space(3))) void *)(d0 + i * 1024), 16, 0, AUX);
   if (REM) {
     if (lane < REM)
       __builtin_amdgcn_global_load_lds((const void *)(s0 + FULL * 1024 + off),
-                                       (__attribute__((address_space(3))) void *)(d0 + FULL * 1024), 16, 0, 0);
+                                       (__attribute__((address_space(3))) void *)(d0 + FULL * 1024), 16, 0, AUX);
   }
 }
 // s_waitcnt immediates (gfx9 encoding): all vector-memory operations done (the

@@ -60,7 +60,8 @@ hipError_t launch_a11_fp64(const Box &b, const double *coords, const double *u, 
 // subtracts the continuity source from yp
 hipError_t launch_stokes_fp64(const Box &b, const double *coords, const double *u, const double *p,
                               const uint8_t *mask, const double *eta_bm, double *yu, double *yp, const double *fp,
-                              bool add, hipStream_t s, double *facebuf, const BcRows<double> *bc = nullptr);
+                              bool add, hipStream_t s, double *facebuf, const BcRows<double> *bc = nullptr,
+                              bool gather = true);
 hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, const float *fac, float *y, bool add,
                            hipStream_t s, float *facebuf = nullptr, bool gather = true,
                            const ChebOut<float> *co = nullptr, const BcRows<float> *bc = nullptr);
@@ -103,9 +104,11 @@ hipError_t launch_a12(const Box &b, const double *coords, const double *p, doubl
 hipError_t launch_diag(const Box &b, const double *coords, const double *eta_bm, double *d, bool add, double *facebuf,
                        hipStream_t s, const BcRows<double> *bc = nullptr);
 // y (+)= the body-force load of fu (3 per quadrature point, element-major)
-// one launch with owner-writes output into facebuf (nbricks * FACEVALS doubles) plus the face pass
+// one launch with owner-writes output into facebuf (nbricks * FACEVALS doubles) plus the face pass; pending:
+// facebuf and y hold an apply whose face pass is still to run, and this one adds to both
 hipError_t launch_body_force(const Box &b, const double *coords, const double *fu, double *y, bool add,
-                             double *facebuf, hipStream_t s, double scale = 1.0, const BcRows<double> *bc = nullptr);
+                             double *facebuf, hipStream_t s, double scale = 1.0, const BcRows<double> *bc = nullptr,
+                             bool pending = false);
 // out = u with the Dirichlet values of phi (null: zero) on the mask's dofs
 hipError_t launch_insert_bc(int64_t n, const double *u, const uint8_t *mask, const double *phi, double *out,
                             hipStream_t s);

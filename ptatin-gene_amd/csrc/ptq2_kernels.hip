@@ -105,7 +105,8 @@ __global__ __launch_bounds__(CWAVES * BEL, 2) void k_a11_fp64_batch(BatchArgs<do
 // Geometric factors are precomputed in FP64 (k_build_fac32) and stored rounded
 // to FP32 as F = sqrt(w eta / det) * adj(J), 9 per quadrature point, brick-major
 // [brick][q][m][lane] so that every load instruction is one contiguous 256-byte
-// segment.  Then dv = F^T (M + M^T) with M = F g (diagonal doubled), all FP32.
+// segment.  Each is read once per apply, non-temporally (80^3 apply 180 -> 169 us, full block of 140k
+// elements 80 -> 73 us).  Then dv = F^T (M + M^T) with M = F g (diagonal doubled), all FP32.
 
 // one quadrature point of the FP32 A11 row: F = sqrt(w eta / det) adj(J) (9 floats)
 template <int qa>
@@ -178,7 +179,7 @@ __device__ __forceinline__ void fp32_rows(const float *Us, float *Fs, const floa
     for (int n = 0; n < 18; n++) F12[n] = Fs[(9 + n) * BEL + lane];
     if (row + 1 < row1) {
       __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
-      lds_copy_async<FROW * 4>(fsrc + (row + 1) * FROW, Fs, lane);
+      lds_copy_async<FROW * 4, AUX_NT>(fsrc + (row + 1) * FROW, Fs, lane);
     }
     if (qb == 0) slab_z32(Us, base, cc, ZB, ZD);
     float ur0[3][3], ur1[3][3], ur2[3][3];
@@ -216,7 +217,7 @@ __device__ __forceinline__ void a11_fp32_brick(const Box &b, const BrickId &br, 
   const int lane = threadIdx.x;
   const Tile t = tile_of(b, br);
   const float *fsrc = fac + (int64_t)br.lin * 243 * BEL;
-  lds_copy_async<FROW * 4>(fsrc, Fs, lane);
+  lds_copy_async<FROW * 4, AUX_NT>(fsrc, Fs, lane);
   load_tile(b, t, br, u, mask, Us, lane);
   __syncthreads();
   const int base = lane_base(lane);
@@ -285,7 +286,7 @@ __global__ __launch_bounds__(3 * BEL) void k_a11_fp32_split(Box b, const float *
   const BrickId br = brick_xcd(b, blockIdx.x);
   const Tile t = tile_of(b, br);
   const float *fsrc = fac + (int64_t)br.lin * 243 * BEL;
-  lds_copy_async<FROW * 4>(fsrc + 3 * w * FROW, Fs[w], lane);
+  lds_copy_async<FROW * 4, AUX_NT>(fsrc + 3 * w * FROW, Fs[w], lane);
   if (w == 0) load_tile(b, t, br, u, mask, Us, lane);
   if (w == 1) zero_tile(Ts, lane);
   __syncthreads();
@@ -512,8 +513,8 @@ __global__ __launch_bounds__(BEL) void k_stokes_fp32(Box b, int color, const flo
   const Tile t = tile_of(b, br);
   const float *fsrc = fac + (int64_t)br.lin * 243 * BEL;
   const float *bsrc = facb + (int64_t)br.lin * 108 * BEL;
-  lds_copy_async<FROW * 4>(fsrc, Fs, lane);
-  lds_copy_async<BROW * 4>(bsrc, Bs, lane);
+  lds_copy_async<FROW * 4, AUX_NT>(fsrc, Fs, lane);
+  lds_copy_async<BROW * 4, AUX_NT>(bsrc, Bs, lane);
   load_tile(b, t, br, u, mask, Us, lane);
   __syncthreads();
   const int base = lane_base(lane);
@@ -570,8 +571,8 @@ __global__ __launch_bounds__(BEL) void k_stokes_fp32(Box b, int color, const flo
       }
       if (row < 8) {
         __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
-        lds_copy_async<FROW * 4>(fsrc + (row + 1) * FROW, Fs, lane);
-        lds_copy_async<BROW * 4>(bsrc + (row + 1) * BROW, Bs, lane);
+        lds_copy_async<FROW * 4, AUX_NT>(fsrc + (row + 1) * FROW, Fs, lane);
+        lds_copy_async<BROW * 4, AUX_NT>(bsrc + (row + 1) * BROW, Bs, lane);
       }
       row_fence();
       acc_row_elem_rt(cb, cc, P0, P1, P2, Y);
@@ -1020,6 +1021,8 @@ __device__ __forceinline__ void bf_slab(double *Ys, int base, const double r[27]
   }
 }
 
+// ALL: the load is added to y and to the face slots of the pass before it, whose face pass serves both.
+template <bool ALL>
 __global__ __launch_bounds__(BEL) void k_body_force(Box b, const double *__restrict__ coords,
                                                     const double *__restrict__ fu, double *__restrict__ y,
                                                     int add_mode, double sc, double *__restrict__ facebuf) {
@@ -1051,7 +1054,8 @@ __global__ __launch_bounds__(BEL) void k_body_force(Box b, const double *__restr
   if (active) bf_slab<1>(Xs, base, r1, wd);
   if (active) bf_slab<2>(Xs, base, r0, wd);
   __syncthreads();
-  store_tile_own(b, br, t, Xs, y, facebuf, add_mode != 0, lane);
+  store_tile_own<false, TPAIRS, ALL>(b, br, t, Xs, y, facebuf, add_mode != 0, lane,
+                                     (const ChebOut<double> *)nullptr);
 }
 
 // ---------------------------------------------------------------- diagonal
@@ -1376,10 +1380,10 @@ template hipError_t launch_a11_batch<float>(const BatchArgs<float> &, hipStream_
 
 hipError_t launch_stokes_fp64(const Box &b, const double *coords, const double *u, const double *p,
                               const uint8_t *mask, const double *eta_bm, double *yu, double *yp, const double *fp,
-                              bool add, hipStream_t s, double *facebuf, const BcRows<double> *bc) {
+                              bool add, hipStream_t s, double *facebuf, const BcRows<double> *bc, bool gather) {
   hipLaunchKernelGGL(k_stokes_fp64, dim3(nbricks(b)), dim3(CWAVES * BEL), 0, s, b, coords, u, mask, eta_bm, yu,
                      (int)(add ? OUT_ADD : OUT_SET), facebuf, BlockArgs{p, coords, yp, fp});
-  return launch_gather<double>(b, facebuf, yu, s, nullptr, bc);
+  return gather ? launch_gather<double>(b, facebuf, yu, s, nullptr, bc) : hipGetLastError();
 }
 
 hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, const float *fac, float *y, bool add,
@@ -1472,8 +1476,12 @@ hipError_t launch_a12(const Box &b, const double *coords, const double *p, doubl
 }
 
 hipError_t launch_body_force(const Box &b, const double *coords, const double *fu, double *y, bool add,
-                             double *facebuf, hipStream_t s, double scale, const BcRows<double> *bc) {
-  hipLaunchKernelGGL(k_body_force, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, fu, y, add ? 1 : 0, scale, facebuf);
+                             double *facebuf, hipStream_t s, double scale, const BcRows<double> *bc, bool pending) {
+  if (pending)
+    hipLaunchKernelGGL(k_body_force<true>, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, fu, y, 1, scale, facebuf);
+  else
+    hipLaunchKernelGGL(k_body_force<false>, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, fu, y, add ? 1 : 0, scale,
+                       facebuf);
   hipError_t e = hipGetLastError();
   return e != hipSuccess ? e : launch_gather<double>(b, facebuf, y, s, nullptr, bc);
 }
