@@ -105,8 +105,11 @@ __global__ __launch_bounds__(CWAVES * BEL, 2) void k_a11_fp64_batch(BatchArgs<do
 // Geometric factors are precomputed in FP64 (k_build_fac32) and stored rounded
 // to FP32 as F = sqrt(w eta / det) * adj(J), 9 per quadrature point, brick-major
 // [brick][q][m][lane] so that every load instruction is one contiguous 256-byte
-// segment.  Each is read once per apply, non-temporally (80^3 apply 180 -> 169 us, full block of 140k
-// elements 80 -> 73 us).  Then dv = F^T (M + M^T) with M = F g (diagonal doubled), all FP32.
+// segment.  Each is read once per apply: where they alone fill most of the 256 MB cache (FAC_NT),
+// non-temporally (80^3 apply 180 -> 169 us, full block of 140k elements 80 -> 73 us, 64^3 86 -> 84 and
+// 108 -> 95 us); below, the next apply finds part of them there (56^3 apply 62 against 64 us, 48^3
+// block 43 against 45 us non-temporally).  Then dv = F^T (M + M^T) with M = F g (diagonal doubled), all
+// FP32.
 
 // one quadrature point of the FP32 A11 row: F = sqrt(w eta / det) adj(J) (9 floats)
 template <int qa>
@@ -164,6 +167,7 @@ constexpr int FROW = 27 * BEL;
 // Quadrature rows row0 .. row1-1 of the FP32 element, accumulated into Y.  On entry the factors
 // of row0 are on their way into Fs (lds_copy_async from fsrc + row0 * FROW); each row's
 // successor is copied in while it computes.  row0 starts a slab (row0 % 3 == 0).
+template <int AUX>
 __device__ __forceinline__ void fp32_rows(const float *Us, float *Fs, const float *fsrc, int base, int lane, int row0,
                                           int row1, float Y[3][3][3][3]) {
   float ZB[3][3][3], ZD[3][3][3];
@@ -179,7 +183,7 @@ __device__ __forceinline__ void fp32_rows(const float *Us, float *Fs, const floa
     for (int n = 0; n < 18; n++) F12[n] = Fs[(9 + n) * BEL + lane];
     if (row + 1 < row1) {
       __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
-      lds_copy_async<FROW * 4, AUX_NT>(fsrc + (row + 1) * FROW, Fs, lane);
+      lds_copy_async<FROW * 4, AUX>(fsrc + (row + 1) * FROW, Fs, lane);
     }
     if (qb == 0) slab_z32(Us, base, cc, ZB, ZD);
     float ur0[3][3], ur1[3][3], ur2[3][3];
@@ -202,7 +206,10 @@ __device__ __forceinline__ void fp32_rows(const float *Us, float *Fs, const floa
   }
 }
 
-template <bool CH>
+constexpr int64_t FAC_NT = 200000000;  // bytes
+inline bool factors_nt(int64_t nb, int values) { return nb * values * BEL * (int64_t)sizeof(float) >= FAC_NT; }
+
+template <bool CH, int AUX>
 __device__ __forceinline__ void a11_fp32_brick(const Box &b, const BrickId &br, int color, const float *__restrict__ u,
                                                const uint8_t *__restrict__ mask, const float *__restrict__ fac,
                                                float *__restrict__ y, int add_mode, float *__restrict__ facebuf,
@@ -217,7 +224,7 @@ __device__ __forceinline__ void a11_fp32_brick(const Box &b, const BrickId &br, 
   const int lane = threadIdx.x;
   const Tile t = tile_of(b, br);
   const float *fsrc = fac + (int64_t)br.lin * 243 * BEL;
-  lds_copy_async<FROW * 4, AUX_NT>(fsrc, Fs, lane);
+  lds_copy_async<FROW * 4, AUX>(fsrc, Fs, lane);
   load_tile(b, t, br, u, mask, Us, lane);
   __syncthreads();
   const int base = lane_base(lane);
@@ -234,7 +241,7 @@ __device__ __forceinline__ void a11_fp32_brick(const Box &b, const BrickId &br, 
   // Row r+1's factors travel HBM -> LDS while row r computes.  Every lane runs the rows
   // (the copies need the whole wave); the inactive lanes of a partial brick compute on
   // tile and factor slots that no element owns and their outputs are discarded.
-  fp32_rows(Us, Fs, fsrc, base, lane, 0, 9, Y);
+  fp32_rows<AUX>(Us, Fs, fsrc, base, lane, 0, 9, Y);
   __syncthreads();
   zero_tile(Ts, lane);
   __syncthreads();
@@ -248,21 +255,22 @@ __device__ __forceinline__ void a11_fp32_brick(const Box &b, const BrickId &br, 
     store_tile_own(b, br, t, Ts, y, facebuf, add_mode != 0, lane);
 }
 
-template <bool CH>
+template <bool CH, int AUX>
 __global__ __launch_bounds__(BEL) void k_a11_fp32(Box b, int color, const float *__restrict__ u,
                                                   const uint8_t *__restrict__ mask, const float *__restrict__ fac,
                                                   float *__restrict__ y, int add_mode, float *__restrict__ facebuf,
                                                   ChebOut<float> co) {
   const BrickId br = color >= 0 ? brick_of(b, color, blockIdx.x) : brick_xcd(b, blockIdx.x);
-  a11_fp32_brick<CH>(b, br, color, u, mask, fac, y, add_mode, facebuf, co);
+  a11_fp32_brick<CH, AUX>(b, br, color, u, mask, fac, y, add_mode, facebuf, co);
 }
 
+template <int AUX>
 __global__ __launch_bounds__(BEL) void k_a11_fp32_batch(BatchArgs<float> a) {
   const int p = batch_problem(a.start, a.n, blockIdx.x);
   const Box b = a.box[p];
   const int local = (int)blockIdx.x - a.start[p];
   if (local >= b.nbx * b.nby * b.nbz) return;
-  a11_fp32_brick<false>(b, brick_xcd(b, local), -1, a.u[p], a.mask[p], a.fac[p], a.y[p], a.mode == OUT_ADD, a.face[p],
+  a11_fp32_brick<false, AUX>(b, brick_xcd(b, local), -1, a.u[p], a.mask[p], a.fac[p], a.y[p], a.mode == OUT_ADD, a.face[p],
                         ChebOut<float>{});
 }
 
@@ -286,7 +294,7 @@ __global__ __launch_bounds__(3 * BEL) void k_a11_fp32_split(Box b, const float *
   const BrickId br = brick_xcd(b, blockIdx.x);
   const Tile t = tile_of(b, br);
   const float *fsrc = fac + (int64_t)br.lin * 243 * BEL;
-  lds_copy_async<FROW * 4, AUX_NT>(fsrc + 3 * w * FROW, Fs[w], lane);
+  lds_copy_async<FROW * 4>(fsrc + 3 * w * FROW, Fs[w], lane);
   if (w == 0) load_tile(b, t, br, u, mask, Us, lane);
   if (w == 1) zero_tile(Ts, lane);
   __syncthreads();
@@ -301,7 +309,7 @@ __global__ __launch_bounds__(3 * BEL) void k_a11_fp32_split(Box b, const float *
       for (int j = 0; j < 3; j++)
 #pragma unroll
         for (int i = 0; i < 3; i++) Y[c][k][j][i] = 0.0f;
-  fp32_rows(Us, Fs[w], fsrc, base, lane, 3 * w, 3 * w + 3, Y);
+  fp32_rows<0>(Us, Fs[w], fsrc, base, lane, 3 * w, 3 * w + 3, Y);
   __syncthreads();
   for (int k = 0; k < 3; k++) {
     if (w == k && active) emit_element(Ts, base, Y);
@@ -495,6 +503,7 @@ __device__ __forceinline__ void stokes_qp32(const float ur0[3][3], const float u
   acc_row<qa>(dv, P0, P1, P2);
 }
 
+template <int AUX>
 __global__ __launch_bounds__(BEL) void k_stokes_fp32(Box b, int color, const float *__restrict__ u,
                                                      const float *__restrict__ p, const uint8_t *__restrict__ mask,
                                                      const float *__restrict__ fac, const float *__restrict__ facb,
@@ -513,8 +522,8 @@ __global__ __launch_bounds__(BEL) void k_stokes_fp32(Box b, int color, const flo
   const Tile t = tile_of(b, br);
   const float *fsrc = fac + (int64_t)br.lin * 243 * BEL;
   const float *bsrc = facb + (int64_t)br.lin * 108 * BEL;
-  lds_copy_async<FROW * 4, AUX_NT>(fsrc, Fs, lane);
-  lds_copy_async<BROW * 4, AUX_NT>(bsrc, Bs, lane);
+  lds_copy_async<FROW * 4, AUX>(fsrc, Fs, lane);
+  lds_copy_async<BROW * 4, AUX>(bsrc, Bs, lane);
   load_tile(b, t, br, u, mask, Us, lane);
   __syncthreads();
   const int base = lane_base(lane);
@@ -571,8 +580,8 @@ __global__ __launch_bounds__(BEL) void k_stokes_fp32(Box b, int color, const flo
       }
       if (row < 8) {
         __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
-        lds_copy_async<FROW * 4, AUX_NT>(fsrc + (row + 1) * FROW, Fs, lane);
-        lds_copy_async<BROW * 4, AUX_NT>(bsrc + (row + 1) * BROW, Bs, lane);
+        lds_copy_async<FROW * 4, AUX>(fsrc + (row + 1) * FROW, Fs, lane);
+        lds_copy_async<BROW * 4, AUX>(bsrc + (row + 1) * BROW, Bs, lane);
       }
       row_fence();
       acc_row_elem_rt(cb, cc, P0, P1, P2, Y);
@@ -1369,7 +1378,8 @@ hipError_t launch_a11_batch(const BatchArgs<T> &a, hipStream_t s) {
   if constexpr (sizeof(T) == 8)
     hipLaunchKernelGGL(k_a11_fp64_batch, dim3(nb), dim3(CWAVES * BEL), 0, s, a);
   else
-    hipLaunchKernelGGL(k_a11_fp32_batch, dim3(nb), dim3(BEL), 0, s, a);
+    hipLaunchKernelGGL(factors_nt(nb, 243) ? k_a11_fp32_batch<AUX_NT> : k_a11_fp32_batch<0>, dim3(nb), dim3(BEL), 0, s,
+                       a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_gather_faces_batch<T>, dim3(nb), dim3(256), 0, s, a);
@@ -1389,19 +1399,22 @@ hipError_t launch_stokes_fp64(const Box &b, const double *coords, const double *
 hipError_t launch_a11_fp32(const Box &b, const float *u, const uint8_t *mask, const float *fac, float *y, bool add,
                            hipStream_t s, float *facebuf, bool gather, const ChebOut<float> *co,
                            const BcRows<float> *bc) {
+  const bool nt = factors_nt(nbricks(b), 243);
   if (facebuf) {
     if (co) {
-      hipLaunchKernelGGL(k_a11_fp32<true>, dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, u, mask, fac, y, 0, facebuf, *co);
+      hipLaunchKernelGGL((nt ? k_a11_fp32<true, AUX_NT> : k_a11_fp32<true, 0>), dim3(nbricks(b)), dim3(BEL), 0, s, b,
+                         -1, u, mask, fac, y, 0, facebuf, *co);
       return hipGetLastError();
     }
-    hipLaunchKernelGGL(k_a11_fp32<false>, dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, u, mask, fac, y, add ? 1 : 0,
+    hipLaunchKernelGGL((nt ? k_a11_fp32<false, AUX_NT> : k_a11_fp32<false, 0>), dim3(nbricks(b)), dim3(BEL), 0, s, b,
+                       -1, u, mask, fac, y, add ? 1 : 0,
                        facebuf, ChebOut<float>{});
     return gather ? launch_gather<float>(b, facebuf, y, s, nullptr, bc) : hipGetLastError();
   }
   for (int c = 0; c < 8; c++) {
     int nb = nbricks_color(b, c);
     if (nb == 0) continue;
-    hipLaunchKernelGGL(k_a11_fp32<false>, dim3(nb), dim3(BEL), 0, s, b, c, u, mask, fac, y, add ? 1 : 0,
+    hipLaunchKernelGGL((k_a11_fp32<false, 0>), dim3(nb), dim3(BEL), 0, s, b, c, u, mask, fac, y, add ? 1 : 0,
                        (float *)nullptr, ChebOut<float>{});
   }
   return bc ? launch_bc_rows<float>(bc->n, bc->idx, bc->x, y, bc->mode, s, bc->v) : hipGetLastError();
@@ -1438,14 +1451,15 @@ hipError_t launch_stokes_fp32(const Box &b, const float *u, const float *p, cons
                               const float *facb, float *yu, float *yp, bool add, hipStream_t s, float *facebuf,
                               const BcRows<float> *bc) {
   if (facebuf) {
-    hipLaunchKernelGGL(k_stokes_fp32, dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, u, p, mask, fac, facb, yu, yp,
+    hipLaunchKernelGGL(factors_nt(nbricks(b), 351) ? k_stokes_fp32<AUX_NT> : k_stokes_fp32<0>, dim3(nbricks(b)),
+                       dim3(BEL), 0, s, b, -1, u, p, mask, fac, facb, yu, yp,
                        add ? 1 : 0, facebuf);
     return launch_gather<float>(b, facebuf, yu, s, nullptr, bc);
   }
   for (int c = 0; c < 8; c++) {
     int nb = nbricks_color(b, c);
     if (nb == 0) continue;
-    hipLaunchKernelGGL(k_stokes_fp32, dim3(nb), dim3(BEL), 0, s, b, c, u, p, mask, fac, facb, yu, yp, add ? 1 : 0,
+    hipLaunchKernelGGL(k_stokes_fp32<0>, dim3(nb), dim3(BEL), 0, s, b, c, u, p, mask, fac, facb, yu, yp, add ? 1 : 0,
                        (float *)nullptr);
   }
   return bc ? launch_bc_rows<float>(bc->n, bc->idx, bc->x, yu, bc->mode, s, bc->v) : hipGetLastError();
