@@ -61,8 +61,8 @@ typedef struct {
      of 0 (default): the apply storing A x, then one update pass over all dofs */
   int fused_smoother;
   /* 1 (default): at set-up, time each kernel of every level's smoother apply
-     (PTQ2_MG_KERNEL_*: one wave per brick of 4x4x4 elements; three waves per brick, each
-     running a slab of quadrature rows; with FP32 smoothing, the matrix-core form) with fast
+     (PTQ2_MG_KERNEL_*; FP32: one wave per brick of 4x4x4 elements, the row-split form, the
+     matrix-core form; FP64 has one kernel, on four waves per brick) with fast
      or general tile addressing where every tile is full, and keep the fastest
      (ptq2_mg_tuning reports the choice).  The kernels sum in different orders, so two
      hierarchies whose choices differ round differently in the last bits.  0: one wave per
@@ -128,8 +128,8 @@ int ptq2_mg_rigid_info(const ptq2_mg *mg, int *ninclusions, int *ncolumns, int32
 int ptq2_mg_eigs(const ptq2_mg *mg, double *emin, double *emax);
 /* Kernels of the smoother apply (ptq2_mg_tuning) */
 enum {
-  PTQ2_MG_KERNEL_BRICK = 0,       /* one wave per brick of 4x4x4 elements */
-  PTQ2_MG_KERNEL_SPLIT = 1,       /* three waves per brick, one slab of quadrature rows each */
+  PTQ2_MG_KERNEL_BRICK = 0,       /* FP32: one wave per brick of 4x4x4 elements; FP64 */
+  PTQ2_MG_KERNEL_SPLIT = 1,       /* FP32: three or (up to 256 bricks) nine waves per brick */
   PTQ2_MG_KERNEL_MFMA = 2,        /* the FP32 operator's matrix-core form */
   PTQ2_MG_KERNEL_STENCIL = 3,     /* Galerkin level: its assembled 5x5x5 block stencil */
   PTQ2_MG_KERNEL_GALERKIN_MF = 4  /* Galerkin level: R A P through the matrix-free level above */

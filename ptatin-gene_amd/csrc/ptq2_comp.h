@@ -1,4 +1,4 @@
-// ptq2_comp.h -- the FP64 A11 element pass on four waves per brick.
+// ptq2_comp.h -- the FP64 A11 (and full-block) element pass on four waves per brick.
 //
 // Four waves share a brick of 4x4x4 elements (lane = element, as everywhere): U wave c (0, 1, 2) owns
 // component c of the velocity and of the output, the G wave the geometry.  Per quadrature row (three
@@ -21,14 +21,13 @@
 // The 1D contractions work on (m, b, a) = (u1, u2 - u0, u0 - 2 u1 + u2) instead of the nodal
 // values: with x = sqrt(3/5), u(+-x) = m + 0.3 a +- (x/2) b, u(0) = m, 2 u'(+-x) = b +- 2 x a and
 // 2 u'(0) = b, 5 operations for three values and three derivatives against 14 with the nodal
-// tables.  An element takes ~6.1k VALU instructions, the one-wave form with nodal tables 12.9k.
-//  All derivatives carry the factor 2; it is taken out in the point weights (w / 8:
+// tables.  A brick takes 6.4k VALU instructions, the one-wave form with nodal tables 12.9k.  All derivatives carry the factor 2; it is taken out in the point weights (w / 8:
 // J' = 2 J, adj(J') = 4 adj(J), det J' = 8 det J, and the transposed derivative applies 2 again).
 //
 // What bounds it: a workgroup's chain of load, nine rows with a barrier each, output and store takes
 // 21k cycles alone and 33k beside a second workgroup (a row 1.3k and 1.8k, of which ~0.6k are VALU),
-// and two workgroups fit a CU (212 VGPRs, 81 KB of LDS).  128^3 elements: 1117 us per apply (955 us this
-// pass, 158 us the face pass; loads and stores alone 547 us), 1300-1330 us with the one-wave kernel;
+// and two workgroups fit a CU (212 VGPRs, 81 KB of LDS).  128^3 elements: 1020-1110 us per apply by mesh
+// (158 us of it the face pass; this pass' loads and stores alone 547 us), 1300-1330 us with the one-wave kernel;
 // 8^3 (one brick's latency): 17 us against 39 us; 37x22x45: 36 us against 48 us.
 #pragma once
 #include "ptq2_device.h"

@@ -1,7 +1,8 @@
 // ptq2_device.h -- device-side building blocks shared by the operator kernels.
 //
-// Work decomposition (MI355X, gfx950): one 64-lane wavefront owns a brick of
-// 4x4x4 Q2 elements, lane = element.  The brick's 9x9x9 node tile of
+// Work decomposition (MI355X, gfx950): a brick is 4x4x4 Q2 elements, lane =
+// element.  One 64-lane wavefront owns it here; ptq2_comp.h and ptq2_rows.h share
+// it among waves.  The brick's 9x9x9 node tile of
 // coordinates and velocity is staged once in LDS with row-contiguous global
 // loads; every lane then runs the whole sum-factorized element computation in
 // registers (no cross-lane traffic), accumulates its 81 outputs into an LDS
