@@ -92,6 +92,15 @@ ptq2::BcRows<T> bc_of(const ptq2_ctx *c, bool mm, int mode, const T *x = nullptr
   return ptq2::BcRows<T>{mm ? c->ndir : 0, c->dir_idx, c->mask, x, v, mode};
 }
 
+// face slots of A12 and the diagonal for a call on the context's present stream, or null: coloured launches
+double *face2_of(ptq2_ctx *c) {
+  if (!c->face2_used) {
+    c->face2_used = true;
+    c->face2_stream = c->stream;
+  }
+  return c->stream == c->face2_stream ? (double *)c->facebuf2 : nullptr;
+}
+
 int ensure(ptq2_ctx *c, void **buf, size_t *have, size_t need) {
   if (*have >= need) return PTQ2_OK;
   dev_free(*buf);
@@ -338,7 +347,8 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   dev_free(c->pwork);
   c->coords = nullptr; c->mask = nullptr; c->dir_idx = nullptr; c->eta_bm = nullptr;
   c->xtile = nullptr; c->bdir = nullptr;
-  c->fac32 = nullptr; c->facb32 = nullptr; c->geo64 = nullptr; c->facebuf = c->facebuf_own = nullptr;
+  c->fac32 = nullptr; c->facb32 = nullptr; c->geo64 = nullptr; c->facebuf = c->facebuf_own = c->facebuf2 = nullptr;
+  c->face2_used = false;
   c->pwork = nullptr; c->pwork_bytes = 0;
   c->mesh_ready = c->eta_ready = c->fac32_valid = c->facb32_valid = c->geo64_valid = c->has_state = false;
   c->ndir = 0;
@@ -384,11 +394,14 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   // face slots gets them, or the error, in the first call that needs them.
   const size_t neta = (size_t)nb * 27 * ptq2::BEL, nface = (size_t)nb * ptq2::FACEVALS + 1,
                nxt = nb >= 8192 ? (size_t)nb * 3 * ptq2::TCS : 0;
-  const size_t oface = neta, oxt = oface + (nface & ~(size_t)1);  // 16-byte aligned parts
+  const size_t oface = neta, oface2 = oface + (nface & ~(size_t)1), oxt = oface2 + (nface & ~(size_t)1);  // 16-byte aligned
   rc = nxt ? dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * (oxt + nxt)) : PTQ2_ERR_ALLOC;
   if (rc == PTQ2_OK) c->xtile = c->eta_bm + oxt;
   if (rc) rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * oxt);
-  if (rc == PTQ2_OK) c->facebuf = c->eta_bm + oface;
+  if (rc == PTQ2_OK) {
+    c->facebuf = c->eta_bm + oface;
+    c->facebuf2 = c->eta_bm + oface2;
+  }
   if (rc && (rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * neta))) return rc;
   b.xtile = c->xtile;
   c->box = b;
@@ -646,10 +659,8 @@ int ptq2_a11_diag(ptq2_ctx *c, double *d, unsigned flags) {
     if (add) HIPCHK(c, hipMemcpyAsync(c->sy, d, sizeof(double) * (size_t)n, hipMemcpyHostToDevice, c->stream));
     dd = (double *)c->sy;
   }
-  void *fb = ptq2_internal_facebuf(c, &rc);
-  if (rc) return rc;
   const auto bc = bc_of<double>(c, mm, 2);
-  HIPCHK(c, ptq2::launch_diag(c->box, c->coords, c->eta_bm, dd, add, (double *)fb, c->stream, &bc));
+  HIPCHK(c, ptq2::launch_diag(c->box, c->coords, c->eta_bm, dd, add, face2_of(c), c->stream, &bc));
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(d, dd, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -675,10 +686,8 @@ int ptq2_a12_apply(ptq2_ctx *c, const double *p, double *yu, unsigned flags) {
     dp = c->sp;
     dy = (double *)c->sy;
   }
-  void *fb = ptq2_internal_facebuf(c, &rc);
-  if (rc) return rc;
   const auto bc = bc_of<double>(c, mm, 1);
-  HIPCHK(c, ptq2::launch_a12(c->box, c->coords, dp, dy, add, (double *)fb, c->stream, &bc));
+  HIPCHK(c, ptq2::launch_a12(c->box, c->coords, dp, dy, add, face2_of(c), c->stream, &bc));
   if (!dev) {
     HIPCHK(c, hipMemcpyAsync(yu, dy, sizeof(double) * (size_t)c->nvel, hipMemcpyDeviceToHost, c->stream));
     int bits = 0;

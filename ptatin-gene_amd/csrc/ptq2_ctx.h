@@ -40,6 +40,12 @@ struct ptq2_ctx {
   // memory phases of some bricks overlapped with the arithmetic of others, which 8 coloured
   // launches of a few waves per SIMD do not.
   void *facebuf = nullptr;      // beside eta_bm, or facebuf_own
+  // Slots of A12 and the diagonal, which need none to run (8 coloured launches): calls on the stream that used
+  // them first share these, calls on any other stream run coloured, so that neither can meet another
+  // stream's apply in facebuf.
+  void *facebuf2 = nullptr;
+  hipStream_t face2_stream = nullptr;
+  bool face2_used = false;
   void *facebuf_own = nullptr;  // allocated on first use where the mesh set-up had no room
   // u with the Dirichlet values inserted, for the residual (allocated on first use)
   double *ures = nullptr;

@@ -99,6 +99,7 @@ hipError_t launch_eta_to_bm(const Box &b, const double *eta, double *eta_bm, int
 hipError_t launch_check_mesh(const Box &b, const double *coords, double *xtile, int *err, hipStream_t s);
 hipError_t launch_a21(const Box &b, const double *coords, const double *u, const uint8_t *mask, double *yp, bool add,
                       hipStream_t s);
+// A12 and the diagonal: one launch plus the face pass, or 8 coloured launches without face slots (facebuf null)
 hipError_t launch_a12(const Box &b, const double *coords, const double *p, double *y, bool add, double *facebuf,
                       hipStream_t s, const BcRows<double> *bc = nullptr);
 hipError_t launch_diag(const Box &b, const double *coords, const double *eta_bm, double *d, bool add, double *facebuf,

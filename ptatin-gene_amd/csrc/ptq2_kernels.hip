@@ -899,11 +899,12 @@ __device__ __forceinline__ void a12_rows(const double *Xs, int base, const PBasi
   if constexpr (R < 8) a12_rows<R + 1>(Xs, base, pb, ps, x, RB, RD, Y);
 }
 
-__global__ __launch_bounds__(BEL) void k_a12(Box b, const double *__restrict__ coords, const double *__restrict__ p,
+__global__ __launch_bounds__(BEL) void k_a12(Box b, int color, const double *__restrict__ coords,
+                                             const double *__restrict__ p,
                                              double *__restrict__ y, int add_mode, double *__restrict__ facebuf) {
   __shared__ double Xs[3 * TCS];
   const int lane = threadIdx.x;
-  const BrickId br = brick_xcd(b, blockIdx.x);
+  const BrickId br = color >= 0 ? brick_of(b, color, blockIdx.x) : brick_xcd(b, blockIdx.x);
   const Tile t = tile_of(b, br);
   const bool active = lane_active(t, lane);
   const double *pe = p + 4 * (active ? lane_element(b, t, lane) : 0);
@@ -933,7 +934,10 @@ __global__ __launch_bounds__(BEL) void k_a12(Box b, const double *__restrict__ c
     }
   }
   __syncthreads();
-  store_tile_own(b, br, t, Xs, y, facebuf, add_mode != 0, lane);
+  if (color >= 0)
+    store_tile(b, br, t, Xs, y, add_mode != 0, lane);
+  else
+    store_tile_own(b, br, t, Xs, y, facebuf, add_mode != 0, lane);
 }
 
 // ---------------------------------------------------------------- body force
@@ -1131,12 +1135,12 @@ __device__ __forceinline__ void diag_rows(const double *Xs, int base, const doub
   if constexpr (R < 8) diag_rows<R + 1>(Xs, base, ep, x, X);
 }
 
-__global__ __launch_bounds__(BEL) void k_diag(Box b, const double *__restrict__ coords,
+__global__ __launch_bounds__(BEL) void k_diag(Box b, int color, const double *__restrict__ coords,
                                               const double *__restrict__ eta_bm, double *__restrict__ d, int add_mode,
                                               double *__restrict__ facebuf) {
   __shared__ double Xs[3 * TCS];
   const int lane = threadIdx.x;
-  const BrickId br = brick_xcd(b, blockIdx.x);
+  const BrickId br = color >= 0 ? brick_of(b, color, blockIdx.x) : brick_xcd(b, blockIdx.x);
   const Tile t = tile_of(b, br);
   load_tile(b, t, br, coords, (const uint8_t *)nullptr, Xs, lane);
   __syncthreads();
@@ -1163,7 +1167,10 @@ __global__ __launch_bounds__(BEL) void k_diag(Box b, const double *__restrict__ 
         }
   }
   __syncthreads();
-  store_tile_own(b, br, t, Xs, d, facebuf, add_mode != 0, lane);
+  if (color >= 0)
+    store_tile(b, br, t, Xs, d, add_mode != 0, lane);
+  else
+    store_tile_own(b, br, t, Xs, d, facebuf, add_mode != 0, lane);
 }
 
 // ------------------------------------------------------------- BC helpers
@@ -1485,8 +1492,16 @@ hipError_t launch_a21(const Box &b, const double *coords, const double *u, const
 
 hipError_t launch_a12(const Box &b, const double *coords, const double *p, double *y, bool add, double *facebuf,
                       hipStream_t s, const BcRows<double> *bc) {
-  hipLaunchKernelGGL(k_a12, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, p, y, add ? 1 : 0, facebuf);
-  return launch_gather<double>(b, facebuf, y, s, nullptr, bc);
+  if (facebuf) {
+    hipLaunchKernelGGL(k_a12, dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, coords, p, y, add ? 1 : 0, facebuf);
+    return launch_gather<double>(b, facebuf, y, s, nullptr, bc);
+  }
+  for (int c = 0; c < 8; c++) {
+    const int nb = nbricks_color(b, c);
+    if (nb == 0) continue;
+    hipLaunchKernelGGL(k_a12, dim3(nb), dim3(BEL), 0, s, b, c, coords, p, y, add ? 1 : 0, (double *)nullptr);
+  }
+  return bc ? launch_bc_rows<double>(bc->n, bc->idx, bc->x, y, bc->mode, s, bc->v) : hipGetLastError();
 }
 
 hipError_t launch_body_force(const Box &b, const double *coords, const double *fu, double *y, bool add,
@@ -1509,8 +1524,16 @@ hipError_t launch_insert_bc(int64_t n, const double *u, const uint8_t *mask, con
 
 hipError_t launch_diag(const Box &b, const double *coords, const double *eta_bm, double *d, bool add, double *facebuf,
                        hipStream_t s, const BcRows<double> *bc) {
-  hipLaunchKernelGGL(k_diag, dim3(nbricks(b)), dim3(BEL), 0, s, b, coords, eta_bm, d, add ? 1 : 0, facebuf);
-  return launch_gather<double>(b, facebuf, d, s, nullptr, bc);
+  if (facebuf) {
+    hipLaunchKernelGGL(k_diag, dim3(nbricks(b)), dim3(BEL), 0, s, b, -1, coords, eta_bm, d, add ? 1 : 0, facebuf);
+    return launch_gather<double>(b, facebuf, d, s, nullptr, bc);
+  }
+  for (int c = 0; c < 8; c++) {
+    const int nb = nbricks_color(b, c);
+    if (nb == 0) continue;
+    hipLaunchKernelGGL(k_diag, dim3(nb), dim3(BEL), 0, s, b, c, coords, eta_bm, d, add ? 1 : 0, (double *)nullptr);
+  }
+  return bc ? launch_bc_rows<double>(bc->n, bc->idx, bc->x, d, bc->mode, s, bc->v) : hipGetLastError();
 }
 
 template <typename T>

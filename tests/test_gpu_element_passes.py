@@ -176,3 +176,28 @@ def test_full_block_and_residual(dims):
     F0 = A.ctx.residual(ud, pd, dev(fu), None, dev(phi))[1]
     assert rel(F0.cpu().numpy(), rp) <= 1e-12
     assert rel((F0 + F1).cpu().numpy(), Fp.cpu().numpy()) <= 1e-12
+
+
+@pytest.mark.parametrize("dims", [(4, 4, 4), (5, 4, 4), (9, 12, 8), (3, 13, 17)])
+def test_gradient_diagonal_on_a_second_stream(dims):
+    """A12 and the diagonal on a stream other than the one that used the face slots first run coloured:
+    set, ADD and MatMult equal to the oracle there too, and to the first stream's to rounding."""
+    print("case: A12 and diagonal on a second stream", dims, flush=True)
+    P = problem(dims)
+    A = ptq2.MatA11MF("hip")
+    A.setup(P)
+    p = M.uniform(4, 4 * int(np.prod(dims)), -1.0, 1.0)
+    pd = torch.from_numpy(p).to(DEV)
+    c = A.ctx
+    d = P.mask > 0
+    side = torch.cuda.Stream(device=DEV)
+    for ref, f, bc in ((O.a12(*dims, P.coords, p), lambda y, fl: c.a12(pd, y, fl), 0.0),
+                       (O.diag_a11(*dims, P.coords, P.eta), lambda y, fl: c.a11_diag(y, fl), 1.0)):
+        first = f(torch.zeros(P.nvel, dtype=torch.float64, device=DEV), 0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            y = [f(torch.full((P.nvel,), 0.5, dtype=torch.float64, device=DEV), fl) for fl in (0, _lib.ADD, _lib.MATMULT)]
+        torch.cuda.synchronize()
+        for got, want in zip(y, (ref, ref + 0.5, np.where(d, bc, ref))):
+            assert rel(got.cpu().numpy(), want) <= 1e-12
+        assert rel(first.cpu().numpy(), ref) <= 1e-12
