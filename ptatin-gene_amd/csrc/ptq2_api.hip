@@ -9,6 +9,7 @@
 // per-call re-uploads of mesh data); device-pointer calls are stream ordered.
 #include <hip/hip_runtime.h>
 
+#include <cfloat>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -156,10 +157,7 @@ int ptq2_internal_build_fac32(ptq2_ctx *c, bool block) {
 
 void *ptq2_internal_facebuf(ptq2_ctx *c, int *rc) {
   *rc = PTQ2_OK;
-  if (!c->facebuf) {
-    *rc = dev_alloc(c, &c->facebuf_own, sizeof(double) * (size_t)c->nbricks * ptq2::FACEVALS);
-    c->facebuf = c->facebuf_own;
-  }
+  if (!c->facebuf) *rc = dev_alloc(c, &c->facebuf, sizeof(double) * (size_t)c->nbricks * ptq2::FACEVALS);
   return c->facebuf;
 }
 
@@ -265,7 +263,7 @@ int ptq2_destroy(ptq2_ctx **pc) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   dev_free(c->coords); dev_free(c->mask); dev_free(c->dir_idx); dev_free(c->eta_bm);
-  dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf_own);
+  dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf);
   dev_free(c->pwork);
   dev_free(c->err); dev_free(c->su); dev_free(c->sy); dev_free(c->sp); dev_free(c->syp); dev_free(c->ures);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
@@ -303,19 +301,41 @@ int ptq2_sizes(const ptq2_ctx *c, int64_t *nv, int64_t *np, int64_t *ne) {
 }  // extern "C"
 
 namespace {
-// sets the flag of every brick whose tile holds box node n
-void mark_bricks(const Box &b, int64_t n, uint8_t *flag) {
-  const int e[3] = {(int)(n % b.NX) - b.i0, (int)(n / b.NX % b.NY) - b.j0, (int)(n / ((int64_t)b.NX * b.NY)) - b.k0};
-  const int m[3] = {b.mx, b.my, b.mz}, nb[3] = {b.nbx, b.nby, b.nbz};
-  int lo[3], hi[3];
-  for (int d = 0; d < 3; d++) {
-    if (e[d] < 0 || e[d] > 2 * m[d]) return;  // a ghost node of no owned element
-    hi[d] = std::min(e[d] / (2 * ptq2::BE), nb[d] - 1);
-    lo[d] = e[d] % (2 * ptq2::BE) == 0 && e[d] > 0 ? e[d] / (2 * ptq2::BE) - 1 : hi[d];
+// the bricks lo .. hi along an axis of m elements and nb bricks whose tiles hold node e (counted from the
+// first element's); lo > hi for a ghost node of no owned element
+struct BrickSpan {
+  int lo, hi;
+  BrickSpan(int e, int m, int nb) : lo(1), hi(0) {
+    constexpr int UP = 2 * ptq2::BE;
+    if (e < 0 || e > 2 * m) return;
+    hi = std::min(e / UP, nb - 1);
+    lo = e % UP == 0 && e > 0 ? e / UP - 1 : hi;
   }
-  for (int z = lo[2]; z <= hi[2]; z++)
-    for (int y = lo[1]; y <= hi[1]; y++)
-      for (int x = lo[0]; x <= hi[0]; x++) flag[x + (int64_t)b.nbx * (y + (int64_t)b.nby * z)] = 1;
+};
+// The Dirichlet dofs of the mask, and the flag of every brick whose tile holds one; row by row, as a division
+// per dof would be a tenth of a small mesh's set-up.
+void dirichlet_dofs(const Box &b, const uint8_t *mask, std::vector<int64_t> &idx, std::vector<uint8_t> &flag) {
+  for (int Z = 0; Z < b.NZ; Z++) {
+    const BrickSpan z(Z - b.k0, b.mz, b.nbz);
+    for (int Y = 0; Y < b.NY; Y++) {
+      const BrickSpan y(Y - b.j0, b.my, b.nby);
+      const int64_t row = 3 * (int64_t)b.NX * (Y + (int64_t)b.NY * Z);
+      for (int k = 0; k < 3 * b.NX; k++) {
+        uint64_t eight = 1;  // most rows hold none: eight dofs per test
+        if (k + 8 <= 3 * b.NX) memcpy(&eight, mask + row + k, 8);
+        if (!eight) {
+          k += 7;
+          continue;
+        }
+        if (!mask[row + k]) continue;
+        idx.push_back(row + k);
+        const BrickSpan x(k / 3 - b.i0, b.mx, b.nbx);
+        for (int bz = z.lo; bz <= z.hi; bz++)
+          for (int by = y.lo; by <= y.hi; by++)
+            for (int bx = x.lo; bx <= x.hi; bx++) flag[bx + (int64_t)b.nbx * (by + (int64_t)b.nby * bz)] = 1;
+      }
+    }
+  }
 }
 }  // namespace
 
@@ -336,18 +356,24 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   if (nn > ((int64_t)1 << 32) || ne > ((int64_t)1 << 31)) return fail(c, PTQ2_ERR_SIZE, "mesh too large");
   int rc = set_device(c);
   if (rc) return rc;
-  for (int64_t i = 0; i < 3 * nn; i++)
-    if (!std::isfinite(coords[i])) return fail(c, PTQ2_ERR_NONFINITE, "non-finite coordinate at dof %lld", (long long)i);
+  // in chunks without an early exit: the compiler vectorises those
+  for (int64_t i0 = 0; i0 < 3 * nn; i0 += 4096) {
+    const int64_t i1 = std::min<int64_t>(i0 + 4096, 3 * nn);
+    int bad = 0;
+    for (int64_t i = i0; i < i1; i++) bad |= !(std::fabs(coords[i]) <= DBL_MAX);
+    for (int64_t i = i0; bad && i < i1; i++)
+      if (!std::isfinite(coords[i])) return fail(c, PTQ2_ERR_NONFINITE, "non-finite coordinate at dof %lld", (long long)i);
+  }
 
   // release a previous mesh
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->gen++;
   dev_free(c->coords); dev_free(c->mask); dev_free(c->dir_idx); dev_free(c->eta_bm);
-  dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf_own);
+  dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf);
   dev_free(c->pwork);
   c->coords = nullptr; c->mask = nullptr; c->dir_idx = nullptr; c->eta_bm = nullptr;
   c->xtile = nullptr; c->bdir = nullptr;
-  c->fac32 = nullptr; c->facb32 = nullptr; c->geo64 = nullptr; c->facebuf = c->facebuf_own = c->facebuf2 = nullptr;
+  c->fac32 = nullptr; c->facb32 = nullptr; c->geo64 = nullptr; c->facebuf = c->facebuf2 = nullptr;
   c->face2_used = false;
   c->pwork = nullptr; c->pwork_bytes = 0;
   c->mesh_ready = c->eta_ready = c->fac32_valid = c->facb32_valid = c->geo64_valid = c->has_state = false;
@@ -369,11 +395,7 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   if (mask) {
     std::vector<int64_t> idx;
     std::vector<uint8_t> bdir((size_t)nb, 0);
-    for (int64_t i = 0; i < 3 * nn; i++)
-      if (mask[i]) {
-        idx.push_back(i);
-        mark_bricks(b, i / 3, bdir.data());
-      }
+    dirichlet_dofs(b, mask, idx, bdir);
     if ((rc = dev_alloc(c, (void **)&c->mask, 3 * (size_t)nn + (size_t)nb))) return rc;
     HIPCHK(c, hipMemcpy(c->mask, mask, 3 * (size_t)nn, hipMemcpyHostToDevice));
     c->bdir = c->mask + 3 * (size_t)nn;
@@ -385,23 +407,19 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
       HIPCHK(c, hipMemcpy(c->dir_idx, idx.data(), sizeof(int64_t) * idx.size(), hipMemcpyHostToDevice));
     }
   }
-  // Viscosity, face slots and the resident coordinate tiles share an allocation (a hipMalloc of its own for
-  // the slots makes the set-up of a 40^3 mesh a tenth longer, and in an operator's first call it would be
-  // refused under capture).  The tiles pay where the vectors come from HBM, not from the 256 MB cache before it:
-  // FP64 apply 1113 us with, 1163 us without at 128^3 elements (32768 bricks), 145 us with and without at 64^3
-  // (4096 bricks), where they would only make the set-up longer (by a tenth at 33^3).  A mesh that fits
-  // the device only without them runs its FP64 passes from the coordinates too; one that fits only without the
-  // face slots gets them, or the error, in the first call that needs them.
+  // Viscosity, the face slots of A12 and the diagonal (which thus never allocate) and the resident coordinate
+  // tiles share an allocation.  The tiles pay where the vectors come from HBM, not from the 256 MB cache before
+  // it: FP64 apply 1113 us with, 1163 us without at 128^3 elements (32768 bricks), 145 us with and without at
+  // 64^3 (4096 bricks), where they would only make the set-up longer (by a tenth at 33^3).  A mesh that fits
+  // the device only without them runs its FP64 passes from the coordinates too; one that fits only without
+  // those slots runs A12 and the diagonal in coloured launches.
   const size_t neta = (size_t)nb * 27 * ptq2::BEL, nface = (size_t)nb * ptq2::FACEVALS + 1,
                nxt = nb >= 8192 ? (size_t)nb * 3 * ptq2::TCS : 0;
-  const size_t oface = neta, oface2 = oface + (nface & ~(size_t)1), oxt = oface2 + (nface & ~(size_t)1);  // 16-byte aligned
+  const size_t oxt = neta + (nface & ~(size_t)1);  // 16-byte aligned
   rc = nxt ? dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * (oxt + nxt)) : PTQ2_ERR_ALLOC;
   if (rc == PTQ2_OK) c->xtile = c->eta_bm + oxt;
   if (rc) rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * oxt);
-  if (rc == PTQ2_OK) {
-    c->facebuf = c->eta_bm + oface;
-    c->facebuf2 = c->eta_bm + oface2;
-  }
+  if (rc == PTQ2_OK) c->facebuf2 = c->eta_bm + neta;
   if (rc && (rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * neta))) return rc;
   b.xtile = c->xtile;
   c->box = b;

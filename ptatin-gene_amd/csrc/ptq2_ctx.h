@@ -39,14 +39,13 @@ struct ptq2_ctx {
   // pass adds the face slots into their owners (ptq2::launch_a11_*).  One launch keeps the
   // memory phases of some bricks overlapped with the arithmetic of others, which 8 coloured
   // launches of a few waves per SIMD do not.
-  void *facebuf = nullptr;      // beside eta_bm, or facebuf_own
+  void *facebuf = nullptr;
   // Slots of A12 and the diagonal, which need none to run (8 coloured launches): calls on the stream that used
   // them first share these, calls on any other stream run coloured, so that neither can meet another
   // stream's apply in facebuf.
-  void *facebuf2 = nullptr;
+  void *facebuf2 = nullptr;  // beside eta_bm
   hipStream_t face2_stream = nullptr;
   bool face2_used = false;
-  void *facebuf_own = nullptr;  // allocated on first use where the mesh set-up had no room
   // u with the Dirichlet values inserted, for the residual (allocated on first use)
   double *ures = nullptr;
   size_t ures_bytes = 0;
