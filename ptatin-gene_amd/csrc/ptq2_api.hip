@@ -165,9 +165,13 @@ namespace {
 
 int build_fac32(ptq2_ctx *c) { return ptq2_internal_build_fac32(c); }
 
-// how the FP64 A11 pass leaves y (it writes the Dirichlet rows of a MatMult itself)
+// how the FP64 A11 pass leaves y (it writes the Dirichlet rows of a MatMult itself, those of its tiles)
 ptq2::OutMode out_mode(const ptq2_ctx *c, bool mm, bool add) {
   return mm && c->mask ? ptq2::OUT_BC : (add ? ptq2::OUT_ADD : ptq2::OUT_SET);
+}
+// the Dirichlet rows of a MatMult that no tile holds
+ptq2::BcRows<double> ghost_bc_of(const ptq2_ctx *c, bool mm, const double *x) {
+  return ptq2::BcRows<double>{mm ? c->ndir_ghost : 0, c->dir_idx + (c->ndir - c->ndir_ghost), c->mask, x, nullptr, 0};
 }
 
 // resident FP64 geometry of the stored-geometry A11 kernel (depends on the mesh only)
@@ -313,8 +317,10 @@ struct BrickSpan {
   }
 };
 // The Dirichlet dofs of the mask, and the flag of every brick whose tile holds one; row by row, as a division
-// per dof would be a tenth of a small mesh's set-up.
-void dirichlet_dofs(const Box &b, const uint8_t *mask, std::vector<int64_t> &idx, std::vector<uint8_t> &flag) {
+// per dof would be a tenth of a small mesh's set-up.  Those that no tile holds (on ghost nodes of no owned
+// element) come last; returns their number.
+int64_t dirichlet_dofs(const Box &b, const uint8_t *mask, std::vector<int64_t> &idx, std::vector<uint8_t> &flag) {
+  std::vector<int64_t> ghost;
   for (int Z = 0; Z < b.NZ; Z++) {
     const BrickSpan z(Z - b.k0, b.mz, b.nbz);
     for (int Y = 0; Y < b.NY; Y++) {
@@ -328,14 +334,16 @@ void dirichlet_dofs(const Box &b, const uint8_t *mask, std::vector<int64_t> &idx
           continue;
         }
         if (!mask[row + k]) continue;
-        idx.push_back(row + k);
         const BrickSpan x(k / 3 - b.i0, b.mx, b.nbx);
+        (x.lo > x.hi || y.lo > y.hi || z.lo > z.hi ? ghost : idx).push_back(row + k);
         for (int bz = z.lo; bz <= z.hi; bz++)
           for (int by = y.lo; by <= y.hi; by++)
             for (int bx = x.lo; bx <= x.hi; bx++) flag[bx + (int64_t)b.nbx * (by + (int64_t)b.nby * bz)] = 1;
       }
     }
   }
+  idx.insert(idx.end(), ghost.begin(), ghost.end());
+  return (int64_t)ghost.size();
 }
 }  // namespace
 
@@ -377,7 +385,7 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   c->face2_used = false;
   c->pwork = nullptr; c->pwork_bytes = 0;
   c->mesh_ready = c->eta_ready = c->fac32_valid = c->facb32_valid = c->geo64_valid = c->has_state = false;
-  c->ndir = 0;
+  c->ndir = c->ndir_ghost = 0;
 
   Box b{};
   b.mx = mx; b.my = my; b.mz = mz; b.NX = NX; b.NY = NY; b.NZ = NZ; b.i0 = i0; b.j0 = j0; b.k0 = k0;
@@ -395,7 +403,7 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   if (mask) {
     std::vector<int64_t> idx;
     std::vector<uint8_t> bdir((size_t)nb, 0);
-    dirichlet_dofs(b, mask, idx, bdir);
+    c->ndir_ghost = dirichlet_dofs(b, mask, idx, bdir);
     if ((rc = dev_alloc(c, (void **)&c->mask, 3 * (size_t)nn + (size_t)nb))) return rc;
     HIPCHK(c, hipMemcpy(c->mask, mask, 3 * (size_t)nn, hipMemcpyHostToDevice));
     c->bdir = c->mask + 3 * (size_t)nn;
@@ -538,10 +546,10 @@ int ptq2_a11_apply(ptq2_ctx *c, const void *u, void *y, unsigned flags) {
                                       (float *)tb, true, nullptr, &bc));
     }
   } else {
-    const auto bc = bc_of(c, mm, 0, (const double *)du);
+    const auto bc = bc_of(c, mm, 0, (const double *)du), ghost = ghost_bc_of(c, mm, (const double *)du);
     if (otf)
       HIPCHK(c, ptq2::launch_a11_fp64(c->box, c->coords, (const double *)du, mask, c->eta_bm, (double *)dy,
-                                      out_mode(c, mm, add), c->stream, (double *)tb));
+                                      out_mode(c, mm, add), c->stream, (double *)tb, true, nullptr, &ghost));
     else
       HIPCHK(c, ptq2::launch_a11_fp64g(c->box, (const double *)du, mask, c->geo64, c->eta_bm, (double *)dy, add,
                                        c->stream, (double *)tb, &bc));
@@ -573,8 +581,9 @@ int ptq2_a11_apply_noalloc(ptq2_ctx *c, const double *u, double *y, unsigned fla
   const bool mm = flags & PTQ2_MATMULT, add = flags & PTQ2_ADD;
   // every face slot the gather pass reads is written by the apply launch before it in stream
   // order, so the array needs no clearing between calls
+  const auto ghost = ghost_bc_of(c, mm, u);
   HIPCHK(c, ptq2::launch_a11_fp64(c->box, c->coords, u, mm ? c->mask : nullptr, c->eta_bm, y, out_mode(c, mm, add),
-                                  c->stream, scr));
+                                  c->stream, scr, true, nullptr, &ghost));
   return PTQ2_OK;
 }
 
@@ -633,9 +642,11 @@ int a11_batch(ptq2_ctx *const *cs, int n, const void *const *u, void *const *y, 
     HIPCHK(c0, hipStreamWaitEvent(c0->stream, c->ev, 0));
   }
   HIPCHK(c0, ptq2::launch_a11_batch<T>(a, c0->stream));
-  if (mm && f32)  // the FP64 pass writes the Dirichlet rows itself
-    for (int i = 0; i < n; i++)
-      HIPCHK(c0, ptq2::launch_bc_rows<T>(cs[i]->ndir, cs[i]->dir_idx, (const T *)u[i], (T *)y[i], 0, c0->stream));
+  for (int i = 0; mm && i < n; i++) {
+    const int64_t nd = f32 ? cs[i]->ndir : cs[i]->ndir_ghost;  // the FP64 pass writes those of its tiles itself
+    HIPCHK(c0, ptq2::launch_bc_rows<T>(nd, cs[i]->dir_idx + (cs[i]->ndir - nd), (const T *)u[i], (T *)y[i], 0,
+                                       c0->stream));
+  }
   bool others = false;
   for (int i = 1; i < n; i++) others |= cs[i]->stream != c0->stream;
   if (others) {

@@ -20,6 +20,7 @@ struct ptq2_ctx {
   uint8_t *bdir = nullptr;  // box.bdir: bricks that hold a Dirichlet dof
   int64_t *dir_idx = nullptr;
   int64_t ndir = 0;
+  int64_t ndir_ghost = 0;  // the last of dir_idx: dofs of ghost nodes that no brick's tile holds
   double *eta_bm = nullptr;
   float *fac32 = nullptr;
   bool fac32_valid = false;

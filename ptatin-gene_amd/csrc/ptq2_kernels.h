@@ -53,9 +53,11 @@ struct BcRows {
 // slots itself); without facebuf, 8 coloured launches store/add directly.
 // co (one-launch path only): the owned nodes that no face slot adds to get the Chebyshev update
 // of co instead of being stored into y (the face pass updates the rest)
+// ghost (FP64, OUT_BC): the mask's dofs that no brick's tile holds, which the face pass writes
 hipError_t launch_a11_fp64(const Box &b, const double *coords, const double *u, const uint8_t *mask,
                            const double *eta_bm, double *y, OutMode mode, hipStream_t s, double *facebuf,
-                           bool gather = true, const ChebOut<double> *co = nullptr);
+                           bool gather = true, const ChebOut<double> *co = nullptr,
+                           const BcRows<double> *ghost = nullptr);
 // the full block [A11 A12; A21 0] in one element pass (FP64); fp (27 per element, may be null)
 // subtracts the continuity source from yp
 hipError_t launch_stokes_fp64(const Box &b, const double *coords, const double *u, const double *p,

@@ -1333,7 +1333,7 @@ hipError_t launch_gather(const Box &b, const T *face, T *y, hipStream_t s, const
 
 hipError_t launch_a11_fp64(const Box &b, const double *coords, const double *u, const uint8_t *mask,
                            const double *eta_bm, double *y, OutMode mode, hipStream_t s, double *facebuf, bool gather,
-                           const ChebOut<double> *co) {
+                           const ChebOut<double> *co, const BcRows<double> *ghost) {
   const dim3 grid(nbricks(b)), block(CWAVES * BEL);
   if (co) {
     hipLaunchKernelGGL(k_a11_fp64_t<true>, grid, block, 0, s, b, coords, u, mask, eta_bm, y, (int)OUT_SET, facebuf, *co);
@@ -1341,7 +1341,8 @@ hipError_t launch_a11_fp64(const Box &b, const double *coords, const double *u, 
   }
   hipLaunchKernelGGL(k_a11_fp64_t<false>, grid, block, 0, s, b, coords, u, mask, eta_bm, y, (int)mode, facebuf,
                      ChebOut<double>{});
-  return gather ? launch_gather(b, (const double *)facebuf, y, s, mode == OUT_BC ? mask : nullptr) : hipGetLastError();
+  return gather ? launch_gather(b, (const double *)facebuf, y, s, mode == OUT_BC ? mask : nullptr, ghost)
+                : hipGetLastError();
 }
 
 hipError_t launch_gather_faces(const Box &b, const float *face, float *y, hipStream_t s, const BcRows<float> *bc) {
