@@ -218,6 +218,13 @@ __host__ __device__ __forceinline__ uint32_t fast_eoff(const Box &b, const FastL
   if (it == STEPS - 1 && L.p == 1) return (uint32_t)L.col;
   return (fast_wrap(it) ? L.ew : L.e0) + fast_step(b, it);
 }
+// this lane's LDS offset at step it of ROWS rows from the first one's plane on (row 0 for the lanes that store
+// nothing at that step: the row after the last may lie past the tile)
+template <int ROWS>
+__host__ __device__ __forceinline__ int fast_loff(const FastLane &L, int it) {
+  if (2 * it + 1 >= ROWS && L.p == 1) return L.lds0 - TRS;
+  return (fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it);
+}
 // (y, z) of this lane's row at step it
 __host__ __device__ __forceinline__ void fast_row(const FastLane &L, int it, int &y, int &z) {
   const int odd = L.p == 1, y0 = (2 * it) % TN, z0 = (2 * it) / TN;
@@ -478,7 +485,7 @@ __device__ __forceinline__ void store_rows_full(const Box &b, const BrickId &br,
   s += TPS * z0;
   T val[STEPS];
 #pragma unroll
-  for (int it = 0; it < STEPS; it++) val[it] = T(s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)]);
+  for (int it = 0; it < STEPS; it++) val[it] = T(s[fast_loff<ROWS>(L, it)]);
   if (!ALL && add_mode && ownz) {
     T old[STEPS];
 #pragma unroll
