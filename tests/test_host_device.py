@@ -8,7 +8,7 @@ REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(REPO, "ptatin-gene_amd", "csrc")
 
 
-@pytest.mark.parametrize("name,line", [("test_tile_rows", "tile rows ok")])
+@pytest.mark.parametrize("name,line", [("test_tile_rows", "tile rows ok"), ("test_row_sums", "row sums ok")])
 def test_host_check(tmp_path, name, line):
     exe = str(tmp_path / name)
     subprocess.check_call(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "-O1", "-std=c++17", "-x", "hip", "-I", CSRC,
