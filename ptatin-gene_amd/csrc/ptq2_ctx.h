@@ -41,12 +41,12 @@ struct ptq2_ctx {
   // memory phases of some bricks overlapped with the arithmetic of others, which 8 coloured
   // launches of a few waves per SIMD do not.
   void *facebuf = nullptr;
-  // Slots of A12 and the diagonal, which need none to run (8 coloured launches): calls on the stream that used
-  // them first share these, calls on any other stream run coloured, so that neither can meet another
-  // stream's apply in facebuf.
+  // Slots of A12 and the diagonal, which need none to run (8 coloured launches): apart from facebuf, which an
+  // apply on another stream may be using, and handed from call to call by an event.
   void *facebuf2 = nullptr;  // beside eta_bm
-  hipStream_t face2_stream = nullptr;
-  bool face2_used = false;
+  hipEvent_t face2_ev = nullptr;
+  bool face2_used = false;             // since the mesh set-up
+  hipStream_t face2_stream = nullptr;  // of the last use
   // u with the Dirichlet values inserted, for the residual (allocated on first use)
   double *ures = nullptr;
   size_t ures_bytes = 0;
