@@ -9,6 +9,7 @@
 // per-call re-uploads of mesh data); device-pointer calls are stream ordered.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cfloat>
 #include <cmath>
 #include <cstdarg>
@@ -75,6 +76,10 @@ int dev_alloc(ptq2_ctx *c, void **p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) return PTQ2_OK;
   hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && ptq2_internal_give_back(c)) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
   if (e != hipSuccess) {
     (void)hipGetLastError();
     *p = nullptr;
@@ -93,12 +98,50 @@ ptq2::BcRows<T> bc_of(const ptq2_ctx *c, bool mm, int mode, const T *x = nullptr
   return ptq2::BcRows<T>{mm ? c->ndir : 0, c->dir_idx, c->mask, x, v, mode};
 }
 
-// Whether work on s is being captured into a graph (or s is the null stream and another's capture forbids its use).
-bool capturing(hipStream_t s) {
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
-  (void)hipGetLastError();
-  return true;
+bool capturing(hipStream_t s) { return ptq2_internal_capturing(s); }
+
+// Spare memory of all contexts of a device: a sixteenth of it at most, so that programs that fill the device
+// with other data do not miss it.
+std::atomic<size_t> g_spare[NOALLOC_MAXDEV];
+void take_spare(ptq2_ctx *c, size_t nslots, size_t ntiles) {
+  size_t avail = 0, total = 0;
+  if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  for (size_t tiles : {ntiles, size_t(0)}) {
+    const size_t bytes = sizeof(double) * (nslots + tiles);
+    bool room = g_spare[c->device].fetch_add(bytes) + bytes <= total / 16;
+    if (room && hipMalloc(&c->spare, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      c->spare = nullptr;
+      room = false;
+    }
+    if (!room) {
+      g_spare[c->device] -= bytes;
+      continue;
+    }
+    c->spare_bytes = bytes;
+    c->facebuf2 = c->spare;
+    if (tiles) c->box.xtile = (double *)c->spare + nslots;
+    return;
+  }
+}
+void free_spare(ptq2_ctx *c) {
+  if (!c->spare) return;
+  (void)hipFree(c->spare);
+  g_spare[c->device] -= c->spare_bytes;
+  c->spare = c->facebuf2 = nullptr;
+  c->spare_bytes = 0;
+  c->spare_held = false;
+  c->box.xtile = nullptr;
+}
+
+// the box of an FP64 apply on s: without the tiles for a captured one, whose graph may outlive them
+Box box_of(const ptq2_ctx *c, hipStream_t s) {
+  Box b = c->box;
+  if (b.xtile && capturing(s)) b.xtile = nullptr;
+  return b;
 }
 
 // The face slots of A12 and the diagonal for a call on the context's present stream, or null: 8 coloured
@@ -165,6 +208,25 @@ int clear_err(ptq2_ctx *c) {
 }
 
 }  // namespace
+
+bool ptq2_internal_capturing(hipStream_t s) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+bool ptq2_internal_give_back(ptq2_ctx *c, bool work) {
+  if (!c) return false;
+  const bool any = (c->spare && !c->spare_held) || (work && c->pwork);
+  if (!c->spare_held) free_spare(c);  // hipFree waits for what runs on them
+  if (work) {
+    dev_free(c->pwork);
+    c->pwork = nullptr;
+    c->pwork_bytes = 0;
+  }
+  return any;
+}
 
 int ptq2_internal_build_fac32(ptq2_ctx *c, bool block) {
   if (c->fac32_valid && (!block || c->facb32_valid)) return PTQ2_OK;
@@ -304,6 +366,7 @@ int ptq2_destroy(ptq2_ctx **pc) {
   dev_free(c->coords); dev_free(c->mask); dev_free(c->dir_idx); dev_free(c->eta_bm);
   dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf);
   dev_free(c->pwork);
+  free_spare(c);
   dev_free(c->err); dev_free(c->su); dev_free(c->sy); dev_free(c->sp); dev_free(c->syp); dev_free(c->ures);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
   if (c->ev) (void)hipEventDestroy(c->ev);
@@ -415,8 +478,9 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   dev_free(c->coords); dev_free(c->mask); dev_free(c->dir_idx); dev_free(c->eta_bm);
   dev_free(c->fac32); dev_free(c->facb32); dev_free(c->geo64); dev_free(c->facebuf);
   dev_free(c->pwork);
+  free_spare(c);
   c->coords = nullptr; c->mask = nullptr; c->dir_idx = nullptr; c->eta_bm = nullptr;
-  c->xtile = nullptr; c->bdir = nullptr;
+  c->bdir = nullptr;
   c->fac32 = nullptr; c->facb32 = nullptr; c->geo64 = nullptr; c->facebuf = c->facebuf2 = nullptr;
   c->face2_used = false;
   c->pwork = nullptr; c->pwork_bytes = 0;
@@ -451,25 +515,20 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
       HIPCHK(c, hipMemcpy(c->dir_idx, idx.data(), sizeof(int64_t) * idx.size(), hipMemcpyHostToDevice));
     }
   }
-  // Viscosity, the face slots of A12 and the diagonal (which thus never allocate) and the resident coordinate
-  // tiles share an allocation.  The tiles pay where the vectors come from HBM, not from the 256 MB cache before
-  // it: FP64 apply 1113 us with, 1163 us without at 128^3 elements (32768 bricks), 145 us with and without at
-  // 64^3 (4096 bricks), where they would only make the set-up longer (by a tenth at 33^3).  A mesh that fits
-  // the device only without them runs its FP64 passes from the coordinates too; one that fits only without
-  // those slots runs A12 and the diagonal in coloured launches.
-  const size_t neta = (size_t)nb * 27 * ptq2::BEL, nface = (size_t)nb * ptq2::FACEVALS + 1,
-               nxt = nb >= 8192 ? (size_t)nb * 3 * ptq2::TCS : 0;
-  const size_t oxt = neta + (nface & ~(size_t)1);  // 16-byte aligned
-  rc = nxt ? dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * (oxt + nxt)) : PTQ2_ERR_ALLOC;
-  if (rc == PTQ2_OK) c->xtile = c->eta_bm + oxt;
-  if (rc) rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * oxt);
-  if (rc == PTQ2_OK) c->facebuf2 = c->eta_bm + neta;
-  if (rc && (rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * neta))) return rc;
-  b.xtile = c->xtile;
   c->box = b;
   c->nnodes = nn; c->nvel = 3 * nn; c->nel = ne; c->npres = 4 * ne; c->nbricks = nb;
+  // The face slots of A12 and the diagonal, which thus never allocate, share the viscosity's allocation on small
+  // meshes (48 MB at most; one of their own would make a small set-up longer).  Large ones take them and the
+  // resident coordinate tiles as spare memory.  The tiles pay where the vectors come from HBM, not from the 256 MB
+  // cache before it: FP64 apply 1113 us with, 1163 us without at 128^3 elements (32768 bricks), 145 us with and
+  // without at 64^3 (4096 bricks).  A mesh without the slots runs A12 and the diagonal in coloured launches.
+  const size_t neta = (size_t)nb * 27 * ptq2::BEL, nface = ((size_t)nb * ptq2::FACEVALS + 1) & ~(size_t)1;
+  if (nb < 8192 && (rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * (neta + nface))) == PTQ2_OK)
+    c->facebuf2 = c->eta_bm + neta;
+  if (!c->eta_bm && (rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * neta))) return rc;
+  if (nb >= 8192) take_spare(c, nface, (size_t)nb * 3 * ptq2::TCS);
   if ((rc = clear_err(c))) return rc;
-  HIPCHK(c, ptq2::launch_check_mesh(b, c->coords, c->xtile, c->err, c->stream));
+  HIPCHK(c, ptq2::launch_check_mesh(c->box, c->coords, const_cast<double *>(c->box.xtile), c->err, c->stream));
   int bits = 0;
   if ((rc = read_err(c, &bits))) return rc;
   if (bits & ptq2::ERRBIT_MESH) return fail(c, PTQ2_ERR_MESH, "non-positive Jacobian determinant in the mesh");
@@ -584,7 +643,7 @@ int ptq2_a11_apply(ptq2_ctx *c, const void *u, void *y, unsigned flags) {
   } else {
     const auto bc = bc_of(c, mm, 0, (const double *)du), ghost = ghost_bc_of(c, mm, (const double *)du);
     if (otf)
-      HIPCHK(c, ptq2::launch_a11_fp64(c->box, c->coords, (const double *)du, mask, c->eta_bm, (double *)dy,
+      HIPCHK(c, ptq2::launch_a11_fp64(box_of(c, c->stream), c->coords, (const double *)du, mask, c->eta_bm, (double *)dy,
                                       out_mode(c, mm, add), c->stream, (double *)tb, true, nullptr, &ghost));
     else
       HIPCHK(c, ptq2::launch_a11_fp64g(c->box, (const double *)du, mask, c->geo64, c->eta_bm, (double *)dy, add,
@@ -618,7 +677,7 @@ int ptq2_a11_apply_noalloc(ptq2_ctx *c, const double *u, double *y, unsigned fla
   // every face slot the gather pass reads is written by the apply launch before it in stream
   // order, so the array needs no clearing between calls
   const auto ghost = ghost_bc_of(c, mm, u);
-  HIPCHK(c, ptq2::launch_a11_fp64(c->box, c->coords, u, mm ? c->mask : nullptr, c->eta_bm, y, out_mode(c, mm, add),
+  HIPCHK(c, ptq2::launch_a11_fp64(box_of(c, c->stream), c->coords, u, mm ? c->mask : nullptr, c->eta_bm, y, out_mode(c, mm, add),
                                   c->stream, scr, true, nullptr, &ghost));
   return PTQ2_OK;
 }
@@ -653,7 +712,7 @@ int a11_batch(ptq2_ctx *const *cs, int n, const void *const *u, void *const *y, 
     void *fb = ptq2_internal_facebuf(c, &rc);
     if (rc) return fail(c0, rc, "problem %d: %s", i, c->last.c_str());
     a.start[i] = (int)blocks;
-    a.box[i] = c->box;
+    a.box[i] = box_of(c, c0->stream);
     a.u[i] = (const T *)u[i];
     a.y[i] = (T *)y[i];
     a.face[i] = (T *)fb;
@@ -870,7 +929,7 @@ int ptq2_stokes_apply(ptq2_ctx *c, const void *u, const void *p, void *yu, void 
     const auto bc = bc_of(c, mm, 0, (const double *)du);
     if (otf) {
       // momentum A11 u + A12 p and continuity A21 u in one element pass (MFStokesWrapper_A_AVX)
-      HIPCHK(c, ptq2::launch_stokes_fp64(c->box, c->coords, (const double *)du, (const double *)dp, mask, c->eta_bm,
+      HIPCHK(c, ptq2::launch_stokes_fp64(box_of(c, c->stream), c->coords, (const double *)du, (const double *)dp, mask, c->eta_bm,
                                          (double *)dyu, (double *)dyp, nullptr, add, c->stream, (double *)fb, &bc));
     } else {
       // resident geometry: the A11 kernel of that form, then A12 and A21
@@ -939,7 +998,7 @@ int ptq2_stokes_residual(ptq2_ctx *c, const double *u, const double *p, const do
   void *fb = ptq2_internal_facebuf(c, &rc);
   if (rc) return rc;
   // Fu = A11 u_loc + A12 p, Fp = A21 u_loc - int N^p fp (one element pass), then Fu -= Be
-  HIPCHK(c, ptq2::launch_stokes_fp64(c->box, c->coords, ul, dp, nullptr, c->eta_bm, dFu, dFp, dfp, false, c->stream,
+  HIPCHK(c, ptq2::launch_stokes_fp64(box_of(c, c->stream), c->coords, ul, dp, nullptr, c->eta_bm, dFu, dFp, dfp, false, c->stream,
                                      (double *)fb, nullptr, false));
   // Dirichlet rows: Fu_D = u_D - phi_D (BCListResidualDirichlet, src/dmda_bcs.c:614-648)
   const auto bc = bc_of(c, true, 3, du, dphi);

@@ -15,7 +15,6 @@ struct ptq2_ctx {
   ptq2::Box box{};
   int64_t nnodes = 0, nvel = 0, nel = 0, npres = 0, nbricks = 0;
   double *coords = nullptr;
-  double *xtile = nullptr;  // box.xtile: the bricks' coordinate tiles
   uint8_t *mask = nullptr;
   uint8_t *bdir = nullptr;  // box.bdir: bricks that hold a Dirichlet dof
   int64_t *dir_idx = nullptr;
@@ -43,10 +42,15 @@ struct ptq2_ctx {
   void *facebuf = nullptr;
   // Slots of A12 and the diagonal, which need none to run (8 coloured launches): apart from facebuf, which an
   // apply on another stream may be using, and handed from call to call by an event.
-  void *facebuf2 = nullptr;  // beside eta_bm
+  void *facebuf2 = nullptr;  // beside eta_bm, or in spare
   hipEvent_t face2_ev = nullptr;
   bool face2_used = false;             // since the mesh set-up
   hipStream_t face2_stream = nullptr;  // of the last use
+  // What a large mesh runs faster with but not only with: the slots facebuf2 and the coordinate tiles box.xtile.
+  // Given back when an allocation of this context (or of a hierarchy on it) finds no memory.
+  void *spare = nullptr;
+  size_t spare_bytes = 0;
+  bool spare_held = false;  // a graph that a caller captured may hold its addresses
   // u with the Dirichlet values inserted, for the residual (allocated on first use)
   double *ures = nullptr;
   size_t ures_bytes = 0;
@@ -67,6 +71,10 @@ struct ptq2_ctx {
 // (re)build the FP32 geometric factors of the smoother operator if stale; with block,
 // also those of the FP32 full block
 int ptq2_internal_build_fac32(ptq2_ctx *c, bool block = false);
+// Gives spare memory (and, with work, the projection's workspace) back; whether there was any.  Waits for the device.
+bool ptq2_internal_give_back(ptq2_ctx *c, bool work = true);
+// whether work on s is being captured into a graph (or s is the null stream and another's capture forbids its use)
+bool ptq2_internal_capturing(hipStream_t s);
 // the tile buffer of the uncoloured output path if this mesh uses it (allocated on first
 // use), else nullptr; *rc receives an allocation error
 void *ptq2_internal_facebuf(ptq2_ctx *c, int *rc);

@@ -257,11 +257,23 @@ int pfail(ptq2_ctx *c, int code, const char *fmt, ...) {
   return code;
 }
 
+// hipMalloc that has the context's spare memory given back before it fails
+hipError_t take(ptq2_ctx *c, void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && ptq2_internal_give_back(c, false)) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
 // device scratch of one projection call, freed on every return path
 struct Scratch {
   static constexpr int CAP = 16;  // a call takes at most 11 buffers
+  ptq2_ctx *c;
   void *p[CAP] = {};
   int n = 0;
+  explicit Scratch(ptq2_ctx *c_) : c(c_) {}
   ~Scratch() {
     for (int i = 0; i < n; i++)
       if (p[i]) (void)hipFree(p[i]);
@@ -273,7 +285,7 @@ struct Scratch {
       *out = nullptr;
       return hipErrorOutOfMemory;
     }
-    hipError_t e = hipMalloc(&q, bytes ? bytes : 1);
+    const hipError_t e = take(c, &q, bytes ? bytes : 1);
     if (e == hipSuccess) p[n++] = q;
     *out = (T *)q;
     return e;
@@ -287,7 +299,7 @@ hipError_t grow(ptq2_ctx *c, size_t bytes) {
   if (c->pwork) (void)hipFree(c->pwork);
   c->pwork = nullptr;
   c->pwork_bytes = 0;
-  const hipError_t e = hipMalloc(&c->pwork, bytes);
+  const hipError_t e = take(c, &c->pwork, bytes);
   if (e == hipSuccess) c->pwork_bytes = bytes;
   else c->pwork = nullptr;
   return e;
@@ -323,7 +335,7 @@ extern "C" int ptq2_project_points_q1(ptq2_ctx *c, int64_t np, const double *xi,
   const bool dev = flags & PTQ2_DEVICE;
   const int64_t ne = c->nel, nn = c->nnodes;
   hipStream_t s = c->stream;
-  Scratch S;
+  Scratch S(c);
   const double *dxi = xi, *deta = eta_p, *drho = rho_p;
   const int32_t *dwil = wil;
   double *deq = eta_qp, *drq = rho_qp;

@@ -1208,7 +1208,8 @@ struct ptq2_mg {
   std::vector<double *> gst64;          // its stencil in FP64 (probing, FP64 applies)
   std::vector<float *> gst32;           // and in FP32 (FP32 smoothing)
   std::vector<void *> gmf_in, gmf_out;  // Galerkin level applied as R A P: vectors of the level above
-  std::vector<ptq2::Box> lbox;          // per level: the box of the level's launches (tuned fast32)
+  std::vector<ptq2::Box> lbox;          // per level: the box of the level's launches (tuned fast32; level_box)
+  bool no_tiles = false;                // the V-cycle is being captured by the caller
   bool prof = false;                    // record per-level events in the eager V-cycle
   std::vector<hipEvent_t> pev;          // 4 per level: entry, before / after the coarser level, exit
   int nl = 0;
@@ -1225,6 +1226,7 @@ struct ptq2_mg {
   VcIO *io = nullptr;                   // input/output record of the V-cycle (level 0, FP64 vectors)
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  int graph_tiles = 0;                  // levels that had resident coordinate tiles when it was captured
   // Krylov workspace.  FP64 basis: Vk[j] holds candidate j, then basis vector j.  FP32 basis
   // (basis32): candidates alternate between Vk[0] and Vk[1], finished vectors go to V32[j].
   bool basis32 = false;
@@ -1266,8 +1268,33 @@ int mgfail(ptq2_mg *g, int code, const char *msg) {
     if (r_ != PTQ2_OK) return r_; \
   } while (0)
 
+// the spare memory of every level; whether there was any
+bool give_back(ptq2_mg *mg) {
+  bool any = false;
+  for (ptq2_ctx *c : mg->ctx) any |= ptq2_internal_give_back(c);
+  return any;
+}
+// a call that allocates for one level, again if the others' spare memory makes room
+#define MGMEM(call)                                             \
+  do {                                                          \
+    int m_ = (call);                                            \
+    if (m_ == PTQ2_ERR_ALLOC && give_back(mg)) m_ = (call);     \
+    if (m_ != PTQ2_OK) return m_;                               \
+  } while (0)
+
+int level_facebuf(ptq2_ctx *c) {
+  int rc = PTQ2_OK;
+  (void)ptq2_internal_facebuf(c, &rc);
+  return rc;
+}
+
 int mg_alloc(ptq2_mg *mg, void **p, size_t bytes) {
-  if (hipMalloc(p, bytes) != hipSuccess) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && give_back(mg)) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
+  if (e != hipSuccess) {
     (void)hipGetLastError();
     *p = nullptr;
     return mgfail(mg, PTQ2_ERR_ALLOC, "hipMalloc failed in the multigrid set-up");
@@ -1287,10 +1314,22 @@ bool level_own(const ptq2_mg *mg, int l) {
   return mg->f32 && mg->tune[l].split == 1 && !mg->gal[l] && ptq2::own_blocks_fit(mg->lbox[l]);
 }
 
+// the level's box with the resident tiles that its context has now (they may be given back)
+ptq2::Box level_box(const ptq2_mg *mg, int l) {
+  ptq2::Box b = mg->lbox[l];
+  b.xtile = mg->no_tiles ? nullptr : mg->ctx[l]->box.xtile;
+  return b;
+}
+int resident_tiles(const ptq2_mg *mg) {
+  int n = 0;
+  for (const ptq2_ctx *c : mg->ctx) n += c->box.xtile != nullptr;
+  return n;
+}
+
 // (the row-split choice is made for the smoothing precision and applies to it only)
 hipError_t level_launch(ptq2_mg *mg, int l, const double *x, double *y, bool gather) {
   ptq2_ctx *c = mg->ctx[l];
-  const ptq2::Box &b = mg->lbox[l];
+  const ptq2::Box b = level_box(mg, l);
   if (mg->gal[l] && mg->tune[l].split == 4 && !mg->f32) return galerkin_mf<double>(mg, l, x, y);
   if (mg->gal[l]) {
     hipLaunchKernelGGL(k_stencil_apply<double>, dim3(nblk(c->nnodes)), dim3(TPB), 0, mg->stream, b.NX, b.NY, b.NZ,
@@ -1369,7 +1408,7 @@ int level_apply_cheb(ptq2_mg *mg, int l, const T *x, T *y, const ptq2::ChebOut<T
 template <>
 int level_apply_cheb<double>(ptq2_mg *mg, int l, const double *x, double *y, const ptq2::ChebOut<double> &co) {
   ptq2_ctx *c = mg->ctx[l];
-  MGCHK(ptq2::launch_a11_fp64(mg->lbox[l], c->coords, x, c->mask, c->eta_bm, y, ptq2::OUT_SET, mg->stream,
+  MGCHK(ptq2::launch_a11_fp64(level_box(mg, l), c->coords, x, c->mask, c->eta_bm, y, ptq2::OUT_SET, mg->stream,
                               (double *)c->facebuf, false, &co));
   return PTQ2_OK;
 }
@@ -2145,9 +2184,51 @@ int rigid_setup(ptq2_mg *mg) {
 }
 
 
+// the graph of one V-cycle
+int capture_vcycle(ptq2_mg *mg) {
+  MGCHK(hipStreamBeginCapture(mg->stream, hipStreamCaptureModeThreadLocal));
+  int rc = vcycle_body(mg);
+  hipGraph_t gph = nullptr;
+  hipError_t e = hipStreamEndCapture(mg->stream, &gph);
+  if (rc) {
+    if (gph) (void)hipGraphDestroy(gph);
+    return rc;
+  }
+  if (e != hipSuccess) return mgfail(mg, PTQ2_ERR_DEVICE, hipGetErrorString(e));
+  mg->graph = gph;
+  mg->graph_tiles = resident_tiles(mg);
+  MGCHK(hipGraphInstantiate(&mg->exec, mg->graph, nullptr, nullptr, 0));
+  return PTQ2_OK;
+}
+
+// Before V-cycles: the graph again if tiles that it holds were given back (which waited for the device); a
+// caller's capture of the kernels runs without tiles, one of the graph holds on to them.
+int check_tiles(ptq2_mg *mg) {
+  mg->no_tiles = false;
+  const int tiles = resident_tiles(mg);
+  if (tiles && ptq2_internal_capturing(mg->stream)) {
+    if (mg->exec)
+      for (ptq2_ctx *c : mg->ctx) c->spare_held = true;
+    else
+      mg->no_tiles = true;
+  }
+  if (!mg->exec || tiles == mg->graph_tiles) return PTQ2_OK;
+  MGCHK(hipGraphExecDestroy(mg->exec));
+  mg->exec = nullptr;
+  MGCHK(hipGraphDestroy(mg->graph));
+  mg->graph = nullptr;
+  // as at the set-up, on a stream that can be captured
+  hipStream_t s = mg->stream;
+  mg->stream = mg->ctx[0]->own_stream;
+  const int rc = capture_vcycle(mg);
+  mg->stream = s;
+  return rc;
+}
+
 // z = M^-1 (scale r): one V-cycle reading r and writing z directly (the input is read in full
 // by the graph's first kernel before its last kernel writes z, so r and z may alias)
 int vcycle_scaled(ptq2_mg *mg, const double *r, double scale, double *z) {
+  MGRC(check_tiles(mg));
   hipLaunchKernelGGL(k_set_io, dim3(1), dim3(64), 0, mg->stream, mg->io, r, z, scale, 1.0);
   if (mg->exec) MGCHK(hipGraphLaunch(mg->exec, mg->stream));
   else MGRC(vcycle_body(mg));
@@ -2296,7 +2377,7 @@ int ptq2_mg_create(ptq2_mg **out, ptq2_ctx *fine, const ptq2_mg_opts *opts) {
     mg->ctx.push_back(c);
     mg->owned.push_back(true);
     ptq2_set_stream(c, mg->stream);
-    MGRC(ptq2_setup_mesh(c, mx, my, mz, cc.data(), nullptr, fine->mask ? mc.data() : nullptr));
+    MGMEM(ptq2_setup_mesh(c, mx, my, mz, cc.data(), nullptr, fine->mask ? mc.data() : nullptr));
     if (o.coarse_eta_mean == PTQ2_ETA_MEAN_Q1PROJ) {
       // the reference's hierarchy: the lattice field of the level above, restricted, then
       // interpolated to this level's quadrature points
@@ -2304,7 +2385,7 @@ int ptq2_mg_create(ptq2_mg **out, ptq2_ctx *fine, const ptq2_mg_opts *opts) {
       q1_restrict_nodal(mx, my, mz, q1nodal, nc);
       q1_interpolate_qp(mx, my, mz, nc, ec);
       q1nodal.swap(nc);
-      MGRC(ptq2_set_viscosity(c, ec.data(), 0, 0));
+      MGMEM(ptq2_set_viscosity(c, ec.data(), 0, 0));
     } else {
       // viscosity from the finer level
       double *etac = nullptr;
@@ -2333,11 +2414,7 @@ int ptq2_mg_create(ptq2_mg **out, ptq2_ctx *fine, const ptq2_mg_opts *opts) {
   mg->gst32.assign(mg->nl, nullptr);
   mg->gmf_in.assign(mg->nl, nullptr);
   mg->gmf_out.assign(mg->nl, nullptr);
-  for (int l = 0; l + 1 < mg->nl; l++) {
-    int rc = PTQ2_OK;
-    (void)ptq2_internal_facebuf(mg->ctx[l], &rc);
-    MGRC(rc);
-  }
+  for (int l = 0; l + 1 < mg->nl; l++) MGMEM(level_facebuf(mg->ctx[l]));
   for (int l = mg->nl - 1 - o.galerkin_levels; l + 1 < mg->nl; l++) MGRC(build_galerkin_level(mg, l));
 
   // ---- small reduction buffers (also used by the solve)
@@ -2362,7 +2439,7 @@ int ptq2_mg_create(ptq2_mg **out, ptq2_ctx *fine, const ptq2_mg_opts *opts) {
     MGRC(mg_alloc(mg, &mg->vp2[l], es * n));
     MGRC(mg_alloc(mg, &mg->vdinv[l], es * n));
     ptq2_ctx *c = mg->ctx[l];
-    if (mg->f32) MGRC(ptq2_internal_build_fac32(c));
+    if (mg->f32) MGMEM(ptq2_internal_build_fac32(c));
     double *d = nullptr, *v = nullptr, *w = nullptr;
     MGRC(mg_alloc(mg, (void **)&d, sizeof(double) * n));
     MGRC(mg_alloc(mg, (void **)&v, sizeof(double) * n));
@@ -2423,11 +2500,7 @@ int ptq2_mg_create(ptq2_mg **out, ptq2_ctx *fine, const ptq2_mg_opts *opts) {
     MGRC(rc);
   }
   // ---- launch shapes of the smoother applies
-  for (int l = 0; l + 1 < mg->nl; l++) {
-    int rc = PTQ2_OK;
-    (void)ptq2_internal_facebuf(mg->ctx[l], &rc);
-    MGRC(rc);
-  }
+  for (int l = 0; l + 1 < mg->nl; l++) MGMEM(level_facebuf(mg->ctx[l]));
   MGRC(mg->f32 ? autotune<float>(mg) : autotune<double>(mg));
   // ---- dense coarse inverse, assembled and inverted on the device
   {
@@ -2525,19 +2598,7 @@ int ptq2_mg_create(ptq2_mg **out, ptq2_ctx *fine, const ptq2_mg_opts *opts) {
   if (o.rigid_deflation) MGRC(rigid_setup(mg));
   // ---- graph of one V-cycle
   MGRC(mg_alloc(mg, (void **)&mg->io, sizeof(VcIO)));
-  if (o.use_graph) {
-    MGCHK(hipStreamBeginCapture(mg->stream, hipStreamCaptureModeThreadLocal));
-    int rc = vcycle_body(mg);
-    hipGraph_t gph = nullptr;
-    hipError_t e = hipStreamEndCapture(mg->stream, &gph);
-    if (rc) {
-      if (gph) (void)hipGraphDestroy(gph);
-      return rc;
-    }
-    if (e != hipSuccess) return mgfail(mg, PTQ2_ERR_DEVICE, hipGetErrorString(e));
-    mg->graph = gph;
-    MGCHK(hipGraphInstantiate(&mg->exec, mg->graph, nullptr, nullptr, 0));
-  }
+  if (o.use_graph) MGRC(capture_vcycle(mg));
   MGCHK(hipStreamSynchronize(mg->stream));
   guard.release();
   *out = mg;
@@ -2611,6 +2672,7 @@ int ptq2_mg_vcycle(ptq2_mg *mg, const double *r, double *z) {
 int ptq2_mg_level_times(ptq2_mg *mg, const double *r, double *z, int reps, double *ms) {
   if (!mg || !r || !z || !ms || reps < 1) return PTQ2_ERR_INVALID_ARG;
   MGRC(check_fine(mg));
+  MGRC(check_tiles(mg));
   if (mg->pev.empty()) {
     mg->pev.assign(4 * (size_t)mg->nl, nullptr);
     for (hipEvent_t &e : mg->pev) MGCHK(hipEventCreate(&e));

@@ -1,18 +1,30 @@
-"""Host compiles of the kernels' address and arithmetic helpers (no GPU needed)."""
+"""Host compiles of the kernels' address and arithmetic helpers, and the library's host side on a stand-in for
+the HIP runtime (no GPU needed)."""
 import os
 import subprocess
 
 import pytest
 
 REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-CSRC = os.path.join(REPO, "ptatin-gene_amd", "csrc")
+PKG = os.path.join(REPO, "ptatin-gene_amd")
+CSRC = os.path.join(PKG, "csrc")
 
 
 @pytest.mark.parametrize("name,line", [("test_tile_rows", "tile rows ok"), ("test_row_sums", "row sums ok")])
 def test_host_check(tmp_path, name, line):
+    run_check(tmp_path, name, line)
+
+
+def test_host_logic(tmp_path):
+    """libptq2.so itself, its runtime calls answered by the test program: memory limits and graph capture."""
+    run_check(tmp_path, "test_host_logic", "host logic ok",
+              ["-x", "none", os.path.join(PKG, "libptq2.so"), "-Wl,-rpath," + PKG, "-rdynamic"])
+
+
+def run_check(tmp_path, name, line, link=()):
     exe = str(tmp_path / name)
     subprocess.check_call(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "-O1", "-std=c++17", "-x", "hip", "-I", CSRC,
-                           "-I", os.path.join(REPO, "include"), os.path.join(REPO, "tests", "c", name + ".cpp"),
+                           "-I", os.path.join(REPO, "include"), os.path.join(REPO, "tests", "c", name + ".cpp"), *link,
                            "-o", exe])
     out = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0, out.stderr + out.stdout
