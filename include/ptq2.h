@@ -164,7 +164,8 @@ int ptq2_stokes_residual(ptq2_ctx *ctx, const double *u, const double *p, const 
    elements in ascending order, so the result is bitwise reproducible; it equals the
    reference's point-order sums to rounding.  flags: PTQ2_DEVICE (every array a device pointer).
    Synchronous.  A workspace of about 350 bytes per element (more with more than 8 points per element,
-   750 at most) stays with the context until its next mesh set-up or its end.  Needs a single-rank box
+   750 at most) stays with the context until its next mesh set-up or its end, or until the context needs the
+   memory; without room for it a call takes 16 bytes per node and sorts the points.  Needs a single-rank box
    (ptq2_setup_mesh, or ptq2_setup_mesh_box without a ghost layer); a box with a ghost layer is
    PTQ2_ERR_UNSUPPORTED.  An element index out of range is PTQ2_ERR_INVALID_ARG, a non-finite
    coordinate or value PTQ2_ERR_NONFINITE.  Pass eta_qp to ptq2_set_viscosity to use it. */

@@ -78,3 +78,8 @@ bool ptq2_internal_capturing(hipStream_t s);
 // the tile buffer of the uncoloured output path if this mesh uses it (allocated on first
 // use), else nullptr; *rc receives an allocation error
 void *ptq2_internal_facebuf(ptq2_ctx *c, int *rc);
+// ptq2_project_points_q1 with at most max_work bytes of workspace kept in the context (tests of the path that a
+// device without room takes)
+extern "C" int ptq2_internal_project_points(ptq2_ctx *c, int64_t np, const double *xi, const int32_t *wil,
+                                            const double *eta_p, const double *rho_p, double *eta_qp, double *rho_qp,
+                                            unsigned flags, size_t max_work);

@@ -110,6 +110,19 @@ __device__ __forceinline__ int adjacent(int I, int m, int el[2], int loc[2]) {
 
 // Q1 basis of the vertex at local node index l (0 or 2) along one axis at coordinate x
 __device__ __forceinline__ double q1_1d(int l, double x) { return l == 0 ? 1.0 - x : 1.0 + x; }
+// A point's weight a b at a vertex, and its share of the three sums; fused explicitly, so that the element sums and
+// the nodes' own have the same bits.
+struct VertexWeight {
+  double a, b;
+  __device__ __forceinline__ VertexWeight(int lx, int ly, int lz, const double *xi)
+      : a(0.125 * q1_1d(lx, xi[0]) * q1_1d(ly, xi[1])), b(q1_1d(lz, xi[2])) {}
+};
+__device__ __forceinline__ void add_point(double a, double b, double v, double r, double &sv, double &sr, double &sw) {
+  const double w = a * b;
+  sv = fma(w, v, sv);
+  sr = fma(w, r, sr);
+  sw = fma(a, b, sw);
+}
 
 // Sums over an element's points in index order: eight lanes per element, one per vertex, walk the points
 // together (a point's values are one broadcast load).  part, arrays of ne values: 3 l + 0..2 the sums of w
@@ -151,11 +164,9 @@ __global__ __launch_bounds__(PTB) void k_points_sums(int64_t ne, int cap, const 
 #pragma unroll 4
   for (int64_t k = 0; k < n; k++) {
     const int64_t p = list[k];
-    const double w = 0.125 * q1_1d(lx, xi[3 * p]) * q1_1d(ly, xi[3 * p + 1]) * q1_1d(lz, xi[3 * p + 2]);
+    const VertexWeight w(lx, ly, lz, xi + 3 * p);
     const double v = eta[p], r = rho ? rho[p] : 0.0;
-    a1 += w * v;
-    a2 += w * r;
-    bw += w;
+    add_point(w.a, w.b, v, r, a1, a2, bw);
     c1 += v;
     c2 += r;
   }
@@ -169,8 +180,17 @@ __global__ __launch_bounds__(PTB) void k_points_sums(int64_t ne, int cap, const 
   }
 }
 
-// One thread per node: add the sums of the adjacent elements (ascending), divide.
-__global__ void k_points_to_nodes(Box b, const double *__restrict__ part, double *__restrict__ neta,
+// The points of the sort, for nodes that sum them themselves
+struct SortedPoints {
+  const int64_t *off;
+  const int32_t *order;
+  const double *xi, *eta, *rho;
+};
+
+// One thread per node: add the sums of the adjacent elements (ascending), divide.  WALK: without room for the
+// elements' sums every node forms those it needs, in the same order (265 us for 0.5 million points).
+template <bool WALK>
+__global__ void k_points_to_nodes(Box b, const double *__restrict__ part, SortedPoints sp, double *__restrict__ neta,
                                   double *__restrict__ nrho) {
   const int64_t nn = (int64_t)b.NX * b.NY * b.NZ, ne = (int64_t)b.mx * b.my * b.mz;
   for (int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; n < nn; n += (int64_t)gridDim.x * blockDim.x) {
@@ -183,6 +203,18 @@ __global__ void k_points_to_nodes(Box b, const double *__restrict__ part, double
         for (int a = 0; a < nx; a++) {
           const int64_t e = (int64_t)ex[a] + (int64_t)b.mx * ((int64_t)ey[bb] + (int64_t)b.my * ez[c]);
           const bool vert = lx[a] != 1 && ly[bb] != 1 && lz[c] != 1;
+          if (WALK) {
+            double e1 = 0.0, e2 = 0.0, ew = 0.0;
+            for (int64_t k = sp.off[e]; k < sp.off[e + 1]; k++) {
+              const int64_t p = sp.order[k];
+              const VertexWeight w(lx[a], ly[bb], lz[c], sp.xi + 3 * p);
+              add_point(vert ? w.a : 1.0, vert ? w.b : 1.0, sp.eta[p], nrho ? sp.rho[p] : 0.0, e1, e2, ew);
+            }
+            a1 += e1;
+            a2 += e2;
+            bw += ew;
+            continue;
+          }
           const double *s = part + 3 * (vert ? lx[a] / 2 + ly[bb] + 2 * lz[c] : 8) * ne + e;
           a1 += s[0];
           if (nrho) a2 += s[ne];
@@ -257,10 +289,10 @@ int pfail(ptq2_ctx *c, int code, const char *fmt, ...) {
   return code;
 }
 
-// hipMalloc that has the context's spare memory given back before it fails
-hipError_t take(ptq2_ctx *c, void **p, size_t bytes) {
+// hipMalloc that has the context's spare memory (and, with work, this workspace) given back before it fails
+hipError_t take(ptq2_ctx *c, void **p, size_t bytes, bool work) {
   hipError_t e = hipMalloc(p, bytes);
-  if (e == hipErrorOutOfMemory && ptq2_internal_give_back(c, false)) {
+  if (e == hipErrorOutOfMemory && ptq2_internal_give_back(c, work)) {
     (void)hipGetLastError();
     e = hipMalloc(p, bytes);
   }
@@ -273,10 +305,11 @@ struct Scratch {
   ptq2_ctx *c;
   void *p[CAP] = {};
   int n = 0;
+  bool work = true;  // the context's workspace is not in use yet
   explicit Scratch(ptq2_ctx *c_) : c(c_) {}
-  ~Scratch() {
-    for (int i = 0; i < n; i++)
-      if (p[i]) (void)hipFree(p[i]);
+  ~Scratch() { drop(0); }
+  void drop(int keep) {
+    while (n > keep) (void)hipFree(p[--n]);
   }
   template <typename T>
   hipError_t get(T **out, size_t bytes) {
@@ -285,7 +318,7 @@ struct Scratch {
       *out = nullptr;
       return hipErrorOutOfMemory;
     }
-    const hipError_t e = take(c, &q, bytes ? bytes : 1);
+    const hipError_t e = take(c, &q, bytes ? bytes : 1, work);
     if (e == hipSuccess) p[n++] = q;
     *out = (T *)q;
     return e;
@@ -294,12 +327,13 @@ struct Scratch {
 
 inline size_t align(size_t n) { return (n + 255) / 256 * 256; }
 
-// the context's point workspace, at least `bytes` long (contents lost)
-hipError_t grow(ptq2_ctx *c, size_t bytes) {
+// the context's point workspace, at least `bytes` long (contents lost); none above the caller's limit
+hipError_t grow(ptq2_ctx *c, size_t bytes, size_t limit) {
+  if (c->pwork_bytes >= bytes && c->pwork_bytes <= limit) return hipSuccess;
   if (c->pwork) (void)hipFree(c->pwork);
   c->pwork = nullptr;
   c->pwork_bytes = 0;
-  const hipError_t e = take(c, &c->pwork, bytes);
+  const hipError_t e = bytes <= limit ? take(c, &c->pwork, bytes, false) : hipErrorOutOfMemory;
   if (e == hipSuccess) c->pwork_bytes = bytes;
   else c->pwork = nullptr;
   return e;
@@ -321,6 +355,12 @@ hipError_t grow(ptq2_ctx *c, size_t bytes) {
 extern "C" int ptq2_project_points_q1(ptq2_ctx *c, int64_t np, const double *xi, const int32_t *wil,
                                       const double *eta_p, const double *rho_p, double *eta_qp, double *rho_qp,
                                       unsigned flags) {
+  return ptq2_internal_project_points(c, np, xi, wil, eta_p, rho_p, eta_qp, rho_qp, flags, SIZE_MAX);
+}
+
+extern "C" int ptq2_internal_project_points(ptq2_ctx *c, int64_t np, const double *xi, const int32_t *wil,
+                                            const double *eta_p, const double *rho_p, double *eta_qp, double *rho_qp,
+                                            unsigned flags, size_t max_work) {
   using namespace ptq2;
   if (!c) return PTQ2_ERR_INVALID_ARG;
   if (!c->mesh_ready) return pfail(c, PTQ2_ERR_NOT_SETUP, "MF operator not setup: no mesh");
@@ -360,39 +400,57 @@ extern "C" int ptq2_project_points_q1(ptq2_ctx *c, int64_t np, const double *xi,
     if (rho_qp) PCHK(S.get(&drq, sizeof(double) * 27 * (size_t)ne));
   }
   // Workspace, kept in the context until its next mesh or its end: counters (with the error word), slots,
-  // element sums and nodal values, the nodal values alone where the slots do not fit.
+  // element sums and nodal values; where that does not fit, the error word and the nodal values alone.
   int cap = bucket_slots(np, ne);
+  bool sums = true;
   const size_t bcnt = align(sizeof(int32_t) * (size_t)(ne + 1)), bpart = sizeof(double) * 27 * (size_t)ne,
-               bnode = sizeof(double) * (size_t)nn;
-  const auto bytes = [&] { return bcnt + align(sizeof(int32_t) * (size_t)ne * (size_t)cap) + bpart + 2 * bnode; };
-  hipError_t we = hipSuccess;
-  if (c->pwork_bytes < bytes() && (we = grow(c, bytes())) == hipErrorOutOfMemory && cap) {
+               bnodes = sizeof(double) * (size_t)nn * (drho ? 2 : 1);
+  S.work = false;
+  int *err = nullptr;
+  int32_t *slot = nullptr;
+  double *part = nullptr, *neta = nullptr, *nrho = nullptr;
+  const auto work = [&] {
+    const size_t head = sums ? bcnt : align(sizeof(int)), bslot = align(sizeof(int32_t) * (size_t)ne * (size_t)cap),
+                 bsums = sums ? bpart : 0;
+    const hipError_t e = grow(c, head + bslot + bsums + bnodes, max_work);
+    if (e != hipSuccess) return e;
+    char *w = (char *)c->pwork;
+    err = (int *)w;
+    slot = cap ? (int32_t *)(w + head) : nullptr;
+    part = sums ? (double *)(w + head + bslot) : nullptr;
+    neta = (double *)(w + head + bslot + bsums);
+    nrho = drho ? neta + nn : nullptr;
+    return hipMemsetAsync(err, 0, sums ? bcnt : sizeof(int), s);
+  };
+  const auto without_sums = [&] {
     (void)hipGetLastError();
+    if (c->pwork) (void)hipFree(c->pwork);
+    c->pwork = nullptr;
+    c->pwork_bytes = 0;
     cap = 0;
-    we = c->pwork_bytes < bytes() ? grow(c, bytes()) : hipSuccess;
-  }
+    sums = false;
+    return work();
+  };
+  hipError_t we = work();
+  if (we == hipErrorOutOfMemory) we = without_sums();
   PCHK(we);
-  int *err = (int *)c->pwork;
-  int32_t *cnt = (int32_t *)err + 1;
-  int32_t *slot = cap ? (int32_t *)((char *)c->pwork + bcnt) : nullptr;
-  double *part = (double *)((char *)c->pwork + bcnt + align(sizeof(int32_t) * (size_t)ne * (size_t)cap));
-  double *neta = part + 27 * ne, *nrho = drho ? neta + nn : nullptr;
+  SortedPoints sp{nullptr, nullptr, dxi, deta, drho};
   const auto finish = [&] {
-    hipLaunchKernelGGL(k_points_to_nodes, dim3(grid_of(nn)), dim3(PTB), 0, s, b, (const double *)part, neta, nrho);
+    hipLaunchKernelGGL((sums ? k_points_to_nodes<false> : k_points_to_nodes<true>), dim3(grid_of(nn)), dim3(PTB), 0, s, b,
+                       (const double *)part, sp, neta, nrho);
     hipLaunchKernelGGL(k_nodes_to_qp, dim3((unsigned)((ne + 63) / 64), nrho ? 2 : 1), dim3(64), 0, s, b, (const double *)neta,
                        (const double *)nrho, deq, drq, (const int *)err);
   };
   const dim3 sgrid((unsigned)((ne + SUM_ELEMS - 1) / SUM_ELEMS));
-  PCHK(hipMemsetAsync(err, 0, bcnt, s));
   if (np > 0) {
-    hipLaunchKernelGGL(k_points_bucket, dim3(grid_of(np)), dim3(PTB), 0, s, np, ne, dxi, dwil, deta, drho, cap, cnt,
-                       slot, err);
+    hipLaunchKernelGGL(k_points_bucket, dim3(grid_of(np)), dim3(PTB), 0, s, np, ne, dxi, dwil, deta, drho, cap,
+                       (int32_t *)err + 1, slot, err);
     PCHK(hipGetLastError());
   }
   if (slot) {
     // before the host has seen the checks: only checked points are in a slot, and an error leaves the outputs alone
     hipLaunchKernelGGL(k_points_sums<true>, sgrid, dim3(PTB), 2 * SUM_ELEMS * cap * sizeof(int32_t), s, ne, cap,
-                       (const int32_t *)cnt, (const int32_t *)slot, (const int64_t *)nullptr, (const int32_t *)nullptr,
+                       (const int32_t *)err + 1, (const int32_t *)slot, (const int64_t *)nullptr, (const int32_t *)nullptr,
                        dxi, deta, drho, part);
     finish();
     PCHK(hipGetLastError());
@@ -404,30 +462,47 @@ extern "C" int ptq2_project_points_q1(ptq2_ctx *c, int64_t np, const double *xi,
   if (bits & PERR_FINITE) return pfail(c, PTQ2_ERR_NONFINITE, "non-finite point coordinate or value");
   if (!slot || (bits & PERR_CROWDED)) {
     // stable bucketing by element
+    const int had = S.n;
     int32_t *keys, *order, *iota;
     int64_t *off;
-    PCHK(S.get(&keys, sizeof(int32_t) * (size_t)np));
-    PCHK(S.get(&order, sizeof(int32_t) * (size_t)np));
-    PCHK(S.get(&iota, sizeof(int32_t) * (size_t)np));
-    PCHK(S.get(&off, sizeof(int64_t) * (size_t)(ne + 1)));
+    void *tmp;
+    size_t tmp_bytes = 0;
+    int end_bit = 1;
+    while (end_bit < 31 && ((int64_t)1 << end_bit) < ne) end_bit++;
+    // the keys are validated non-negative: sort them as unsigned on the bits that can be set
+    const uint32_t *ukin = reinterpret_cast<const uint32_t *>(dwil);
+    const auto buffers = [&] {
+      hipError_t e = S.get(&keys, sizeof(int32_t) * (size_t)np);
+      if (e == hipSuccess) e = S.get(&order, sizeof(int32_t) * (size_t)np);
+      if (e == hipSuccess) e = S.get(&iota, sizeof(int32_t) * (size_t)np);
+      if (e == hipSuccess) e = S.get(&off, sizeof(int64_t) * (size_t)(ne + 1));
+      if (e == hipSuccess && np > 0) {
+        e = hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, ukin, reinterpret_cast<uint32_t *>(keys), iota, order,
+                                               (int)np, 0, end_bit, s);
+        if (e == hipSuccess) e = S.get(&tmp, tmp_bytes);
+      }
+      return e;
+    };
+    hipError_t be = buffers();
+    if (be == hipErrorOutOfMemory && sums) {
+      S.drop(had);
+      be = without_sums();
+      if (be == hipSuccess) be = buffers();
+    }
+    PCHK(be);
     if (np > 0) {
       hipLaunchKernelGGL(k_iota, dim3(grid_of(np)), dim3(PTB), 0, s, np, iota);
       PCHK(hipGetLastError());
-      int end_bit = 1;
-      while (end_bit < 31 && ((int64_t)1 << end_bit) < ne) end_bit++;
-      size_t tmp_bytes = 0;
-      // the keys are validated non-negative: sort them as unsigned on the bits that can be set
-      const uint32_t *ukin = reinterpret_cast<const uint32_t *>(dwil);
-      uint32_t *ukout = reinterpret_cast<uint32_t *>(keys);
-      PCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, ukin, ukout, iota, order, (int)np, 0, end_bit, s));
-      void *tmp;
-      PCHK(S.get(&tmp, tmp_bytes));
-      PCHK(hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, ukin, ukout, iota, order, (int)np, 0, end_bit, s));
+      PCHK(hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, ukin, reinterpret_cast<uint32_t *>(keys), iota, order,
+                                              (int)np, 0, end_bit, s));
     }
     hipLaunchKernelGGL(k_bucket_offsets, dim3(grid_of(ne + 1)), dim3(PTB), 0, s, np, ne, (const int32_t *)keys, off);
     PCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_points_sums<false>, sgrid, dim3(PTB), 0, s, ne, 0, (const int32_t *)nullptr,
-                       (const int32_t *)nullptr, (const int64_t *)off, (const int32_t *)order, dxi, deta, drho, part);
+    sp.off = off;
+    sp.order = order;
+    if (sums)
+      hipLaunchKernelGGL(k_points_sums<false>, sgrid, dim3(PTB), 0, s, ne, 0, (const int32_t *)nullptr,
+                         (const int32_t *)nullptr, (const int64_t *)off, (const int32_t *)order, dxi, deta, drho, part);
     PCHK(hipMemsetAsync(err, 0, sizeof(int), s));
     finish();
     PCHK(hipGetLastError());

@@ -4,7 +4,8 @@
 //
 // Checked: memory that a large mesh runs faster with (Box::xtile, the slots of A12 and the diagonal) never
 // makes a call fail that fits without it, is a sixteenth of the device at most, and is in no graph that may
-// outlive it; A12 and the diagonal run without slots under capture.
+// outlive it; A12 and the diagonal run without slots under capture; the point projection needs no more than
+// its sort and the nodal values.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -16,7 +17,7 @@
 #include <vector>
 
 #include "ptq2.h"
-#include "ptq2_device.h"
+#include "ptq2_ctx.h"
 #include "ptq2_solver.h"
 
 namespace {
@@ -78,7 +79,7 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
 }
 hipError_t hipMalloc(void **p, size_t n) {
   *p = nullptr;
-  if (n > S().limit - S().used) return hipErrorOutOfMemory;
+  if (S().used + n > S().limit) return hipErrorOutOfMemory;
   *p = calloc(n, 1);  // pages are taken when written
   S().mem[*p] = n;
   S().used += n;
@@ -122,6 +123,14 @@ hipError_t hipGetDevice(int *d) {
   *d = 0;
   return hipSuccess;
 }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int) {
+  memset(p, 0, sizeof *p);
+  strcpy(p->gcnArchName, "gfx950");
+  p->multiProcessorCount = 256;
+  p->warpSize = 64;
+  return hipSuccess;
+}
+int hipGetStreamDeviceId(hipStream_t) { return 0; }
 hipError_t hipGetLastError() { return hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "stand-in"; }
 static void *handle() { return (void *)(uintptr_t)(0x1000 + 16 * ++S().handles); }
@@ -306,6 +315,44 @@ void operators_under_capture() {
   ptq2_destroy(&c);
 }
 
+// The projection where only the sort's buffers and the nodal values fit: what it needed before it had a
+// workspace of its own.
+void projection_at_the_limit() {
+  const Mesh m(4, 4, 2048);
+  const int64_t ne = 32768, np = 8 * ne, nn = m.nvel / 3;
+  std::vector<double> xi(3 * np, 0.0), v(np, 1.0), out(27 * ne);
+  std::vector<int32_t> wil(np, 0);
+  for (int dev = 0; dev < 2; dev++) {
+    ptq2_ctx *c = m.make();
+    const unsigned f = dev ? PTQ2_DEVICE : 0;
+    const auto project = [&] {
+      S().launches.clear();
+      return ptq2_project_points_q1(c, np, xi.data(), wil.data(), v.data(), v.data(), out.data(), out.data(), f);
+    };
+    const size_t before = S().used;
+    // the sort's keys, order and positions, its own scratch (at least keys and values), offsets, nodal values, staging
+    const size_t need = (size_t)np * (12 + 8) + 8 * (size_t)(ne + 1) + 16 * (size_t)nn +
+                        (dev ? 0 : (size_t)np * (24 + 4 + 16) + 2 * 27 * 8 * (size_t)ne);
+    EXPECT(project() == PTQ2_OK && count("k_points_sums") == 1 && count("k_points_to_nodesILb0") == 1);
+    const size_t kept = S().used - before;
+    // a second call may use what the first one kept; without room the nodes sum the points themselves
+    S().limit = before + need + (1 << 20);
+    EXPECT(project() == PTQ2_OK && (dev || count("k_points_to_nodesILb1") == 1));
+    EXPECT(ptq2_setup_mesh(c, 4, 4, 2048, m.coords.data(), nullptr, m.mask.data()) == PTQ2_OK);
+    EXPECT(project() == PTQ2_OK && count("k_points_to_nodesILb1") == 1);
+    // and an apply's buffers take the place of what it kept
+    S().limit = SIZE_MAX;
+    EXPECT(project() == PTQ2_OK && S().used >= before + kept);
+    EXPECT(ptq2_set_viscosity(c, m.eta.data(), 3, 0) == PTQ2_OK);
+    S().limit = S().used;
+    double d[1];
+    EXPECT(ptq2_a11_apply(c, d, d + 1, PTQ2_DEVICE) == PTQ2_OK);
+    S().limit = SIZE_MAX;
+    ptq2_destroy(&c);
+    EXPECT(S().used == 0);
+  }
+}
+
 void hierarchy_at_the_limit() {
   const Mesh m(128, 128, 32);  // 8192 bricks
   const size_t spare = spare_of(8192);
@@ -359,6 +406,7 @@ void hierarchy_at_the_limit() {
 int main() {
   operators_at_the_limit();
   operators_under_capture();
+  projection_at_the_limit();
   hierarchy_at_the_limit();
   if (bad) return 1;
   std::printf("host logic ok\n");
