@@ -137,7 +137,8 @@ enum {
 /* Launch shape the autotuner chose for the smoother apply of each level l < nlevels - 1:
    kernel (PTQ2_MG_KERNEL_*), tile addressing (1: fast full-tile path, 0: general), and the
    measured ms per apply of the chosen and of the default shape (both 0 when autotune was off
-   or forced).  Any output may be NULL. */
+   or forced; on FP32 levels small enough for overlapping blocks, whose apply is complete, with
+   the face pass and Dirichlet rows of the other kernels).  Any output may be NULL. */
 int ptq2_mg_tuning(const ptq2_mg *mg, int *kernel, int *fast_tiles, double *ms, double *ms_default);
 /* Per-level time of the V-cycle: reps V-cycles z = M^-1 r launched kernel by kernel (not from
    the graph) with events between the levels; ms[l] = the mean time of level l's own work

@@ -1583,7 +1583,9 @@ int build_galerkin_level(ptq2_mg *mg, int l) {
 }
 
 // ms per apply of level l's smoother apply (no face pass) in the current launch shape: the
-// fastest of 3 timed batches of reps launches, after 2 untimed ones
+// fastest of 3 timed batches of reps launches, after 2 untimed ones.  Where the row-split kernel would be the one in
+// overlapping blocks, which leaves nothing to a face pass, every kernel is timed with the face pass and the
+// Dirichlet rows.
 template <typename T>
 int time_level(ptq2_mg *mg, int l, int reps, double *ms) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1595,11 +1597,16 @@ int time_level(ptq2_mg *mg, int l, int reps, double *ms) {
   }
   const T *x = (const T *)mg->vx[l];
   T *y = (T *)mg->vy[l];
+  const bool whole = sizeof(T) == 4 && !mg->gal[l] && ptq2::own_blocks_fit(mg->lbox[l]);
+  const auto apply = [&] {
+    if (whole) return level_matmult<T>(mg, l, x, y) == PTQ2_OK ? hipSuccess : hipErrorLaunchFailure;
+    return level_launch(mg, l, x, y, false);
+  };
   double best = 1e30;
-  for (int k = 0; k < 2 && e == hipSuccess; k++) e = level_launch(mg, l, x, y, false);
+  for (int k = 0; k < 2 && e == hipSuccess; k++) e = apply();
   for (int k = 0; k < 3 && e == hipSuccess; k++) {
     e = hipEventRecord(e0, mg->stream);
-    for (int i = 0; i < reps && e == hipSuccess; i++) e = level_launch(mg, l, x, y, false);
+    for (int i = 0; i < reps && e == hipSuccess; i++) e = apply();
     if (e == hipSuccess) e = hipEventRecord(e1, mg->stream);
     if (e == hipSuccess) e = hipEventSynchronize(e1);
     float t = 0.0f;

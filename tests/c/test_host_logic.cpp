@@ -401,6 +401,34 @@ void hierarchy_at_the_limit() {
     S().limit = SIZE_MAX;
   }
 }
+// The kernels that the autotuner compares do the same work: on a level of overlapping blocks, whose apply is
+// complete, the others are launched with their face pass.
+void autotuner_compares_like_with_like() {
+  for (int m : {8, 64}) {
+    const Mesh mesh(m, m, m);
+    ptq2_ctx *c = mesh.make();
+    ptq2_mg_opts o;
+    ptq2_mg_default_opts(&o);
+    o.nlevels = m == 8 ? 2 : 4;
+    o.esteig_its = 1;
+    S().launches.clear();
+    ptq2_mg *mg = nullptr;
+    EXPECT(ptq2_mg_create(&mg, c, &o) == PTQ2_OK);
+    // up to 16^3 elements (5 blocks per axis) every level is one of overlapping blocks; 64^3 and 32^3 are not
+    int with = 0, without = 0, own = 0;
+    const std::vector<Launch> &l = S().launches;
+    for (size_t i = 0; i + 1 < l.size(); i++) {
+      own += l[i].name.find("k_a11_fp32_own") != std::string::npos;
+      if (l[i].name.find("k_a11_fp32") == std::string::npos || l[i].name.find("_own") != std::string::npos) continue;
+      const bool face = l[i + 1].name.find("k_gather_faces") != std::string::npos;
+      (face ? with : without)++;
+    }
+    EXPECT(own > 0 && with > 0);
+    EXPECT(m == 8 ? without == 0 : without > 0);
+    ptq2_mg_destroy(&mg);
+    ptq2_destroy(&c);
+  }
+}
 }  // namespace
 
 int main() {
@@ -408,6 +436,7 @@ int main() {
   operators_under_capture();
   projection_at_the_limit();
   hierarchy_at_the_limit();
+  autotuner_compares_like_with_like();
   if (bad) return 1;
   std::printf("host logic ok\n");
   return 0;
