@@ -140,9 +140,8 @@ __device__ __forceinline__ void row_grad(const double v[18], double g[3][3]) {
   double r0[3];
   row_grad<QB>(v, g, r0);
 }
-// slab 1 -> slab 0; a[n] gets the z direction's a, which slab 2 needs (u0: layer 0, still nodal)
-__device__ __forceinline__ void fold_slab0(double v[18], double u0[9], double a[9]) {
-  modal_layer(u0);
+// slab 1 -> slab 0; a[n] gets the z direction's a, which slab 2 needs (u0: layer 0, nodal along z only; may be a)
+__device__ __forceinline__ void fold_slab0(double v[18], const double u0[9], double a[9]) {
 #pragma unroll
   for (int n = 0; n < 9; n++) {
     a[n] = fma(2.0, u0[n] - v[n], v[n + 9]);  // u0 - 2 u1 + u2
@@ -284,11 +283,10 @@ __device__ __forceinline__ void get3(const double *slot, int lane, double &a, do
 __host__ __device__ constexpr int row_qc(int r) { return r / 3 == 0 ? 1 : (r / 3 == 1 ? 0 : 2); }
 __host__ __device__ constexpr int row_qb(int r) { return r % 3 == 0 ? 0 : (r % 3 == 1 ? 2 : 1); }
 
-// slab 0 -> slab 2 from the nodal layer 2 instead of a: v = m + V2 a - V1 b and d = b - D2 a in slab 0, and
+// slab 0 -> slab 2 from layer 2 (nodal along z only) instead of a: v = m + V2 a - V1 b and d = b - D2 a in slab 0, and
 // u2 = m + (b + a) / 2 gives a (1/2 - V2 + (1/2 + V1) D2) = u2 - v - (1/2 + V1) d
-__device__ __forceinline__ void fold_slab2_layer(double v[18], double u2[9]) {
+__device__ __forceinline__ void fold_slab2_layer(double v[18], const double u2[9]) {
   constexpr double e = 0.5 + MOD_V1, f = 1.0 / (0.5 - MOD_V2 + e * MOD_D2);
-  modal_layer(u2);
 #pragma unroll
   for (int n = 0; n < 9; n++) {
     const double a = f * fma(-e, v[n + 9], u2[n] - v[n]);
@@ -362,6 +360,7 @@ struct GWave {
       if (BLK && (R == 3 || R == 6)) {
 #pragma unroll
         for (int n = 0; n < 9; n++) t[c][n] -= avg[c];
+        modal_layer(t[c]);
         if (R == 3)
           fold_slab0(x[c], t[c], t[c]);
         else
@@ -372,6 +371,7 @@ struct GWave {
 #pragma unroll
         for (int n = 0; n < 9; n++) t[n] = park[(9 * c + n) * BEL + lane];
         if (R == 3) {
+          modal_layer(t);
           fold_slab0(x[c], t, t);
 #pragma unroll
           for (int n = 0; n < 9; n++) park[(9 * c + n) * BEL + lane] = t[n];
@@ -449,7 +449,10 @@ struct UWave {
   // gradients of row R; the two foreign points' values go to G
   template <int R>
   __device__ __forceinline__ void forward(double *row, int lane) {
-    if (R == 3) fold_slab0(u, u + 18, u + 18);
+    if (R == 3) {
+      modal_layer(u + 18);
+      fold_slab0(u, u + 18, u + 18);
+    }
     if (R == 6) fold_slab2(u, u + 18);
     if (R == 3 || R == 6) pin<18>(u);
     double G[3][3];

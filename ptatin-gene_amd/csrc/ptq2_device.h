@@ -532,62 +532,54 @@ __device__ __forceinline__ void store_rows_full(const Box &b, const BrickId &br,
   }
 }
 
-// the Chebyshev store of a full tile, with the addressing of load_tile2_fast
+// the Chebyshev store of a full tile, with the addressing of load_tile2_fast (FP32 passes; the FP64 pass stores by
+// store_tile4)
 template <typename S, typename T>
 __device__ __forceinline__ void store_tile_cheb_fast(const Box &b, const BrickId &br, const Tile &t,
                                                      const S *__restrict__ s, T *__restrict__ g,
                                                      T *__restrict__ face, int lane, const ChebOut<T> *co) {
-  constexpr int STEPS = TPAIRS;
   const FastLane L = fast_lane(b, lane);
   const bool ownx = L.ii < 2 * BE || br.bx == b.nbx - 1;
   const bool lasty = br.by == b.nby - 1, lastz = br.bz == b.nbz - 1;
   const int64_t node0 = t.node0;
   T *gb = g + 3 * node0;
   T *fo = face + (int64_t)br.lin * FACEVALS + L.c;
-  // the update's operands of a chunk of steps are all loaded before the first is used (one
-  // exposed memory latency per chunk, not per step); every tile address is inside the box
-  constexpr int CHUNK = sizeof(T) == 4 ? STEPS : 14;
+  // the update's operands are all loaded before the first is used (one exposed memory latency, not one per
+  // step); every tile address is inside the box
   const T *bb = co->b + 3 * node0, *bd = co->dinv + 3 * node0, *bx = co->x + 3 * node0;
   const T *bp = co->pkm1 ? co->pkm1 + 3 * node0 : nullptr;
   const uint8_t *bm = co->mask ? co->mask + 3 * node0 : nullptr;
   T *bo = co->out + 3 * node0;
+  T vb[TPAIRS], vd[TPAIRS], vx[TPAIRS], vp[TPAIRS];
+  int vm[TPAIRS];
 #pragma unroll
-  for (int c0 = 0; c0 < STEPS; c0 += CHUNK) {
-    T vb[CHUNK], vd[CHUNK], vx[CHUNK], vp[CHUNK];
-    int vm[CHUNK];
+  for (int it = 0; it < TPAIRS; it++) {
+    const uint32_t e = fast_eoff(b, L, it);
+    vb[it] = fast_at(bb, e);
+    vd[it] = fast_at(bd, e);
+    vx[it] = fast_at(bx, e);
+    vp[it] = bp ? fast_at(bp, e) : T(0);
+    vm[it] = bm ? (int)fast_at(bm, e) : 0;
+  }
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int k = 0; k < CHUNK; k++) {
-      const int it = c0 + k;
-      if (it >= STEPS) break;
-      const uint32_t e = fast_eoff(b, L, it);
-      vb[k] = fast_at(bb, e);
-      vd[k] = fast_at(bd, e);
-      vx[k] = fast_at(bx, e);
-      vp[k] = bp ? fast_at(bp, e) : T(0);
-      vm[k] = bm ? (int)fast_at(bm, e) : 0;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int k = 0; k < CHUNK; k++) {
-      const int it = c0 + k;
-      if (it >= STEPS) break;
-      if (!fast_stores(L, it)) continue;
-      int y, z;
-      fast_row(L, it, y, z);
-      const bool owny = y < 2 * BE || lasty, ownz = z < 2 * BE || lastz;
-      const S val = s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)];
-      const uint32_t e = fast_eoff(b, L, it);
-      if (ownx && owny && ownz) {
-        const bool lower = (L.ii == 0 && br.bx > 0) || (y == 0 && br.by > 0) || (z == 0 && br.bz > 0);
-        if (vm[k] || !lower) {
-          fast_at(bo, e) = cheb_value(*co, vd[k], vb[k], vm[k] ? vx[k] : T(val), vx[k], vp[k], bp != nullptr);
-        } else {
-          fast_at(gb, e) = T(val);
-        }
+  for (int it = 0; it < TPAIRS; it++) {
+    if (!fast_stores(L, it)) continue;
+    int y, z;
+    fast_row(L, it, y, z);
+    const bool owny = y < 2 * BE || lasty, ownz = z < 2 * BE || lastz;
+    const S val = s[(fast_wrap(it) ? L.ldsw : L.lds0) + fast_lds_step(it)];
+    const uint32_t e = fast_eoff(b, L, it);
+    if (ownx && owny && ownz) {
+      const bool lower = (L.ii == 0 && br.bx > 0) || (y == 0 && br.by > 0) || (z == 0 && br.bz > 0);
+      if (vm[it] || !lower) {
+        fast_at(bo, e) = cheb_value(*co, vd[it], vb[it], vm[it] ? vx[it] : T(val), vx[it], vp[it], bp != nullptr);
       } else {
-        const int slot = !ownx ? z * TN + y : (!owny ? TN * TN + z * TN + L.ii : 2 * TN * TN + y * TN + L.ii);
-        fo[3 * slot] = T(val);
+        fast_at(gb, e) = T(val);
       }
+    } else {
+      const int slot = !ownx ? z * TN + y : (!owny ? TN * TN + z * TN + L.ii : 2 * TN * TN + y * TN + L.ii);
+      fo[3 * slot] = T(val);
     }
   }
 }

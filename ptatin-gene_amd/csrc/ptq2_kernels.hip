@@ -750,11 +750,10 @@ __device__ __forceinline__ void load_layer(const double *s, int base, int c, dou
   modal_layer(v);
   v[0] -= shift;
 }
-// One field's values and derivatives along z (row_grad) for the slab of row R, when R opens a slab;
-// field values are taken relative to shift.  The third z coefficient a, which slab 1 does not need,
-// is formed again in the other two from a layer read from the tile: kept, it would cost 54 registers of the
-// three (or six) fields.  Slab 0 has v = m + V2 a - V1 b, d = b - D2 a, and u2 = m + (b + a) / 2 gives
-// a (1/2 - V2 + (1/2 + V1) D2) = u2 - v - (1/2 + V1) d.
+// One field's values and derivatives along z (row_grad) for the slab of row R, when R opens a slab; field
+// values are taken relative to shift.  The third z coefficient, which slab 1 does not need, is formed again in
+// the other two from a layer read from the tile: kept, it would cost 54 registers of the three (or six)
+// fields.
 template <int R>
 __device__ __forceinline__ void to_row_slab(const double *s, int base, int c, double shift, double v[18]) {
   if (R == 0) {
@@ -767,23 +766,11 @@ __device__ __forceinline__ void to_row_slab(const double *s, int base, int c, do
   } else if (R == 3) {
     double u0[9];
     load_layer<0>(s, base, c, shift, u0);
-#pragma unroll
-    for (int n = 0; n < 9; n++) {
-      const double a = fma(2.0, u0[n] - v[n], v[n + 9]);
-      v[n] = fma(-MOD_V1, v[n + 9], fma(MOD_V2, a, v[n]));
-      v[n + 9] = fma(-MOD_D2, a, v[n + 9]);
-    }
+    fold_slab0(v, u0, u0);
   } else if (R == 6) {
-    constexpr double e = 0.5 + MOD_V1, f = 1.0 / (0.5 - MOD_V2 + e * MOD_D2);
     double u2[9];
     load_layer<2>(s, base, c, shift, u2);
-#pragma unroll
-    for (int n = 0; n < 9; n++) {
-      const double a = f * fma(-e, v[n + 9], u2[n] - v[n]);
-      const double b = fma(MOD_D2, a, v[n + 9]);
-      v[n] = fma(2.0 * MOD_V1, b, v[n]);
-      v[n + 9] = fma(MOD_D2, a, b);
-    }
+    fold_slab2_layer(v, u2);
   }
   if (R % 3 == 0) {
     pin<18>(v);
