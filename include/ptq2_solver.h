@@ -66,9 +66,10 @@ typedef struct {
      or general tile addressing where every tile is full, and keep the fastest
      (ptq2_mg_tuning reports the choice).  The kernels sum in different orders, so two
      hierarchies whose choices differ round differently in the last bits.  0: one wave per
-     brick and the mesh's own tile addressing on every level.  2: the three-wave kernel on
-     every level, 3: the matrix-core form on every level (FP32 smoothing), 4: the one-wave
-     kernel, and R A P through the level above on a Galerkin level below a matrix-free one,
+     brick and the mesh's own tile addressing on every level.  2: the row-split kernels on
+     every level, 3: the matrix-core form on every level (FP32 smoothing; with FP64 smoothing
+     0, 2 and 3 run its one kernel, which 2 reports as PTQ2_MG_KERNEL_SPLIT and does not fuse
+     with the Chebyshev update), 4: the one-wave kernel, and R A P through the level above on a Galerkin level below a matrix-free one,
      untimed (for tests and comparisons).  A Galerkin level below a matrix-free one is timed
      as its stencil and as R A P (prolongation, the level above's matrix-free apply,
      restriction), which streams far fewer bytes than the stencil on large levels. */
@@ -128,8 +129,9 @@ int ptq2_mg_rigid_info(const ptq2_mg *mg, int *ninclusions, int *ncolumns, int32
 int ptq2_mg_eigs(const ptq2_mg *mg, double *emin, double *emax);
 /* Kernels of the smoother apply (ptq2_mg_tuning) */
 enum {
-  PTQ2_MG_KERNEL_BRICK = 0,       /* FP32: one wave per brick of 4x4x4 elements; FP64 */
-  PTQ2_MG_KERNEL_SPLIT = 1,       /* FP32: three or (up to 256 bricks) nine waves per brick */
+  PTQ2_MG_KERNEL_BRICK = 0,       /* FP32: one wave per brick of 4x4x4 elements; FP64: its one kernel */
+  PTQ2_MG_KERNEL_SPLIT = 1,       /* FP32: three or (up to 256 bricks) nine waves per brick, or overlapping
+                                     blocks; FP64 with autotune 2: its one kernel */
   PTQ2_MG_KERNEL_MFMA = 2,        /* the FP32 operator's matrix-core form */
   PTQ2_MG_KERNEL_STENCIL = 3,     /* Galerkin level: its assembled 5x5x5 block stencil */
   PTQ2_MG_KERNEL_GALERKIN_MF = 4  /* Galerkin level: R A P through the matrix-free level above */

@@ -480,7 +480,6 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   dev_free(c->pwork);
   free_spare(c);
   c->coords = nullptr; c->mask = nullptr; c->dir_idx = nullptr; c->eta_bm = nullptr;
-  c->bdir = nullptr;
   c->fac32 = nullptr; c->facb32 = nullptr; c->geo64 = nullptr; c->facebuf = c->facebuf2 = nullptr;
   c->face2_used = false;
   c->pwork = nullptr; c->pwork_bytes = 0;
@@ -501,27 +500,28 @@ int ptq2_setup_mesh_box(ptq2_ctx *c, int mx, int my, int mz, int NX, int NY, int
   if ((rc = dev_alloc(c, (void **)&c->coords, sizeof(double) * 3 * (size_t)nn))) return rc;
   HIPCHK(c, hipMemcpy(c->coords, coords, sizeof(double) * 3 * (size_t)nn, hipMemcpyHostToDevice));
   if (mask) {
+    // one allocation and copy for the dofs and the flags
     std::vector<int64_t> idx;
     std::vector<uint8_t> bdir((size_t)nb, 0);
     c->ndir_ghost = dirichlet_dofs(b, mask, idx, bdir);
-    if ((rc = dev_alloc(c, (void **)&c->mask, 3 * (size_t)nn + (size_t)nb))) return rc;
+    if ((rc = dev_alloc(c, (void **)&c->mask, 3 * (size_t)nn))) return rc;
     HIPCHK(c, hipMemcpy(c->mask, mask, 3 * (size_t)nn, hipMemcpyHostToDevice));
-    c->bdir = c->mask + 3 * (size_t)nn;
-    HIPCHK(c, hipMemcpy(c->bdir, bdir.data(), (size_t)nb, hipMemcpyHostToDevice));
-    b.bdir = c->bdir;
     c->ndir = (int64_t)idx.size();
-    if (c->ndir) {
-      if ((rc = dev_alloc(c, (void **)&c->dir_idx, sizeof(int64_t) * idx.size()))) return rc;
-      HIPCHK(c, hipMemcpy(c->dir_idx, idx.data(), sizeof(int64_t) * idx.size(), hipMemcpyHostToDevice));
-    }
+    idx.resize(idx.size() + ((size_t)nb + 7) / 8);
+    memcpy(idx.data() + c->ndir, bdir.data(), (size_t)nb);
+    if ((rc = dev_alloc(c, (void **)&c->dir_idx, sizeof(int64_t) * idx.size()))) return rc;
+    HIPCHK(c, hipMemcpy(c->dir_idx, idx.data(), sizeof(int64_t) * idx.size(), hipMemcpyHostToDevice));
+    b.bdir = (const uint8_t *)(c->dir_idx + c->ndir);
   }
   c->box = b;
   c->nnodes = nn; c->nvel = 3 * nn; c->nel = ne; c->npres = 4 * ne; c->nbricks = nb;
   // The face slots of A12 and the diagonal, which thus never allocate, share the viscosity's allocation on small
   // meshes (48 MB at most; one of their own would make a small set-up longer).  Large ones take them and the
   // resident coordinate tiles as spare memory.  The tiles pay where the vectors come from HBM, not from the 256 MB
-  // cache before it: FP64 apply 1113 us with, 1163 us without at 128^3 elements (32768 bricks), 145 us with and
-  // without at 64^3 (4096 bricks).  A mesh without the slots runs A12 and the diagonal in coloured launches.
+  // cache before it.  FP64 apply with and without, by bricks: 4096 144.1 and 142.9 us, 5832 204 and 209, 8000
+  // 281 and 290, 8820 304 and 318, 13824 470 and 492, 32768 1113 and 1163; full block 166.6 and 158.6, 241 and
+  // 238, 329 and 328, 358 and 359, 551 and 553.  From 8192 bricks on neither loses.  A mesh without the slots runs A12
+  // and the diagonal in coloured launches.
   const size_t neta = (size_t)nb * 27 * ptq2::BEL, nface = ((size_t)nb * ptq2::FACEVALS + 1) & ~(size_t)1;
   if (nb < 8192 && (rc = dev_alloc(c, (void **)&c->eta_bm, sizeof(double) * (neta + nface))) == PTQ2_OK)
     c->facebuf2 = c->eta_bm + neta;

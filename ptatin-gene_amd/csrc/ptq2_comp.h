@@ -21,7 +21,8 @@
 // The 1D contractions work on (m, b, a) = (u1, u2 - u0, u0 - 2 u1 + u2) instead of the nodal
 // values: with x = sqrt(3/5), u(+-x) = m + 0.3 a +- (x/2) b, u(0) = m, 2 u'(+-x) = b +- 2 x a and
 // 2 u'(0) = b, 5 operations for three values and three derivatives against 14 with the nodal
-// tables.  A brick takes 6.4k VALU instructions, the one-wave form with nodal tables 12.9k.  All derivatives carry the factor 2; it is taken out in the point weights (w / 8:
+// tables.  A brick takes 6.4k VALU instructions, the one-wave form with nodal tables 12.9k.  All derivatives
+// carry the factor 2; it is taken out in the point weights (w / 8:
 // J' = 2 J, adj(J') = 4 adj(J), det J' = 8 det J, and the transposed derivative applies 2 again).
 //
 // What bounds it: a workgroup's chain of load, nine rows with a barrier each, output and store takes

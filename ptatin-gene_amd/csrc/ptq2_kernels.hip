@@ -60,7 +60,7 @@ __device__ __forceinline__ void emit_element(S *Ys, int base, const T Y[3][3][3]
 // (and, with fp, minus the continuity source: FormFunctionLocal_P's -int N^p fp,
 // src/stokes_form_function.c:478-580).  The G wave interpolates the pressure, whose basis is linear in the
 // coordinates it has, and takes each point's divergence back; the U waves add one term to the stress.  Bound as
-// the A11 pass is (256 VGPRs, 78 KB of LDS).  64^3: 151 us against 205 us with one wave per brick and nodal tables;
+// the A11 pass is (256 VGPRs with 56 B of scratch per lane, 78 KB of LDS).  64^3: 151 us against 205 us with one wave per brick and nodal tables;
 // 48^3: 69 us against 107 us.
 __global__ __launch_bounds__(CWAVES * BEL, 2) void k_stokes_fp64(Box b, const double *__restrict__ coords,
                                                                 const double *__restrict__ u,
@@ -105,10 +105,7 @@ __global__ __launch_bounds__(CWAVES * BEL, 2) void k_a11_fp64_batch(BatchArgs<do
 // Geometric factors are precomputed in FP64 (k_build_fac32) and stored rounded
 // to FP32 as F = sqrt(w eta / det) * adj(J), 9 per quadrature point, brick-major
 // [brick][q][m][lane] so that every load instruction is one contiguous 256-byte
-// segment.  Each is read once per apply: where they alone fill most of the 256 MB cache (FAC_NT),
-// non-temporally (80^3 apply 180 -> 169 us, full block of 140k elements 80 -> 73 us, 64^3 86 -> 84 and
-// 108 -> 95 us); below, the next apply finds part of them there (56^3 apply 62 against 64 us, 48^3
-// block 43 against 45 us non-temporally).  Then dv = F^T (M + M^T) with M = F g (diagonal doubled), all
+// segment.  Each is read once per apply, non-temporally from FAC_NT bytes of factors on (factors_nt).  Then dv = F^T (M + M^T) with M = F g (diagonal doubled), all
 // FP32.
 
 // one quadrature point of the FP32 A11 row: F = sqrt(w eta / det) adj(J) (9 floats)
@@ -206,6 +203,12 @@ __device__ __forceinline__ void fp32_rows(const float *Us, float *Fs, const floa
   }
 }
 
+// Non-temporal factor copies leave the 256 MB cache to the vectors and face slots.  Which side wins depends on what
+// runs between two applies.  One operator alone, over and over, finds part of its factors there up to about
+// 225 MB: A11 62.3 us non-temporally against 60.8 at 171 MB, 76.7 against 75.8 at 210, 82.4 against 85.6 at 255; block
+// 69.4 against 67.3 at 213 MB, 71.5 against 72.0 at 229, 88.1 against 96.2 at 303.  Of three operators
+// in turn none finds its own: A11 62.1 against 70.6 us at 171 MB, 75.7 against 87.3 at 210; block 69.5 against 79.4 at
+// 213, 88.4 against 103.3 at 303.  At 200 MB the first loses at most 3% and the second gains 14%.
 constexpr int64_t FAC_NT = 200000000;  // bytes
 inline bool factors_nt(int64_t nb, int values) { return nb * values * BEL * (int64_t)sizeof(float) >= FAC_NT; }
 
@@ -735,7 +738,8 @@ __global__ __launch_bounds__(BEL) void k_check_mesh(Box b, const double *__restr
 // --------------------------------------------------------- A21 and A12
 // One wave per brick, the contractions in the modal form of ptq2_comp.h, slab by slab in the order 1, 0, 2
 // of the quadrature points' z.  A wave is alone on its SIMD (all 512 registers), so what bounds both is
-// the number of instructions and every latency between them: 3.1k FP64 operations of 5-6k instructions
+// the number of instructions and every latency between them (A12's 54 coordinate values and 135 accumulators
+// also spill 276 B per lane, A21 nothing): 3.1k FP64 operations of 5-6k instructions
 // per wave (5.3k of 8-11k with the nodal tables and a row's data read from the tile).  64^3 elements:
 // A21 114 -> 79 us; A12 in one launch with the face pass 119 us, against 218 us in 8 coloured ones
 // (512 waves each, half the chip's SIMDs) with nodal tables.
@@ -1063,7 +1067,7 @@ __global__ __launch_bounds__(BEL) void k_body_force(Box b, const double *__restr
 // MatMultMF_Stokes_MixedFEM3d_diagB11 (src/stokes_q2p1_mf_operators_diag_def.c:120-205).
 // With h = A grad_xi N = det grad_x N: w det eta Nx^2 = (w eta / det) h_x^2.
 // The VALU instructions of one wave per brick bound it: 12k with the sums of h^2 below (17.8k with the three
-// weighted sums per point and node).  40x36x44 elements: 36 us (55 us) and 6 us of face pass; 355 us in
+// weighted sums per point and node); 36 B per lane spill.  40x36x44 elements: 36 us (55 us) and 6 us of face pass; 355 us in
 // 8 coloured launches of 125 waves, each one brick's latency.
 
 // At a point, with r = sqrt(w eta / det) and A = r adj(J), h_c(n) = D_i p + B_i q at node (i,j,k) with
@@ -1340,7 +1344,7 @@ hipError_t launch_gather_faces(const Box &b, const double *face, double *y, hipS
 }
 
 // Nine waves per brick while every brick gets a CU of its own: 8 bricks 8.2 us against 12.5 us with three
-// waves, 48 bricks 8.0 against 10.6.  Beyond, the SIMD that runs three of a brick's nine waves is what
+// waves, 48 bricks 8.0 against 10.6 (0.4 us more since their slabs are summed in FP64), 216 bricks 8.7.  Beyond, the SIMD that runs three of a brick's nine waves is what
 // a CU waits for: 384 bricks take 16.7 us, 13.8 us with three waves.
 hipError_t launch_a11_fp32_split(const Box &b, const float *u, const uint8_t *mask, const float *fac, float *y,
                                  bool add, hipStream_t s, float *facebuf, bool gather) {
@@ -1353,6 +1357,8 @@ hipError_t launch_a11_fp32_split(const Box &b, const float *u, const uint8_t *ma
   return gather ? launch_gather<float>(b, facebuf, y, s, nullptr) : hipGetLastError();
 }
 
+// 245 blocks (20x20x16 elements): a Chebyshev step 12.9 us; nine waves per brick with the separate update, at half
+// as many bricks, 9.5 + 5 us.  More blocks than CUs would take a second round.
 bool own_blocks_fit(const Box &b) {
   const bool single = !b.i0 && !b.j0 && !b.k0 && b.NX == 2 * b.mx + 1 && b.NY == 2 * b.my + 1 && b.NZ == 2 * b.mz + 1;
   return single && (int64_t)own_blocks(b.mx) * own_blocks(b.my) * own_blocks(b.mz) <= NUM_CUS;

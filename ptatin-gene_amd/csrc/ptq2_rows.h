@@ -13,8 +13,9 @@
 // unrolled rows would each be fetched cold.  x runs in the modal form of ptq2_comp.h (derivatives times 2, on
 // y and z too; the point weights take it out).
 //
-// What bounds it: a launch's latency; 8 bricks take 8.2 us and 48 bricks 8.0, of which some 5 us are the 1.2k VALU
-// instructions of the three waves that share the first SIMD (12.5 and 10.6 us with three waves per brick).
+// What bounds it: a launch's latency; 8 bricks took 8.2 us and 48 bricks 8.0, of which some 5 us are the 1.2k VALU
+// instructions of the three waves that share the first SIMD (12.5 and 10.6 us with three waves per brick).  The FP64
+// sums over the slabs added 0.4 us (216 bricks 9.2 -> 9.5 us, overlapping blocks of 16x16x12 elements 10.5 -> 10.9).
 #pragma once
 #include "ptq2_comp.h"
 
