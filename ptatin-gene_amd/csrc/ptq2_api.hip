@@ -210,6 +210,7 @@ int clear_err(ptq2_ctx *c) {
 }  // namespace
 
 bool ptq2_internal_capturing(hipStream_t s) {
+  if (!s) return false;  // the null stream cannot be, and the query fails while another stream is
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
   (void)hipGetLastError();

@@ -72,7 +72,7 @@ struct ptq2_ctx {
 int ptq2_internal_build_fac32(ptq2_ctx *c, bool block = false);
 // Gives spare memory (and, with work, the projection's workspace) back; whether there was any.  Waits for the device.
 bool ptq2_internal_give_back(ptq2_ctx *c, bool work = true);
-// whether work on s is being captured into a graph (or s is the null stream and another's capture forbids its use)
+// whether work on s is being captured into a graph
 bool ptq2_internal_capturing(hipStream_t s);
 // the tile buffer of the uncoloured output path if this mesh uses it (allocated on first
 // use), else nullptr; *rc receives an allocation error

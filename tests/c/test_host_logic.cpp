@@ -142,6 +142,7 @@ hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus *c) {
+  if (!s && !S().capture.empty()) return hipErrorStreamCaptureImplicit;
   *c = S().capture.count(s) ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
@@ -311,6 +312,14 @@ void operators_under_capture() {
   S().launches.clear();
   EXPECT(all_operators(c) == PTQ2_OK);
   EXPECT(tiles() == 1 && count("k_a12") == 1 && count("k_diag") == 1);
+  (void)hipGraphDestroy(g);
+  // another stream's capture does not change what a call on the null stream runs
+  (void)hipStreamBeginCapture((hipStream_t)0x10, hipStreamCaptureModeThreadLocal);
+  EXPECT(ptq2_set_stream(c, nullptr) == PTQ2_OK);
+  S().launches.clear();
+  EXPECT(all_operators(c) == PTQ2_OK);
+  EXPECT(tiles() == 1 && count("k_a12") == 1 && count("k_diag") == 1);
+  (void)hipStreamEndCapture((hipStream_t)0x10, &g);
   (void)hipGraphDestroy(g);
   ptq2_destroy(&c);
 }
