@@ -1116,8 +1116,7 @@ __device__ __forceinline__ void diag_rows(const double *Xs, int base, const doub
   for (int q = 0; q < 3; q++) e[q] = ep[(q + 3 * QB + 9 * QC) * BEL];
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    // relative to the element's middle node: a slab is folded from another one's values
-    to_row_slab<R>(Xs, base, c, Xs[base + toff(c, 1, 1, 1)], x[c]);
+    to_row_slab<R>(Xs, base, c, 0.0, x[c]);
     row_grad<QB>(x[c], Jc[c]);
   }
   row_fence();
