@@ -15,8 +15,8 @@ struct ptq2_ctx {
   ptq2::Box box{};
   int64_t nnodes = 0, nvel = 0, nel = 0, npres = 0, nbricks = 0;
   double *coords = nullptr;
-  uint8_t *mask = nullptr;
-  int64_t *dir_idx = nullptr;  // followed by box.bdir
+  uint8_t *mask = nullptr;       // followed by box.bdir and dir_idx
+  int64_t *dir_idx = nullptr;
   int64_t ndir = 0;
   int64_t ndir_ghost = 0;  // the last of dir_idx: dofs of ghost nodes that no brick's tile holds
   double *eta_bm = nullptr;
